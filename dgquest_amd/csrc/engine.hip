@@ -426,11 +426,32 @@ small_kernel(const dq_job *__restrict__ jobs, const dq_block *__restrict__ block
 // ----------------------------------------------------------------------------
 // probabilities
 // ----------------------------------------------------------------------------
-// Stage 1: workgroup g reads amplitudes [g * 2^CB, (g+1) * 2^CB) with
-// CB = min(n, 16), 256 threads, thread t owning indices with low 8 bits = t.
-// It writes 17 partial sums: P0 partials for qubits 0..15 and the total.
-#define PROB_WG_BITS 16
-#define PROB_SLOTS 17
+// P(0) of every qubit over the amplitudes whose index has given values on a
+// set of fixed bits (none for a whole state).  The other bits, in ascending
+// order, number the 2^nf amplitudes read; img[f] is the index bit of number
+// bit f (one-hot) and `fixed` the value of the fixed bits.
+//
+// Stage 1: workgroup g sums the numbers [g * 2^cb, (g + 1) * 2^cb), split as
+// bits 0..5 lane, the next JB bits a load index j, two wave bits, and up to
+// PROB_OUTER bits of a loop.  A wave has its 2^JB loads (1 KiB each in FP64
+// when no lane bit is fixed) in flight together.  It writes cb + 1 partial
+// sums, slot-major (part[slot * groups + g]): P0 of number bits 0..cb-1, then
+// the total.
+//
+// Bound: HBM for large states (16 * 2^n bytes, read once), latency for small
+// ones.  Before, a workgroup always read 2^16 amplitudes one load at a time:
+// a 17-qubit state occupied two workgroups.  Measured, both stages back to
+// back, before -> now: 17 qubits FP32 73 -> 6.8 us, 23 qubits FP64 141 -> 27 us
+// (4.9 TB/s), 26 qubits FP64 245 -> 169 us, 30 qubits FP64 2.97 -> 2.53 ms
+// (6.8 TB/s; 16 loads in flight per thread instead of what one loop step gives).
+#define PROB_OUTER 8
+#define PROB_SLOTS_MAX (8 + 4 + PROB_OUTER + 1)
+#define PROB_MAX_QUBITS 40
+
+struct ProbBits {
+    uint64_t img[PROB_MAX_QUBITS];
+    uint64_t fixed;
+};
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -438,69 +459,130 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256) prob_stage1(const typename V2<T>::type *__restrict__ st, int n, double *__restrict__ part) {
-    __shared__ double red[4][PROB_SLOTS];
-    const uint32_t tid = threadIdx.x;
-    const int cb = n < PROB_WG_BITS ? n : PROB_WG_BITS;
-    const uint64_t g0 = (uint64_t)blockIdx.x << cb;
-    double tot = 0.0;
-    double z[8];  // qubits 8..15 (bits of the per-thread loop index)
+template <typename T, int JB>
+__global__ void __launch_bounds__(256)
+prob_stage1(const typename V2<T>::type *__restrict__ st, const ProbBits pb, int nf, int cb, double *__restrict__ part) {
+    using V = typename V2<T>::type;
+    constexpr int J = 1 << JB;
+    __shared__ double red[4][PROB_SLOTS_MAX];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint64_t base = pb.fixed;
+    for (int i = cb; i < nf; i++) base |= ((blockIdx.x >> (i - cb)) & 1u) ? pb.img[i] : 0ull;
+    base |= ((w & 1u) ? pb.img[6 + JB] : 0ull) | ((w & 2u) ? pb.img[7 + JB] : 0ull);
+    uint64_t lp = 0;
 #pragma unroll
-    for (int q = 0; q < 8; q++) z[q] = 0.0;
-    if (cb >= 8) {
-        const uint32_t npt = 1u << (cb - 8);
-        for (uint32_t i = 0; i < npt; i++) {
-            const typename V2<T>::type v = __builtin_nontemporal_load(st + g0 + ((uint64_t)i << 8) + tid);
-            const double p = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
-            tot += p;
+    for (int i = 0; i < 6; i++) lp |= ((lane >> i) & 1u) ? pb.img[i] : 0ull;
+    uint64_t jm[JB > 0 ? JB : 1];
 #pragma unroll
-            for (int q = 0; q < 8; q++)
-                if (!((i >> q) & 1)) z[q] += p;
+    for (int b = 0; b < JB; b++) jm[b] = pb.img[6 + b];
+    uint64_t S = 0;  // the loop's index bits
+    for (int i = 8 + JB; i < cb; i++) S |= pb.img[i];
+    const uint32_t loops = cb > 8 + JB ? 1u << (cb - 8 - JB) : 1u;
+    const bool on = nf >= 8 || (tid >> nf) == 0;  // fewer than 256 amplitudes: the threads that own one
+    double tot = 0.0, zj[JB > 0 ? JB : 1], zo[PROB_OUTER];
+#pragma unroll
+    for (int b = 0; b < JB; b++) zj[b] = 0.0;
+#pragma unroll
+    for (int b = 0; b < PROB_OUTER; b++) zo[b] = 0.0;
+    uint64_t x = 0;
+    for (uint32_t it = 0; it < loops; it++) {
+        V v[J];
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            uint64_t u = base | x;
+#pragma unroll
+            for (int b = 0; b < JB; b++)
+                if ((j >> b) & 1) u |= jm[b];
+            v[j] = __builtin_nontemporal_load(st + u + lp);
         }
-    } else if (tid < (1u << cb)) {
-        const typename V2<T>::type v = st[g0 + tid];
-        tot = (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+        double s = 0.0;
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const double p = on ? (double)v[j].x * (double)v[j].x + (double)v[j].y * (double)v[j].y : 0.0;
+            s += p;
+#pragma unroll
+            for (int b = 0; b < JB; b++)
+                if (!((j >> b) & 1)) zj[b] += p;
+        }
+        tot += s;
+#pragma unroll
+        for (int b = 0; b < PROB_OUTER; b++)
+            if (!((it >> b) & 1u)) zo[b] += s;
+        x = ((x | ~S) + 1ull) & S;
     }
-    double vals[PROB_SLOTS];
+    // lane bit q: the lanes with the bit 0, other bits summed (valid in lane 0)
+    double t = tot;
 #pragma unroll
-    for (int q = 0; q < 8; q++) vals[q] = ((tid >> q) & 1) ? 0.0 : tot;
+    for (int q = 0; q < 6; q++) {
+        double r = t;
 #pragma unroll
-    for (int q = 0; q < 8; q++) vals[8 + q] = z[q];
-    vals[16] = tot;
-    const uint32_t wave = tid >> 6, lane = tid & 63;
-#pragma unroll
-    for (int s = 0; s < PROB_SLOTS; s++) {
-        const double r = wave_sum(vals[s]);
-        if (lane == 0) red[wave][s] = r;
+        for (int k = q + 1; k < 6; k++) r += __shfl_xor(r, 1 << k, 64);
+        if (lane == 0) red[w][q] = r;
+        t += __shfl_xor(t, 1 << q, 64);
     }
+    if (lane == 0) red[w][PROB_SLOTS_MAX - 1] = t;
+#pragma unroll
+    for (int b = 0; b < JB; b++) {
+        const double r = wave_sum(zj[b]);
+        if (lane == 0) red[w][6 + b] = r;
+    }
+#pragma unroll
+    for (int b = 0; b < PROB_OUTER; b++)
+        if (8 + JB + b < cb) {
+            const double r = wave_sum(zo[b]);
+            if (lane == 0) red[w][8 + JB + b] = r;
+        }
     __syncthreads();
-    if (tid < PROB_SLOTS) {
-        const double r = (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
-        part[(uint64_t)blockIdx.x * PROB_SLOTS + tid] = r;
+    const int s = (int)tid;
+    if (s <= cb) {
+        const int c = PROB_SLOTS_MAX - 1;
+        double r;
+        if (s == cb) r = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
+        else if (s == 6 + JB) r = red[0][c] + red[2][c];
+        else if (s == 7 + JB) r = red[0][c] + red[1][c];
+        else r = (red[0][s] + red[1][s]) + (red[2][s] + red[3][s]);
+        part[(uint64_t)s * gridDim.x + blockIdx.x] = r;
     }
 }
 
-// Stage 2: one workgroup per output q (0..n).  q < 16: sum of the partials
-// of slot q; q >= 16: sum of workgroup totals whose workgroup-index bit
-// (q - 16) is 0; q == n: sum of all totals.
-__global__ void __launch_bounds__(256) prob_stage2(const double *__restrict__ part, uint32_t ngroups, int n, double *__restrict__ out) {
+// What stage 2 makes of each qubit: bit[q] = its number bit, PROB_FIXED0 /
+// PROB_FIXED1 for a fixed one; every result is multiplied by `scale`.
+#define PROB_FIXED0 100
+#define PROB_FIXED1 101
+struct ProbOut {
+    uint8_t bit[PROB_MAX_QUBITS];
+    double scale;
+};
+
+// Stage 2: one workgroup per output q (0..n).  A number bit below cb sums its
+// slot; one at or above cb sums the totals of the workgroups whose index bit
+// (bit - cb) is 0; q == n and a qubit fixed to 0 sum every total.
+__global__ void __launch_bounds__(256) prob_stage2(const double *__restrict__ part, uint32_t groups, int n, int cb,
+                                                   const ProbOut po, double *__restrict__ out) {
     __shared__ double red[4];
     const int q = blockIdx.x;
     const uint32_t tid = threadIdx.x;
+    const int bit = q == n ? PROB_FIXED0 : po.bit[q];
+    const int slot = bit < cb ? bit : cb;
+    const uint32_t skip = bit >= cb && bit < PROB_FIXED0 ? 1u << (bit - cb) : 0u;
+    const double *__restrict__ src = part + (uint64_t)slot * groups;
     double acc = 0.0;
-    for (uint32_t g = tid; g < ngroups; g += 256) {
-        double v;
-        if (q == n) v = part[(uint64_t)g * PROB_SLOTS + 16];
-        else if (q < PROB_WG_BITS) v = part[(uint64_t)g * PROB_SLOTS + q];
-        else v = ((g >> (q - PROB_WG_BITS)) & 1) ? 0.0 : part[(uint64_t)g * PROB_SLOTS + 16];
-        acc += v;
+#pragma unroll 8
+    for (uint32_t g = tid; g < groups; g += 256) {
+        const double v = src[g];
+        acc += (g & skip) ? 0.0 : v;
     }
     acc = wave_sum(acc);
     if ((tid & 63) == 0) red[tid >> 6] = acc;
     __syncthreads();
-    if (tid == 0) out[q] = (red[0] + red[1]) + (red[2] + red[3]);
+    if (tid == 0) out[q] = bit == PROB_FIXED1 ? 0.0 : po.scale * ((red[0] + red[1]) + (red[2] + red[3]));
 }
+
+// The read-out of many states and the comparison split a state in chunks of
+// 2^PROB_WG_BITS amplitudes per workgroup.
+#define PROB_WG_BITS 16
+#define PROB_SLOTS 17
 
 // Device memory of the allocation-free P(0) entry point
 // (dq_prob_zero_all_noalloc): per-workgroup partial sums of one chunk of at
@@ -508,7 +590,7 @@ __global__ void __launch_bounds__(256) prob_stage2(const double *__restrict__ pa
 // for up to NA_MAX_QUBITS qubits; 2.2 MiB on every device the library runs on.
 #define NA_CHUNK_BITS 30
 #define NA_MAX_QUBITS 36
-#define NA_PART_DOUBLES ((1u << (NA_CHUNK_BITS - PROB_WG_BITS)) * PROB_SLOTS)
+#define NA_PART_DOUBLES ((1u << (NA_CHUNK_BITS - PROB_WG_BITS)) * PROB_SLOTS)  // at least prob_part_bytes(NA_CHUNK_BITS)
 #define NA_CHUNK_DOUBLES ((1u << (NA_MAX_QUBITS - NA_CHUNK_BITS)) * (NA_CHUNK_BITS + 1))
 static_assert((size_t)NA_PART_DOUBLES * sizeof(double) % 256 == 0, "chunk results stay 256-byte aligned");
 static __device__ __align__(256) double scratch[NA_PART_DOUBLES + NA_CHUNK_DOUBLES];
@@ -2155,44 +2237,103 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
     return DQ_OK;
 }
 
+// Split of 2^nf amplitudes over prob_stage1's workgroups: cb bits each, 2^JB
+// loads in flight per thread.  Small states spread over up to 256 workgroups
+// (one per CU) before a thread takes a second amplitude; from 2^20 amplitudes
+// a thread has 16 loads in flight and workgroups are added up to 2^PROB_GROUPS,
+// from where the loop inside a workgroup grows.
+#define PROB_GROUPS 13
+struct ProbSplit {
+    int cb, jb;
+    uint32_t groups;
+};
+static ProbSplit prob_split(int nf) {
+    ProbSplit p;
+    p.jb = nf <= 16 ? 0 : std::min(nf - 16, 4);
+    int outer = nf - 8 - p.jb - PROB_GROUPS;
+    outer = std::max(0, std::min(outer, PROB_OUTER));
+    p.cb = std::min(nf, 8 + p.jb + outer);
+    p.groups = 1u << (nf - p.cb);
+    return p;
+}
+
 // bytes of per-workgroup partial sums of prob_stage1
-static size_t prob_part_bytes(int n) {
-    const int cb = n < PROB_WG_BITS ? n : PROB_WG_BITS;
-    const uint64_t groups = 1ull << (n - cb);
-    return align_up(groups * PROB_SLOTS * sizeof(double), 256);
+static size_t prob_part_bytes(int nf) {
+    const ProbSplit p = prob_split(nf);
+    return align_up((size_t)p.groups * (p.cb + 1) * sizeof(double), 256);
 }
 
 extern "C" size_t dq_prob_ws_bytes(int n) { return prob_part_bytes(n) + 64 * sizeof(double); }
 
-extern "C" int dq_prob_zero_all_async(const void *state, int n, int prec, double *d_out, void *d_ws, size_t ws_bytes, void *stream) {
-    if (!state || !d_out || !d_ws || n < 1 || n > 40 || (prec != DQ_F32 && prec != DQ_F64))
+static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, uint64_t fixed_value, double scale,
+                       double *d_out, void *d_ws, size_t ws_bytes, hipStream_t stream) {
+    if (!state || !d_out || !d_ws || n < 1 || n > PROB_MAX_QUBITS || (prec != DQ_F32 && prec != DQ_F64))
         return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad arguments");
-    if (ws_bytes < prob_part_bytes(n)) return fail(DQ_ERR_ARG, "dq_prob_zero_all_async: workspace too small");
-    const int cb = n < PROB_WG_BITS ? n : PROB_WG_BITS;
-    const uint64_t groups = 1ull << (n - cb);
+    if ((fixed_mask >> n) || (fixed_value & ~fixed_mask)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad fixed bits");
+    const int nf = n - __builtin_popcountll(fixed_mask);
+    if (ws_bytes < prob_part_bytes(nf)) return fail(DQ_ERR_ARG, "dq_prob_zero_all_async: workspace too small");
+    const ProbSplit p = prob_split(nf);
+    ProbBits pb;
+    ProbOut po;
+    memset(&pb, 0, sizeof pb);
+    memset(&po, 0, sizeof po);
+    pb.fixed = fixed_value;
+    po.scale = scale;
+    int f = 0;
+    for (int q = 0; q < n; q++) {
+        const uint64_t b = 1ull << q;
+        if (fixed_mask & b) {
+            po.bit[q] = (fixed_value & b) ? PROB_FIXED1 : PROB_FIXED0;
+        } else {
+            po.bit[q] = (uint8_t)f;
+            pb.img[f++] = b;
+        }
+    }
     double *part = (double *)d_ws;
-    if (prec == DQ_F64)
-        hipLaunchKernelGGL(prob_stage1<double>, dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream,
-                           (const V2<double>::type *)state, n, part);
-    else
-        hipLaunchKernelGGL(prob_stage1<float>, dim3((unsigned)groups), dim3(256), 0, (hipStream_t)stream,
-                           (const V2<float>::type *)state, n, part);
+#define DQ_PROB1(T_, JB_)                                                                          \
+    hipLaunchKernelGGL((prob_stage1<T_, JB_>), dim3(p.groups), dim3(256), 0, stream, (const V2<T_>::type *)state, pb, nf, \
+                       p.cb, part)
+#define DQ_PROB1J(T_)                          \
+    switch (p.jb) {                            \
+        case 0: DQ_PROB1(T_, 0); break;        \
+        case 1: DQ_PROB1(T_, 1); break;        \
+        case 2: DQ_PROB1(T_, 2); break;        \
+        case 3: DQ_PROB1(T_, 3); break;        \
+        default: DQ_PROB1(T_, 4); break;       \
+    }
+    if (prec == DQ_F64) {
+        DQ_PROB1J(double)
+    } else {
+        DQ_PROB1J(float)
+    }
+#undef DQ_PROB1J
+#undef DQ_PROB1
     HIPC(hipGetLastError());
-    hipLaunchKernelGGL(prob_stage2, dim3(n + 1), dim3(256), 0, (hipStream_t)stream, part, (uint32_t)groups, n, d_out);
+    hipLaunchKernelGGL(prob_stage2, dim3(n + 1), dim3(256), 0, stream, part, p.groups, n, p.cb, po, d_out);
     HIPC(hipGetLastError());
     return DQ_OK;
 }
 
-extern "C" int dq_prob_zero_all(const void *state, int n, int prec, double *out, void *d_ws, size_t ws_bytes, void *stream) {
+extern "C" int dq_prob_zero_all_async(const void *state, int n, int prec, double *d_out, void *d_ws, size_t ws_bytes, void *stream) {
+    return prob_launch(state, n, prec, 0, 0, 1.0, d_out, d_ws, ws_bytes, (hipStream_t)stream);
+}
+
+extern "C" int dq_prob_zero_all_fixed(const void *state, int n, int prec, uint64_t fixed_mask, uint64_t fixed_value,
+                                      double scale, double *out, void *d_ws, size_t ws_bytes, void *stream) {
     if (!out) return fail(DQ_ERR_ARG, "dq_prob_zero_all: null output");
+    if (n < 1 || n > PROB_MAX_QUBITS) return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad arguments");
     if (ws_bytes < dq_prob_ws_bytes(n)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: workspace too small");
     const size_t part_bytes = prob_part_bytes(n);
     double *d_out = (double *)((unsigned char *)d_ws + part_bytes);
-    int rc = dq_prob_zero_all_async(state, n, prec, d_out, d_ws, part_bytes, stream);
+    const int rc = prob_launch(state, n, prec, fixed_mask, fixed_value, scale, d_out, d_ws, part_bytes, (hipStream_t)stream);
     if (rc) return rc;
     HIPC(hipMemcpyAsync(out, d_out, (n + 1) * sizeof(double), hipMemcpyDeviceToHost, (hipStream_t)stream));
     HIPC(hipStreamSynchronize((hipStream_t)stream));
     return DQ_OK;
+}
+
+extern "C" int dq_prob_zero_all(const void *state, int n, int prec, double *out, void *d_ws, size_t ws_bytes, void *stream) {
+    return dq_prob_zero_all_fixed(state, n, prec, 0, 0, 1.0, out, d_ws, ws_bytes, stream);
 }
 
 // ---- P(0) of every qubit without allocation or workspace --------------------

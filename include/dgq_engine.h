@@ -210,6 +210,15 @@ int dq_prob_zero_all(const void *state, int n_qubits, int prec, double *out,
                      void *d_ws, size_t ws_bytes, void *stream);
 size_t dq_prob_ws_bytes(int n_qubits);
 
+/* The same over the amplitudes whose index has the value fixed_value on the
+ * bits of fixed_mask, every result times `scale`: P(0) and the total of a
+ * state that was collapsed on those qubits and rescaled (scale = the product
+ * of 1 / P of each outcome) without the collapse being written back.  Reads
+ * only the 2^(n - fixed bits) amplitudes that are left.  A qubit fixed to 0
+ * gives the total, one fixed to 1 gives 0.  Workspace as dq_prob_zero_all. */
+int dq_prob_zero_all_fixed(const void *state, int n_qubits, int prec, uint64_t fixed_mask, uint64_t fixed_value,
+                           double scale, double *out, void *d_ws, size_t ws_bytes, void *stream);
+
 /* Same reduction, result left in device memory d_out (n + 1 doubles); no sync. */
 int dq_prob_zero_all_async(const void *state, int n_qubits, int prec, double *d_out,
                            void *d_ws, size_t ws_bytes, void *stream);
