@@ -357,7 +357,43 @@ void flush(QuregState *s) {
     s->last_flush_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
+// Are the recorded gates nothing but measurement collapses, of qubits not
+// collapsed to the other value before?  Then fixed / value are the index bits
+// they keep and scale what they multiply the kept probabilities by.
+static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value, double &scale) {
+    fixed = value = 0;
+    scale = 1.0;
+    if (s->recorder || s->paged || s->init_kind != DQ_INIT_LOAD || s->pending.empty()) return false;
+    for (const Gate &g : s->pending) {
+        if (g.type != OP_COLLAPSE || g.cmask || popc64(g.tmask) != 1) return false;
+        const uint64_t v = g.op[0] != 0.0 ? g.tmask : 0;
+        if ((fixed & g.tmask) && (value & g.tmask) != v) return false;
+        fixed |= g.tmask;
+        value |= v;
+        scale *= g.op[1] * g.op[1];
+    }
+    return true;
+}
+
 void ensure_probs(QuregState *s) {
+    // Measuring qubit after qubit: the collapses stay recorded and P(0) comes
+    // from the amplitudes they keep, half as many for every qubit measured,
+    // instead of a sweep over the whole state and a read of all of it per
+    // measurement.  The next flush runs the collapses with whatever follows.
+    uint64_t fixed, value;
+    double scale;
+    if (only_collapses(s, fixed, value, scale)) {
+        if (!s->probs_dirty) return;
+        ensure_ws(s, dq_prob_ws_bytes(s->n));
+        s->p0.assign(s->n + 1, 0.0);
+        ENG(dq_prob_zero_all_fixed(s->d_state, s->n, s->prec, fixed, value, scale, s->p0.data(), s->d_ws, s->ws_cap,
+                                   s->stream));
+        s->probs_dirty = false;
+        s->det_base = true;
+        s->det_pending = (int)s->pending.size();
+        s->det_slack = 0.0;
+        return;
+    }
     flush(s);
     if (!s->probs_dirty) return;
     s->det_pending = 0;
