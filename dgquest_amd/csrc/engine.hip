@@ -89,6 +89,8 @@ struct Regs {
 #define DQ_FJ 105
 #define DQ_BAUX 32
 #define DQ_RUNS 10
+#define DQ_BA_PROG 30     // [30] byte offset of the block's device programs, [31] their bytes
+#define DQ_WARM_TILES 512 // workgroups that warm the L2 (about the first that run, two per CU)
 
 // Byte offset of a thread's part of an exchange address: xor of the parts of
 // its set thread bits.  The wave bits are wave-uniform (wv is a scalar), so
@@ -178,8 +180,23 @@ __device__ __forceinline__ void exchange(Regs<T, R> &a, const uint32_t *__restri
     }
 }
 
+// Uniform descriptors: read through the constant address space, so that every
+// load is a scalar one whether they lie in the workspace or in the kernel's
+// arguments.
+#define DQ_CONST __attribute__((address_space(4)))
+typedef const DQ_CONST dq_block *CBlock;
+typedef const DQ_CONST uint32_t *CWords;
+
+// What a launch of a single job carries in its arguments: the job, its block
+// and the block's block_aux record.
+struct SweepOne {
+    dq_block blk;
+    uint32_t baux[DQ_BAUX];
+    dq_job job;
+};
+
 // Non-tile qubits of tile number t (t < 2^31) from the block's runs.
-__device__ __forceinline__ uint64_t tile_base_runs(const uint32_t *__restrict__ ba, uint32_t t) {
+__device__ __forceinline__ uint64_t tile_base_runs(CWords ba, uint32_t t) {
     uint64_t base = 0;
 #pragma unroll
     for (int i = 0; i < DQ_RUNS; i++) {
@@ -230,14 +247,16 @@ __device__ __forceinline__ P lane_ptr(P p, uint32_t lane) {
 // ld_reg / ld_wave.  The wave index wv is wave-uniform (a scalar), so every
 // address is "scalar base + lane * sizeof(V)" with no vector math.
 template <typename T, int R, int W>
-__device__ __forceinline__ void load_tile(Regs<T, R> &a, const dq_block *__restrict__ blk,
+__device__ __forceinline__ void load_tile(Regs<T, R> &a, CBlock blk,
                                           const __attribute__((address_space(1))) typename V2<T>::type *st,
                                           uint64_t base, uint32_t wv, uint32_t lane) {
     using V = typename V2<T>::type;
     constexpr int NR = 1 << R;
-    uint64_t wb = 0;
+    uint64_t lw[W > 0 ? W : 1], wb = 0;
 #pragma unroll
-    for (int w = 0; w < W; w++) wb |= ((wv >> w) & 1u) ? blk->ld_wave[w] : 0ull;
+    for (int w = 0; w < W; w++) lw[w] = blk->ld_wave[w];
+#pragma unroll
+    for (int w = 0; w < W; w++) wb |= lw[w] & (0ull - ((wv >> w) & 1u));
     uint64_t qo[R > 0 ? R : 1];
 #pragma unroll
     for (int r = 0; r < R; r++) qo[r] = blk->ld_reg[r];
@@ -277,7 +296,7 @@ __device__ __forceinline__ void load_tile(Regs<T, R> &a, const dq_block *__restr
 #define DQ_STORE_TILE(A, BASE)                                                            \
     do {                                                                                  \
         uint64_t wb_ = 0;                                                                 \
-        _Pragma("unroll") for (int w = 0; w < W; w++) wb_ |= ((wv >> w) & 1u) ? blk->st_wave[w] : 0ull; \
+        _Pragma("unroll") for (int w = 0; w < W; w++) wb_ |= blk->st_wave[w] & (0ull - ((wv >> w) & 1u)); \
         uint64_t qo_[R > 0 ? R : 1];                                                      \
         _Pragma("unroll") for (int r = 0; r < R; r++) qo_[r] = blk->st_reg[r];            \
         _Pragma("unroll") for (int j = 0; j < (1 << R); j++) {                            \
@@ -296,7 +315,7 @@ __device__ __forceinline__ void load_tile(Regs<T, R> &a, const dq_block *__restr
 // two or more phases the first LDS exchange already orders them (each wave
 // writes its loaded tile to LDS before the exchange barrier).
 template <int W>
-__device__ __forceinline__ bool store_needs_barrier(const dq_block *__restrict__ blk) {
+__device__ __forceinline__ bool store_needs_barrier(CBlock blk) {
     if (blk->phase_count != 1) return false;
     bool x = false;
 #pragma unroll
@@ -328,23 +347,60 @@ __device__ __forceinline__ void process_tile(Regs<T, R> &a, const dq_phase *__re
     }
 }
 
+// Brings a block's device program and exchange tables into this XCD's L2 while
+// the tile is still on its way: they are read line by line, each read waiting
+// for the one before, and the first workgroups of a launch would wait for
+// memory at every line.  With the argument-borne descriptors below, measured
+// per sweep before -> now: 17 qubits FP32 R = 3, W = 0 9.6 -> 6.5 us; 16 tiles of
+// 12 bits FP32 19.2 -> 12.4 us; one tile of 10 bits with a whole circuit
+// 155 -> 71 us; 21 qubits FP64 R = 4, W = 3 38 -> 27 us.  Loading the program's
+// lines into the scalar cache as well gained nothing on top.  (Relaxed atomic loads: a plain load whose result
+// nothing uses would be dropped.)
+__device__ __forceinline__ void warm_lines(const unsigned char *p, uint32_t bytes, uint32_t tid, uint32_t threads) {
+    for (uint32_t i = tid * 128u; i < bytes; i += threads * 128u)
+        (void)__hip_atomic_load(reinterpret_cast<const uint32_t *>(p + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
+// A launch of one job reads it, its block and block_aux from the kernel's
+// arguments (`one`): the tile's addresses are then one memory latency away
+// instead of three (argument, job, block).  A batch reads them per job.
 template <typename T, int R, int W, int XM>
 __global__ void __launch_bounds__(64 << W, (sweep_waves_per_eu<T, R, XM>()))
-sweep_kernel(const dq_job *__restrict__ jobs, const dq_block *__restrict__ blocks,
+sweep_kernel(const SweepOne one, const dq_job *__restrict__ jobs, const dq_block *__restrict__ blocks,
              const dq_phase *__restrict__ phases, const unsigned char *__restrict__ prog,
              const uint32_t *__restrict__ phase_aux, const uint32_t *__restrict__ block_aux) {
     using GV = __attribute__((address_space(1))) typename V2<T>::type;
-    const dq_job job = jobs[blockIdx.y];
-    const dq_block *__restrict__ blk = blocks + job.block;
-    GV *__restrict__ st = (GV *)(job.state);
+    (void)one;
+    const auto *ka = (const DQ_CONST SweepOne *)__builtin_amdgcn_kernarg_segment_ptr();
+    CBlock blk = &ka->blk;
+    CWords ba = ka->baux;
+    void *state = ka->job.state;
+    uint64_t hi = ka->job.base_hi;
+    if (gridDim.y > 1) {
+        const auto *job = (const DQ_CONST dq_job *)(uintptr_t)(jobs + blockIdx.y);
+        blk = (CBlock)(uintptr_t)(blocks + job->block);
+        ba = (CWords)(uintptr_t)(block_aux + job->block * DQ_BAUX);
+        state = job->state;
+        hi = job->base_hi;
+    }
+    GV *__restrict__ st = (GV *)(state);
     const uint32_t tid = threadIdx.x;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lane = tid & 63u;
-    const uint64_t base = tile_base_runs(block_aux + job.block * DQ_BAUX, blockIdx.x);
+    const uint64_t base = tile_base_runs(ba, blockIdx.x);
+    const uint32_t *pa = phase_aux + blk->phase_begin * DQ_PAUX;
+    if (blockIdx.x < DQ_WARM_TILES) {
+        warm_lines(prog + ba[DQ_BA_PROG], ba[DQ_BA_PROG + 1], tid, 64u << W);
+        if (blk->phase_count > 1)
+            warm_lines(reinterpret_cast<const unsigned char *>(pa), blk->phase_count * DQ_PAUX * 4u, tid, 64u << W);
+    }
     Regs<T, R> a;
     load_tile<T, R, W>(a, blk, st, base, wv, lane);
-    process_tile<T, R, W, XM>(a, phases + blk->phase_begin, blk->phase_count, phase_aux + blk->phase_begin * DQ_PAUX,
-                                 prog, base | job.base_hi, tid, wv, false);
+    // an opaque copy: knowing the count again after the loop, the compiler
+    // would keep a second copy of the tile for blocks of one phase
+    uint32_t nph = blk->phase_count;
+    asm volatile("" : "+s"(nph));
+    process_tile<T, R, W, XM>(a, phases + blk->phase_begin, nph, pa, prog, base | hi, tid, wv, false);
     if (store_needs_barrier<W>(blk)) __syncthreads();
     DQ_STORE_TILE(a, base);
 }
@@ -1167,7 +1223,7 @@ __global__ void fill_kernel(typename V2<T>::type *__restrict__ st, uint64_t N, i
 // ----------------------------------------------------------------------------
 // kernel table
 // ----------------------------------------------------------------------------
-typedef void (*sweep_fn)(const dq_job *, const dq_block *, const dq_phase *, const unsigned char *, const uint32_t *,
+typedef void (*sweep_fn)(const SweepOne, const dq_job *, const dq_block *, const dq_phase *, const unsigned char *, const uint32_t *,
                          const uint32_t *);
 
 template <typename T>
@@ -2121,6 +2177,8 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
             return fail(DQ_ERR_UNSUPPORTED, "block %u: non-tile qubits in more than %d runs", i, DQ_RUNS);
         const int bxm = exchange_mode(prec, (int)b.reg_bits, (int)b.wave_bits, (int)b.tile_bits);
         const uint32_t es = exchange_elem_bytes(prec, bxm);
+        uint32_t *ba = baux.data() + (size_t)i * DQ_BAUX;
+        ba[DQ_BA_PROG] = (uint32_t)prog.size();
         uint32_t gown[32];
         if (bxm == 1) {
             if (b.tile_bits != 6 + b.wave_bits + b.reg_bits)
@@ -2178,6 +2236,7 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
                 pa[DQ_TB + 6 + w] = swizzle_host(B.wave_t[w], g, L) * es;
             }
         }
+        ba[DQ_BA_PROG + 1] = (uint32_t)prog.size() - ba[DQ_BA_PROG];  // 0 when the phases are an earlier block's
     }
     if (prog.size() + 256 > prog_bound(n_phases, n_ops)) return fail(DQ_ERR_ARG, "dq_apply_blocks: device program overflow");
 
@@ -2229,7 +2288,11 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
                 return fail(DQ_ERR_UNSUPPORTED, "grid too large (at most 2^32 threads per launch)");
             sweep_fn fn = lookup(prec, b0.reg_bits, b0.wave_bits, xm);
             if (!fn) return fail(DQ_ERR_UNSUPPORTED, "no sweep kernel for R=%u W=%u exchange mode %d", b0.reg_bits, b0.wave_bits, xm);
-            hipLaunchKernelGGL(fn, dim3((unsigned)tiles, nj), dim3(64u << b0.wave_bits), lds, (hipStream_t)stream,
+            SweepOne one;
+            one.blk = b0;
+            memcpy(one.baux, baux.data() + (size_t)jobs[j0].block * DQ_BAUX, sizeof one.baux);
+            one.job = jobs[j0];
+            hipLaunchKernelGGL(fn, dim3((unsigned)tiles, nj), dim3(64u << b0.wave_bits), lds, (hipStream_t)stream, one,
                                d_jobs + j0, d_blocks, d_phases, d_prog, d_paux, d_baux);
         }
         HIPC(hipGetLastError());
