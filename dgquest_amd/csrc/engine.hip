@@ -1160,6 +1160,87 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
     }
 }
 
+// Matrices of dense ops as products of gates, formed in FP64 and written in the
+// MFMA operand order of dense_op.  A column (the image of one basis state) takes
+// one wave, 2^k / 64 amplitudes a lane, two columns a wave for k = 5; a gate is a
+// 2x2 on one index bit, its partner amplitude a lane exchange away.  Grid
+// (2^k / columns per workgroup, matrices).  Latency-bound (a few gates' lane
+// exchanges, every matrix at once).  On the host, gate by gate and column by
+// column, the 42 matrices of a 25-qubit grid circuit (k = 7) took 14-17 of the
+// 28.7-31.8 ms of a flush and were uploaded (11 MB); the flush now takes 14.7 ms.
+template <int KL>
+__global__ void __launch_bounds__(256)
+dense_form(const dq_small_gate *__restrict__ gates, const uint32_t *__restrict__ begin, float *__restrict__ mats) {
+    constexpr int K = 1 << KL, M = 2 * K;
+    constexpr int J = KL == 7 ? 2 : 1;      // amplitudes per lane
+    constexpr int CW = KL == 5 ? 2 : 1;     // columns per wave
+    constexpr uint32_t LN = 64 / CW;        // lanes per column
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63u;
+    const uint32_t i0 = lane & (LN - 1);
+    const uint32_t c = (blockIdx.x * 4 + w) * CW + lane / LN;
+    double re[J], im[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        re[j] = i0 + LN * j == c ? 1.0 : 0.0;
+        im[j] = 0.0;
+    }
+    const uint32_t g1 = begin[blockIdx.y + 1];
+    for (uint32_t g = begin[blockIdx.y]; g < g1; g++) {
+        const dq_small_gate *__restrict__ G = gates + g;
+        const uint32_t tm = G->tmask, cm = G->cmask;
+        double u[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) u[i] = G->u[i];
+        if (G->diag) {
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                if (((i0 + LN * j) & cm) == cm) {
+                    const double r = re[j], x = im[j];
+                    re[j] = u[0] * r - u[1] * x;
+                    im[j] = u[0] * x + u[1] * r;
+                }
+            continue;
+        }
+        double pr[J], pi[J];
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            if (tm < LN) {
+                pr[j] = __shfl_xor(re[j], (int)tm, 64);
+                pi[j] = __shfl_xor(im[j], (int)tm, 64);
+            } else {
+                pr[j] = re[J - 1 - j];
+                pi[j] = im[J - 1 - j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < J; j++) {
+            const uint32_t i = i0 + LN * j;
+            const bool hi = (i & tm) != 0;
+            const double r0 = hi ? pr[j] : re[j], m0 = hi ? pi[j] : im[j];
+            const double r1 = hi ? re[j] : pr[j], m1 = hi ? im[j] : pi[j];
+            const double ar = hi ? u[4] : u[0], ai = hi ? u[5] : u[1], br = hi ? u[6] : u[2], bi = hi ? u[7] : u[3];
+            if ((i & cm) == cm) {
+                re[j] = ar * r0 - ai * m0 + br * r1 - bi * m1;
+                im[j] = ar * m0 + ai * r0 + br * m1 + bi * r1;
+            }
+        }
+    }
+    float *__restrict__ D = mats + (size_t)blockIdx.y * ((size_t)M * M);
+    auto put = [&](uint32_t row, uint32_t col, float v) {  // real matrix element (row, col)
+        const uint32_t rb = row >> 5, l = (row & 31u) | ((col & 1u) << 5), p = col >> 1;
+        D[(((size_t)rb * (M / 8) + p / 4) * 64 + l) * 4 + p % 4] = v;
+    };
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const uint32_t r = i0 + LN * j;
+        const float a = (float)re[j], b = (float)im[j];
+        put(r, c, a);
+        put(r, K + c, -b);
+        put(K + r, c, b);
+        put(K + r, K + c, a);
+    }
+}
+
 // one workgroup: out = {re <a|b>, im <a|b>, <a|a>, <b|b>, max |a_i - b_i|}
 __global__ void __launch_bounds__(256) compare_stage2(const double *__restrict__ part, uint32_t ngroups, double *__restrict__ out) {
     __shared__ double red[4][CMP_SLOTS];
@@ -2593,14 +2674,9 @@ extern "C" size_t dq_dense_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, ui
            align_up((size_t)n_ops * DENSE_COLS * sizeof(uint32_t), 256);
 }
 
-extern "C" int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops,
-                              uint32_t n_ops, const double *mats, uint32_t n_mats, void *state, void *d_ws,
-                              size_t ws_bytes, void *stream) {
-    if (k < 5 || k > 7) return fail(DQ_ERR_ARG, "dq_apply_dense: k must be 5, 6 or 7");
-    if (!blocks || !state || !d_ws || (n_ops && !ops) || (n_mats && !mats))
-        return fail(DQ_ERR_ARG, "dq_apply_dense: null argument");
-    const size_t need = dq_dense_ws_bytes(k, n_blocks, n_ops, n_mats);
-    if (ws_bytes < need) return fail(DQ_ERR_ARG, "dq_apply_dense: workspace %zu < %zu bytes", ws_bytes, need);
+// Host-side check of dense blocks and ops against the kernel's grid and tile.
+static int validate_dense(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops, uint32_t n_ops,
+                          uint32_t n_mats) {
     for (uint32_t i = 0; i < n_blocks; i++) {
         const dq_dense_block &b = blocks[i];
         const uint32_t n = b.n_qubits, T = b.tile_bits;
@@ -2623,7 +2699,60 @@ extern "C" int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_bl
         }
         if (n - T > 31) return fail(DQ_ERR_UNSUPPORTED, "dense block %u: grid too large", i);
     }
-    // upload: blocks | ops | real matrices in MFMA operand order
+    return DQ_OK;
+}
+
+// Per op: column c's tile offset, c's bits placed on the block's tile bits
+// outside the op (in ascending order).
+static int dense_columns(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops, uint32_t n_ops,
+                         uint32_t *ct) {
+    std::vector<int> op_T(n_ops, -1);
+    for (uint32_t i = 0; i < n_blocks; i++) {
+        const uint32_t T = blocks[i].tile_bits;
+        for (uint32_t o = blocks[i].op_begin; o < blocks[i].op_begin + blocks[i].op_count; o++) {
+            if (op_T[o] >= 0 && op_T[o] != (int)T) return fail(DQ_ERR_ARG, "dense op %u: in blocks of different tiles", o);
+            op_T[o] = (int)T;
+            uint32_t used = 0, cb[DENSE_T_MAX];
+            for (int j = 0; j < k; j++) used |= 1u << ops[o].bits[j];
+            int nc = 0;
+            for (uint32_t b = 0; b < T; b++)
+                if (!((used >> b) & 1u)) cb[nc++] = b;
+            for (uint32_t c = 0; c < (1u << nc); c++) {
+                uint32_t v = 0;
+                for (int b = 0; b < nc; b++) v |= ((c >> b) & 1u) << cb[b];
+                ct[(size_t)o * DENSE_COLS + c] = v;
+            }
+        }
+    }
+    return DQ_OK;
+}
+
+static int dense_launch(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_block *d_blocks,
+                        const dq_dense_op *d_ops, const float *d_mats, const uint32_t *d_ct, void *state, hipStream_t s) {
+    auto *st = (typename V2<float>::type *)state;
+    for (uint32_t i = 0; i < n_blocks; i++) {
+        const dq_dense_block &b = blocks[i];
+        const unsigned grid = 1u << (b.n_qubits - b.tile_bits);
+        const size_t lds = dense_lds_bytes(b.tile_bits);
+        if (k == 5) hipLaunchKernelGGL(dense_kernel<5>, dim3(grid), dim3(DENSE_THREADS), lds, s, d_blocks + i, d_ops, d_mats, d_ct, st);
+        else if (k == 6) hipLaunchKernelGGL(dense_kernel<6>, dim3(grid), dim3(DENSE_THREADS), lds, s, d_blocks + i, d_ops, d_mats, d_ct, st);
+        else hipLaunchKernelGGL(dense_kernel<7>, dim3(grid), dim3(DENSE_THREADS), lds, s, d_blocks + i, d_ops, d_mats, d_ct, st);
+        HIPC(hipGetLastError());
+    }
+    return DQ_OK;
+}
+
+extern "C" int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops,
+                              uint32_t n_ops, const double *mats, uint32_t n_mats, void *state, void *d_ws,
+                              size_t ws_bytes, void *stream) {
+    if (k < 5 || k > 7) return fail(DQ_ERR_ARG, "dq_apply_dense: k must be 5, 6 or 7");
+    if (!blocks || !state || !d_ws || (n_ops && !ops) || (n_mats && !mats))
+        return fail(DQ_ERR_ARG, "dq_apply_dense: null argument");
+    const size_t need = dq_dense_ws_bytes(k, n_blocks, n_ops, n_mats);
+    if (ws_bytes < need) return fail(DQ_ERR_ARG, "dq_apply_dense: workspace %zu < %zu bytes", ws_bytes, need);
+    int rc = validate_dense(k, blocks, n_blocks, ops, n_ops, n_mats);
+    if (rc) return rc;
+    // upload: blocks | ops | real matrices in MFMA operand order | column tables
     const size_t ob = align_up(n_blocks * sizeof(dq_dense_block), 256);
     const size_t mo = ob + align_up(n_ops * sizeof(dq_dense_op), 256);
     const int K = 1 << k, M = 2 * K;
@@ -2647,46 +2776,83 @@ extern "C" int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_bl
                     D[(((size_t)rb * (M / 8) + p / 4) * 64 + l) * 4 + p % 4] = (float)a;
                 }
     }
-    // per op: column c's tile offset, c's bits placed on the block's tile bits
-    // outside the op (in ascending order)
-    uint32_t *ct = reinterpret_cast<uint32_t *>(buf.data() + co);
-    std::vector<int> op_T(n_ops, -1);
-    for (uint32_t i = 0; i < n_blocks; i++) {
-        const uint32_t T = blocks[i].tile_bits;
-        for (uint32_t o = blocks[i].op_begin; o < blocks[i].op_begin + blocks[i].op_count; o++) {
-            if (op_T[o] >= 0 && op_T[o] != (int)T) return fail(DQ_ERR_ARG, "dense op %u: in blocks of different tiles", o);
-            op_T[o] = (int)T;
-            uint32_t used = 0, cb[DENSE_T_MAX];
-            for (int j = 0; j < k; j++) used |= 1u << ops[o].bits[j];
-            int nc = 0;
-            for (uint32_t b = 0; b < T; b++)
-                if (!((used >> b) & 1u)) cb[nc++] = b;
-            for (uint32_t c = 0; c < (1u << nc); c++) {
-                uint32_t v = 0;
-                for (int b = 0; b < nc; b++) v |= ((c >> b) & 1u) << cb[b];
-                ct[(size_t)o * DENSE_COLS + c] = v;
-            }
-        }
-    }
-    int rc = stage_upload(d_ws, buf, stream);
+    rc = dense_columns(k, blocks, n_blocks, ops, n_ops, reinterpret_cast<uint32_t *>(buf.data() + co));
+    if (rc) return rc;
+    rc = stage_upload(d_ws, buf, stream);
     if (rc) return rc;
     unsigned char *d = (unsigned char *)d_ws;
-    const dq_dense_block *d_blocks = (const dq_dense_block *)d;
-    const dq_dense_op *d_ops = (const dq_dense_op *)(d + ob);
-    const float *d_mats = (const float *)(d + mo);
-    const uint32_t *d_ct = (const uint32_t *)(d + co);
+    return dense_launch(k, blocks, n_blocks, (const dq_dense_block *)d, (const dq_dense_op *)(d + ob), (const float *)(d + mo),
+                        (const uint32_t *)(d + co), state, (hipStream_t)stream);
+}
+
+namespace {
+// Workspace of dq_apply_dense_gates: what is uploaded (blocks | ops | column
+// tables | gates | first gate of each matrix), then the matrices.
+struct DenseGatesWs {
+    size_t ops, cols, gates, begin, upload, mats, total;
+};
+DenseGatesWs dense_gates_ws(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats, uint32_t n_gates) {
+    DenseGatesWs w;
+    w.ops = align_up(n_blocks * sizeof(dq_dense_block), 256);
+    w.cols = w.ops + align_up(n_ops * sizeof(dq_dense_op), 256);
+    w.gates = w.cols + align_up((size_t)n_ops * DENSE_COLS * sizeof(uint32_t), 256);
+    w.begin = w.gates + align_up((size_t)n_gates * sizeof(dq_small_gate), 256);
+    w.upload = w.begin + ((size_t)n_mats + 1) * sizeof(uint32_t);
+    w.mats = align_up(w.upload, 256);
+    w.total = w.mats + (size_t)n_mats * dense_mat_floats(k) * sizeof(float);
+    return w;
+}
+}  // namespace
+
+extern "C" size_t dq_dense_gates_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats, uint32_t n_gates) {
+    if (k < 5 || k > 7) return 0;
+    return dense_gates_ws(k, n_blocks, n_ops, n_mats, n_gates).total;
+}
+
+extern "C" int dq_apply_dense_gates(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops,
+                                    uint32_t n_ops, const dq_small_gate *gates, const uint32_t *gate_begin, uint32_t n_mats,
+                                    void *state, void *d_ws, size_t ws_bytes, void *stream) {
+    if (k < 5 || k > 7) return fail(DQ_ERR_ARG, "dq_apply_dense_gates: k must be 5, 6 or 7");
+    if (!blocks || !state || !d_ws || !gate_begin || (n_ops && !ops)) return fail(DQ_ERR_ARG, "dq_apply_dense_gates: null argument");
+    for (uint32_t i = 0; i < n_mats; i++)
+        if (gate_begin[i + 1] < gate_begin[i]) return fail(DQ_ERR_ARG, "dq_apply_dense_gates: gate ranges not ascending");
+    const uint32_t n_gates = gate_begin[n_mats];
+    if (n_gates && !gates) return fail(DQ_ERR_ARG, "dq_apply_dense_gates: null argument");
+    for (uint32_t i = 0; i < n_gates; i++) {
+        const dq_small_gate &g = gates[i];
+        const bool one = g.tmask && !(g.tmask & (g.tmask - 1));
+        if (((g.tmask | g.cmask) >> k) || (g.tmask & g.cmask) || g.diag > 1 || (g.diag ? g.tmask != 0 : !one))
+            return fail(DQ_ERR_ARG, "dq_apply_dense_gates: gate %u: bad bits", i);
+    }
+    const DenseGatesWs w = dense_gates_ws(k, n_blocks, n_ops, n_mats, n_gates);
+    if (ws_bytes < w.total) return fail(DQ_ERR_ARG, "dq_apply_dense_gates: workspace %zu < %zu bytes", ws_bytes, w.total);
+    int rc = validate_dense(k, blocks, n_blocks, ops, n_ops, n_mats);
+    if (rc) return rc;
+    std::vector<unsigned char> buf(w.upload, 0);
+    memcpy(buf.data(), blocks, n_blocks * sizeof(dq_dense_block));
+    if (n_ops) memcpy(buf.data() + w.ops, ops, n_ops * sizeof(dq_dense_op));
+    rc = dense_columns(k, blocks, n_blocks, ops, n_ops, reinterpret_cast<uint32_t *>(buf.data() + w.cols));
+    if (rc) return rc;
+    if (n_gates) memcpy(buf.data() + w.gates, gates, n_gates * sizeof(dq_small_gate));
+    memcpy(buf.data() + w.begin, gate_begin, ((size_t)n_mats + 1) * sizeof(uint32_t));
+    rc = stage_upload(d_ws, buf, stream);
+    if (rc) return rc;
+    unsigned char *d = (unsigned char *)d_ws;
     hipStream_t s = (hipStream_t)stream;
-    for (uint32_t i = 0; i < n_blocks; i++) {
-        const dq_dense_block &b = blocks[i];
-        const unsigned grid = 1u << (b.n_qubits - b.tile_bits);
-        const size_t lds = dense_lds_bytes(b.tile_bits);
-        auto *st = (typename V2<float>::type *)state;
-        if (k == 5) hipLaunchKernelGGL(dense_kernel<5>, dim3(grid), dim3(DENSE_THREADS), lds, s, d_blocks + i, d_ops, d_mats, d_ct, st);
-        else if (k == 6) hipLaunchKernelGGL(dense_kernel<6>, dim3(grid), dim3(DENSE_THREADS), lds, s, d_blocks + i, d_ops, d_mats, d_ct, st);
-        else hipLaunchKernelGGL(dense_kernel<7>, dim3(grid), dim3(DENSE_THREADS), lds, s, d_blocks + i, d_ops, d_mats, d_ct, st);
+    const auto *d_gates = (const dq_small_gate *)(d + w.gates);
+    const auto *d_begin = (const uint32_t *)(d + w.begin);
+    float *d_mats = (float *)(d + w.mats);
+    for (uint32_t m0 = 0; m0 < n_mats; m0 += 65535u) {
+        const uint32_t nm = std::min(n_mats - m0, 65535u);
+        const uint32_t *gb = d_begin + m0;
+        float *dm = d_mats + (size_t)m0 * dense_mat_floats(k);
+        if (k == 5) hipLaunchKernelGGL(dense_form<5>, dim3(4, nm), dim3(256), 0, s, d_gates, gb, dm);
+        else if (k == 6) hipLaunchKernelGGL(dense_form<6>, dim3(16, nm), dim3(256), 0, s, d_gates, gb, dm);
+        else hipLaunchKernelGGL(dense_form<7>, dim3(32, nm), dim3(256), 0, s, d_gates, gb, dm);
         HIPC(hipGetLastError());
     }
-    return DQ_OK;
+    return dense_launch(k, blocks, n_blocks, (const dq_dense_block *)d, (const dq_dense_op *)(d + w.ops), d_mats,
+                        (const uint32_t *)(d + w.cols), state, s);
 }
 
 extern "C" int dq_event_query(void *ev) {

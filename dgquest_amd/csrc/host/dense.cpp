@@ -101,11 +101,37 @@ void op_matrix(const std::vector<Gate> &gs, const int *q, int k, double *out) {
     }
 }
 
+// The same gate as a factor for the device: masks over the positions q, the
+// arithmetic of apply_gate_small as a 2x2 matrix or a phase.
+dq_small_gate small_gate(const Gate &g, const int *q, int k) {
+    dq_small_gate s;
+    memset(&s, 0, sizeof s);
+    s.tmask = (uint32_t)to_local(g.tmask, q, k);
+    s.cmask = (uint32_t)to_local(g.cmask, q, k);
+    if (g.type <= OP_PHASE_SHIFT) {
+        static const double pr[8] = {1, kR2, 0, -kR2, -1, -kR2, 0, kR2};
+        static const double pi[8] = {0, kR2, 1, kR2, 0, -kR2, -1, -kR2};
+        s.diag = 1;
+        s.u[0] = g.type == OP_PHASE_SHIFT ? std::cos(g.op[0]) : pr[g.type];
+        s.u[1] = g.type == OP_PHASE_SHIFT ? std::sin(g.op[0]) : pi[g.type];
+    } else if (g.type == OP_COLLAPSE) {
+        s.u[g.op[0] != 0.0 ? 6 : 0] = g.op[1];
+    } else if (g.type == OP_ROTATE_Z) {
+        s.u[0] = s.u[6] = std::cos(g.op[0]);
+        s.u[7] = std::sin(g.op[0]);
+        s.u[1] = -s.u[7];
+    } else {
+        gate_matrix(g, s.u);
+    }
+    return s;
+}
+
 }  // namespace
 
-bool plan_dense(const std::vector<Gate> &gates, int n, int k, DensePlan &P, std::string &err) {
+bool plan_dense(const std::vector<Gate> &gates, int n, int k, DensePlan &P, std::string &err, bool form) {
     P = DensePlan();
     P.k = k;
+    P.gate_begin.push_back(0);
     if (k < 5 || k > 7) { err = "dense width k must be 5, 6 or 7"; return false; }
     const int T = n < 13 ? n : 13;
     if (T < k + 5) { err = "register too small for dense sweeps of this width"; return false; }
@@ -156,9 +182,14 @@ bool plan_dense(const std::vector<Gate> &gates, int n, int k, DensePlan &P, std:
                 P.op_qubits.push_back(q[i]);
             }
             op.mat = P.ops.size();
-            const size_t mo = P.mats.size();
-            P.mats.resize(mo + 2 * K * K);
-            op_matrix(og, q, k, P.mats.data() + mo);
+            if (form) {
+                const size_t mo = P.mats.size();
+                P.mats.resize(mo + 2 * K * K);
+                op_matrix(og, q, k, P.mats.data() + mo);
+            }
+            for (const Gate &g : og)
+                if (g.type != OP_ONE && g.type != OP_ROTATE_Z_FAKE) P.gates.push_back(small_gate(g, q, k));
+            P.gate_begin.push_back((uint32_t)P.gates.size());
             P.ops.push_back(op);
             P.flops += 8.0 * (double)K * std::ldexp(1.0, n);
         }

@@ -22,13 +22,17 @@ struct DensePlan {
     std::vector<dq_dense_block> blocks;
     std::vector<dq_dense_op> ops;
     std::vector<int> op_qubits;   // k qubits per op: matrix-index bit j acts on op_qubits[k * op + j]
-    std::vector<double> mats;     // per op: 2^k x 2^k row-major {re, im}
+    std::vector<double> mats;     // per op: 2^k x 2^k row-major {re, im} (plan_dense with form = true)
+    std::vector<dq_small_gate> gates;   // the factors of every op's matrix in order, over its k bits
+    std::vector<uint32_t> gate_begin;   // op i: gates gate_begin[i] .. gate_begin[i + 1] - 1
     double flops = 0.0;           // real flops of the device GEMMs: 8 * 2^k * 2^n per op
 };
 
 // False (with err) when the register is too small for dense sweeps of width
-// k (k + 5 <= min(n, 13) is needed) or k is not 5, 6 or 7.
-bool plan_dense(const std::vector<Gate> &gates, int n, int k, DensePlan &out, std::string &err);
+// k (k + 5 <= min(n, 13) is needed) or k is not 5, 6 or 7.  The matrices
+// themselves are formed here only with form = true; a flush leaves that to the
+// device (dq_apply_dense_gates).
+bool plan_dense(const std::vector<Gate> &gates, int n, int k, DensePlan &out, std::string &err, bool form = true);
 
 // Apply one recorded gate to a state of m qubits held as interleaved
 // {re, im} doubles, gate masks already in this state's bit positions.  The

@@ -320,11 +320,12 @@ void flush(QuregState *s) {
         }
         DensePlan D;
         std::string err;
-        if (!plan_dense(s->pending, s->n, s->dense_k, D, err)) engine_fatal(("dense planning: " + err).c_str(), DQ_ERR_ARG);
+        if (!plan_dense(s->pending, s->n, s->dense_k, D, err, false))
+            engine_fatal(("dense planning: " + err).c_str(), DQ_ERR_ARG);
         const uint32_t nb = (uint32_t)D.blocks.size(), no = (uint32_t)D.ops.size();
-        ensure_ws(s, dq_dense_ws_bytes(s->dense_k, nb, no, no));
-        ENG(dq_apply_dense(s->dense_k, D.blocks.data(), nb, D.ops.data(), no, D.mats.data(), no, s->d_state, s->d_ws,
-                           s->ws_cap, s->stream));
+        ensure_ws(s, dq_dense_gates_ws_bytes(s->dense_k, nb, no, no, (uint32_t)D.gates.size()));
+        ENG(dq_apply_dense_gates(s->dense_k, D.blocks.data(), nb, D.ops.data(), no, D.gates.data(), D.gate_begin.data(), no,
+                                 s->d_state, s->d_ws, s->ws_cap, s->stream));
         s->last_stats = PlanStats();
         s->last_stats.sweeps = (int)nb;
         s->last_stats.ops = (int)no;

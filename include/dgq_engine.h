@@ -266,6 +266,27 @@ int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_blocks, const
                    const double *mats, uint32_t n_mats, void *state, void *d_ws, size_t ws_bytes, void *stream);
 size_t dq_dense_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats);
 
+/* One factor of a dense op's matrix, over the k matrix-index bits.  diag = 0:
+ * the 2x2 complex matrix u (u00, u01, u10, u11 as re, im) on the bit tmask
+ * where all bits of cmask are 1; diag = 1: amplitudes whose bits of cmask are
+ * all 1 times (u[0], u[1]), tmask 0. */
+typedef struct dq_small_gate {
+    uint32_t tmask;
+    uint32_t cmask;
+    uint32_t diag;
+    uint32_t pad;
+    double u[8];
+} dq_small_gate;
+
+/* dq_apply_dense with the matrices formed on the device: matrix i is the
+ * product of gates[gate_begin[i]] .. gates[gate_begin[i + 1] - 1], applied in
+ * that order (gate_begin has n_mats + 1 entries), computed in FP64 and rounded
+ * to float once. */
+int dq_apply_dense_gates(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops, uint32_t n_ops,
+                         const dq_small_gate *gates, const uint32_t *gate_begin, uint32_t n_mats, void *state, void *d_ws,
+                         size_t ws_bytes, void *stream);
+size_t dq_dense_gates_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats, uint32_t n_gates);
+
 /* Read-out of `count` states of n qubits each (device pointers in the host
  * array states[]): for every state, P(qubit q = 0) for q < n and the total
  * probability (n + 1 doubles at d_p0 + i * (n + 1); skipped when d_p0 is
