@@ -70,6 +70,10 @@ GATE_SIGNATURES = {
 
 _NREALS = {"r": 1, "c": 2, "m": 8, "v": 3}
 
+# argument shapes that pyrecord.cpp records (its enum Shape, in order)
+_RECORD_SHAPES = [("q",), ("q", "r"), ("q", "r", "r"), ("q", "r", "r", "r"), ("q", "q"), ("q", "q", "r"),
+                  ("q", "q", "r", "r")]
+
 
 def _descriptor_dtypes():
     """numpy layouts of dq_block, dq_phase and dq_op (include/dgq_engine.h)."""
@@ -186,6 +190,16 @@ class QuEST:
         L.dgq_recorder_plan_dense.argtypes = [Qureg, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                               C.c_void_p, C.c_void_p]
 
+        # circuits are recorded natively (csrc/host/pyrecord.cpp): gate name -> (argument shape, C function)
+        rec = os.path.join(libdir, "libdgq_pyrecord.so")
+        if not os.path.exists(rec):
+            raise RuntimeError(f"{rec} is not built; run dgquest_amd.build.build()")
+        self._record = C.PyDLL(rec).dgq_py_record
+        self._record.restype = C.py_object
+        self._record.argtypes = [C.py_object, C.py_object, C.c_int, C.POINTER(Qureg), C.py_object]
+        self._record_table = {g: (_RECORD_SHAPES.index(ks), C.cast(getattr(L, g), C.c_void_p).value)
+                              for g, ks in GATE_SIGNATURES.items() if ks in _RECORD_SHAPES}
+
     # --- thin pass-throughs -------------------------------------------------
     def __getattr__(self, name):
         return getattr(self.lib, name)
@@ -228,8 +242,13 @@ class QuEST:
         getattr(self.lib, name)(*args)
 
     def apply_circuit(self, q: Qureg, circuit: Iterable):
-        for g in circuit:
+        """Apply every (name, qubits[, params]) entry of `circuit` in order, each as apply() does."""
+
+        def one(g):
             self.apply(q, g[0], g[1], g[2] if len(g) > 2 else ())
+
+        table = self._record_table if type(self).apply is QuEST.apply and "apply" not in self.__dict__ else {}
+        self._record(table, one, self.prec, C.byref(q), circuit)
 
     def seed(self, keys: Sequence[int]):
         arr = (C.c_ulong * len(keys))(*keys)
