@@ -635,6 +635,73 @@ __global__ void __launch_bounds__(256) prob_stage2(const double *__restrict__ pa
     if (tid == 0) out[q] = bit == PROB_FIXED1 ? 0.0 : po.scale * ((red[0] + red[1]) + (red[2] + red[3]));
 }
 
+// Both stages in one launch of one workgroup of 16 waves, for up to 2^PROB_ONE_BITS
+// amplitudes: number bits 0..5 lane, 6..9 wave, 10.. load index.
+#define PROB_ONE_BITS 13
+
+template <typename T>
+__global__ void __launch_bounds__(1024)
+prob_one(const typename V2<T>::type *__restrict__ st, const ProbBits pb, int nf, int n, const ProbOut po,
+         double *__restrict__ out) {
+    using V = typename V2<T>::type;
+    constexpr int JB = PROB_ONE_BITS - 10, J = 1 << JB;
+    __shared__ double red[16][6 + JB + 1];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint64_t base = pb.fixed;
+#pragma unroll
+    for (int i = 0; i < 4; i++) base |= ((w >> i) & 1u) ? pb.img[6 + i] : 0ull;
+    uint64_t lp = 0;
+#pragma unroll
+    for (int i = 0; i < 6; i++) lp |= ((lane >> i) & 1u) ? pb.img[i] : 0ull;
+    const bool on = nf >= 10 || (tid >> nf) == 0;
+    const int nj = nf > 10 ? nf - 10 : 0;
+    V v[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        uint64_t u = base;  // img is 0 past the last number bit: the loads j >> nj repeat an amplitude
+#pragma unroll
+        for (int b = 0; b < JB; b++)
+            if ((j >> b) & 1) u |= pb.img[10 + b];
+        v[j] = st[u + lp];
+    }
+    double t = 0.0, zj[JB];
+#pragma unroll
+    for (int b = 0; b < JB; b++) zj[b] = 0.0;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const double p = on && (j >> nj) == 0 ? (double)v[j].x * (double)v[j].x + (double)v[j].y * (double)v[j].y : 0.0;
+        t += p;
+#pragma unroll
+        for (int b = 0; b < JB; b++)
+            if (!((j >> b) & 1)) zj[b] += p;
+    }
+#pragma unroll
+    for (int q = 0; q < 6; q++) {  // as in prob_stage1
+        double r = t;
+#pragma unroll
+        for (int k = q + 1; k < 6; k++) r += __shfl_xor(r, 1 << k, 64);
+        if (lane == 0) red[w][q] = r;
+        t += __shfl_xor(t, 1 << q, 64);
+    }
+    if (lane == 0) red[w][6 + JB] = t;
+#pragma unroll
+    for (int b = 0; b < JB; b++) {
+        const double r = wave_sum(zj[b]);
+        if (lane == 0) red[w][6 + b] = r;
+    }
+    __syncthreads();
+    const int q = (int)tid;
+    if (q > n) return;
+    const int bit = q == n ? PROB_FIXED0 : po.bit[q];
+    const int slot = bit < 6 ? bit : bit >= 10 && bit < PROB_FIXED0 ? bit - 4 : 6 + JB;
+    const uint32_t skip = bit >= 6 && bit < 10 ? 1u << (bit - 6) : 0u;
+    double acc = 0.0;
+#pragma unroll
+    for (uint32_t g = 0; g < 16; g++) acc += (g & skip) ? 0.0 : red[g][slot];
+    out[q] = bit == PROB_FIXED1 ? 0.0 : po.scale * acc;
+}
+
 // The read-out of many states and the comparison split a state in chunks of
 // 2^PROB_WG_BITS amplitudes per workgroup.
 #define PROB_WG_BITS 16
@@ -1265,14 +1332,20 @@ __global__ void __launch_bounds__(256) compare_stage2(const double *__restrict__
 // ----------------------------------------------------------------------------
 // amplitude gather / scatter / fill
 // ----------------------------------------------------------------------------
+// The qubit map travels in the arguments: a staged upload of it took longer
+// than the kernel.
+struct QubitMap {
+    uint8_t l2p[40];
+};
+
 template <typename T>
-__global__ void read_kernel(const typename V2<T>::type *__restrict__ st, int n, const int *__restrict__ l2p,
+__global__ void read_kernel(const typename V2<T>::type *__restrict__ st, int n, const QubitMap map,
                             uint64_t start, uint64_t count, double *__restrict__ out) {
     const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= count) return;
     const uint64_t li = start + k;
     uint64_t pi = 0;
-    for (int q = 0; q < n; q++) pi |= ((li >> q) & 1ull) << l2p[q];
+    for (int q = 0; q < n; q++) pi |= ((li >> q) & 1ull) << map.l2p[q];
     const typename V2<T>::type v = st[pi];
     out[2 * k] = (double)v.x;
     out[2 * k + 1] = (double)v.y;
@@ -1360,18 +1433,30 @@ static uint32_t exchange_elem_bytes(int prec, int xm) {
 }
 
 // ----------------------------------------------------------------------------
-// staging of descriptors: a pool of pinned host buffers guarded by events.
-// An upload takes a buffer whose last copy has completed, so a stream with a
-// long queue never holds up uploads on other streams; the pool grows to
-// kStageMax buffers before a caller waits.
+// staging of descriptors: a pool of pinned host buffers.  An upload takes a
+// buffer whose last copy has completed, so a stream with a long queue never
+// holds up uploads on other streams; the pool grows to kStageMax buffers before
+// a caller waits.
+//
+// Up to kStageKernelBytes a kernel of one workgroup makes the copy and, once it
+// has read the buffer, stores the upload's number into it.  An event recorded
+// after the copy instead costs the stream 4.5 us before its next kernel starts
+// (two launches and a wait: 12.9 us, with an event between them 17.4 us).  One
+// workgroup has 64 KiB in flight at once, the latency of the host link; longer
+// uploads go through the copy engine and an event.
 // ----------------------------------------------------------------------------
 namespace {
 struct StageSlot {
-    void *host = nullptr;
-    size_t cap = 0;
+    void *host = nullptr;  // kStageHeader bytes with the number of the last upload read, then the data
+    size_t cap = 0;        // of data
+    uint32_t ticket = 0;   // number of the slot's last upload
+    bool by_event = false; // that upload is guarded by ev, not by its number
     hipEvent_t ev = nullptr;
 };
 constexpr unsigned kStageMax = 64;
+constexpr size_t kStageHeader = 256;
+constexpr size_t kStageKernelBytes = 64 * 1024;
+constexpr unsigned kStageThreads = 1024;
 std::mutex g_stage_mu;
 StageSlot g_stage[kStageMax];
 unsigned g_stage_used = 0;
@@ -1384,23 +1469,60 @@ constexpr int kMaxDevices = 64;
 double *g_scratch_dev[kMaxDevices] = {};
 }  // namespace
 
+__global__ void __launch_bounds__(kStageThreads)
+stage_copy(const uint4 *__restrict__ src, uint4 *__restrict__ dst, uint32_t n16, uint32_t *read, uint32_t ticket) {
+    constexpr uint32_t U = kStageKernelBytes / 16 / kStageThreads;
+    uint4 v[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        const uint32_t i = threadIdx.x + u * kStageThreads;
+        if (i < n16) v[u] = src[i];
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; u++) {
+        const uint32_t i = threadIdx.x + u * kStageThreads;
+        if (i < n16) dst[i] = v[u];
+    }
+    __syncthreads();  // every thread has what it read: its stores were issued
+    if (threadIdx.x == 0) __hip_atomic_store(read, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// 1: the slot's last upload has been read, 0: not yet, -1: error (set)
+static int stage_free(const StageSlot &c) {
+    if (!c.host) return 1;
+    if (!c.by_event) return __atomic_load_n((const uint32_t *)c.host, __ATOMIC_ACQUIRE) == c.ticket;
+    const hipError_t e = hipEventQuery(c.ev);
+    if (e == hipSuccess) return 1;
+    if (e == hipErrorNotReady) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    fail(DQ_ERR_HIP, "hipEventQuery failed: %s", hipGetErrorString(e));
+    return -1;
+}
+
 static int stage_upload(void *d_dst, const std::vector<unsigned char> &src, void *stream) {
     std::lock_guard<std::mutex> lk(g_stage_mu);
     StageSlot *slot = nullptr;
     for (unsigned k = 0; k < g_stage_used && !slot; k++) {
         StageSlot &c = g_stage[(g_stage_next + k) % g_stage_used];
-        const hipError_t e = hipEventQuery(c.ev);
-        if (e == hipSuccess) slot = &c;
-        else if (e == hipErrorNotReady) (void)hipGetLastError();
-        else HIPC(e);
+        const int f = stage_free(c);
+        if (f < 0) return DQ_ERR_HIP;
+        if (f) slot = &c;
     }
     if (!slot && g_stage_used < kStageMax) {
-        slot = &g_stage[g_stage_used++];
+        slot = &g_stage[g_stage_used];
         HIPC(hipEventCreateWithFlags(&slot->ev, hipEventDisableTiming));
+        g_stage_used++;
     }
     if (!slot) {
         slot = &g_stage[g_stage_next % g_stage_used];
-        HIPC(hipEventSynchronize(slot->ev));
+        if (slot->by_event) {
+            HIPC(hipEventSynchronize(slot->ev));
+        } else {
+            HIPC(hipDeviceSynchronize());  // the copy's stream may be gone: wait for all of them
+            if (stage_free(*slot) != 1) return fail(DQ_ERR_HIP, "stage_upload: an earlier upload never completed");
+        }
     }
     g_stage_next = (unsigned)(slot - g_stage) + 1;
     StageSlot &s = *slot;
@@ -1408,16 +1530,92 @@ static int stage_upload(void *d_dst, const std::vector<unsigned char> &src, void
         if (s.host) HIPC(hipHostFree(s.host));
         s.host = nullptr;
         s.cap = 0;
-        size_t cap = 64 * 1024;
+        size_t cap = kStageKernelBytes;
         while (cap < src.size()) cap *= 2;
-        HIPC(hipHostMalloc(&s.host, cap, hipHostMallocDefault));
+        HIPC(hipHostMalloc(&s.host, kStageHeader + cap, hipHostMallocPortable));
         s.cap = cap;
+        s.ticket = 0;
+        s.by_event = false;
+        memset(s.host, 0, kStageHeader);
     }
-    memcpy(s.host, src.data(), src.size());
-    HIPC(hipMemcpyAsync(d_dst, s.host, src.size(), hipMemcpyHostToDevice, (hipStream_t)stream));
+    unsigned char *data = (unsigned char *)s.host + kStageHeader;
+    memcpy(data, src.data(), src.size());
+    if (src.size() <= kStageKernelBytes && src.size() % 16 == 0 && (uintptr_t)d_dst % 16 == 0) {
+        s.ticket++;
+        s.by_event = false;
+        hipLaunchKernelGGL(stage_copy, dim3(1), dim3(kStageThreads), 0, (hipStream_t)stream, (const uint4 *)data, (uint4 *)d_dst,
+                           (uint32_t)(src.size() / 16), (uint32_t *)s.host, s.ticket);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            s.ticket--;  // nothing was enqueued: the slot is free
+            return fail(DQ_ERR_HIP, "stage_copy: %s", hipGetErrorString(e));
+        }
+        return DQ_OK;
+    }
+    HIPC(hipMemcpyAsync(d_dst, data, src.size(), hipMemcpyHostToDevice, (hipStream_t)stream));
+    s.by_event = true;
     HIPC(hipEventRecord(s.ev, (hipStream_t)stream));
     return DQ_OK;
 }
+
+// ----------------------------------------------------------------------------
+// results of synchronous read-outs: pinned host slots that kernels write to
+// directly, one per call in progress.  A copy of 200 bytes to a caller's pageable
+// memory took 12.6 us on top of the kernel before it (24 us for 64 KiB); a kernel
+// that stores its results to pinned memory takes no longer than one that stores
+// them to the device.  At most kResultMax slots are ever allocated; a call that
+// finds none free, or needs a larger one, copies from the device as before.
+// ----------------------------------------------------------------------------
+namespace {
+constexpr int kResultMax = 16;
+constexpr size_t kResultBytes = 128 * 1024;
+std::mutex g_result_mu;
+void *g_result[kResultMax] = {};
+bool g_result_taken[kResultMax] = {};
+}  // namespace
+
+extern "C" void *dq_result_acquire(size_t bytes) {
+    if (bytes > kResultBytes) return nullptr;
+    std::lock_guard<std::mutex> lk(g_result_mu);
+    for (int i = 0; i < kResultMax; i++) {
+        if (g_result_taken[i]) continue;
+        if (!g_result[i] && hipHostMalloc(&g_result[i], kResultBytes, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            g_result[i] = nullptr;
+            return nullptr;
+        }
+        g_result_taken[i] = true;
+        return g_result[i];
+    }
+    return nullptr;
+}
+
+extern "C" void dq_result_release(void *slot) {
+    if (!slot) return;
+    std::lock_guard<std::mutex> lk(g_result_mu);
+    for (int i = 0; i < kResultMax; i++)
+        if (g_result[i] == slot) g_result_taken[i] = false;
+}
+
+namespace {
+// Where a read-out of `bytes` writes: a result slot, or `fallback` on the device.
+struct ResultSlot {
+    void *host;
+    void *dst;
+    ResultSlot(size_t bytes, void *fallback) : host(dq_result_acquire(bytes)), dst(host ? host : fallback) {}
+    ~ResultSlot() { dq_result_release(host); }
+    ResultSlot(const ResultSlot &) = delete;
+    ResultSlot &operator=(const ResultSlot &) = delete;
+    // Waits for the kernels enqueued on `stream` and hands their results over.
+    int collect(void *out, size_t bytes, void *stream) {
+        hipStream_t s = (hipStream_t)stream;
+        if (!host) HIPC(hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToHost, s));
+        HIPC(hipStreamSynchronize(s));
+        if (host) memcpy(out, host, bytes);
+        return DQ_OK;
+    }
+};
+}  // namespace
 
 // ----------------------------------------------------------------------------
 // C ABI: plumbing
@@ -2321,22 +2519,25 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
     }
     if (prog.size() + 256 > prog_bound(n_phases, n_ops)) return fail(DQ_ERR_ARG, "dq_apply_blocks: device program overflow");
 
-    // pack and upload
-    std::vector<unsigned char> buf(need, 0);
+    // pack and upload what the kernels read: the sweep kernels run the device
+    // programs, only small_kernel reads op descriptors
+    bool small = false;
+    for (uint32_t i = 0; i < n_blocks; i++) small |= blocks[i].reg_bits == 0;
+    const uint32_t up_ops = small ? n_ops : 0;
     size_t off_b = 0, off_p = align_up(n_blocks * sizeof(dq_block), 256);
     size_t off_o = off_p + align_up(n_phases * sizeof(dq_phase), 256);
-    size_t off_j = off_o + align_up(n_ops * sizeof(dq_op), 256);
+    size_t off_j = off_o + align_up(up_ops * sizeof(dq_op), 256);
     size_t off_pa = off_j + align_up(n_jobs * sizeof(dq_job), 256);
     size_t off_ba = off_pa + align_up((size_t)n_phases * DQ_PAUX * sizeof(uint32_t), 256);
     size_t off_pg = off_ba + align_up((size_t)n_blocks * DQ_BAUX * sizeof(uint32_t), 256);
+    std::vector<unsigned char> buf(align_up(off_pg + prog.size() + 256, 16), 0);  // + the interpreter's read-ahead
     memcpy(buf.data() + off_b, blocks, n_blocks * sizeof(dq_block));
     memcpy(buf.data() + off_p, phases, n_phases * sizeof(dq_phase));
-    if (n_ops) memcpy(buf.data() + off_o, ops, n_ops * sizeof(dq_op));
+    if (up_ops) memcpy(buf.data() + off_o, ops, up_ops * sizeof(dq_op));
     memcpy(buf.data() + off_j, jobs, n_jobs * sizeof(dq_job));
     if (n_phases) memcpy(buf.data() + off_pa, paux.data(), paux.size() * sizeof(uint32_t));
     memcpy(buf.data() + off_ba, baux.data(), baux.size() * sizeof(uint32_t));
     if (!prog.empty()) memcpy(buf.data() + off_pg, prog.data(), prog.size());
-    buf.resize(off_pg + prog.size() + 256, 0);  // upload only what is used (+ padding)
     int rc = stage_upload(d_ws, buf, stream);
     if (rc) return rc;
     unsigned char *d = (unsigned char *)d_ws;
@@ -2433,6 +2634,16 @@ static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, 
             pb.img[f++] = b;
         }
     }
+    // One launch where a workgroup's 8 loads per thread cover the state: the second
+    // launch takes longer (3.5 us) than what more workgroups would save.
+    if (nf <= PROB_ONE_BITS) {
+        if (prec == DQ_F64)
+            hipLaunchKernelGGL(prob_one<double>, dim3(1), dim3(1024), 0, stream, (const V2<double>::type *)state, pb, nf, n, po, d_out);
+        else
+            hipLaunchKernelGGL(prob_one<float>, dim3(1), dim3(1024), 0, stream, (const V2<float>::type *)state, pb, nf, n, po, d_out);
+        HIPC(hipGetLastError());
+        return DQ_OK;
+    }
     double *part = (double *)d_ws;
 #define DQ_PROB1(T_, JB_)                                                                          \
     hipLaunchKernelGGL((prob_stage1<T_, JB_>), dim3(p.groups), dim3(256), 0, stream, (const V2<T_>::type *)state, pb, nf, \
@@ -2469,11 +2680,10 @@ extern "C" int dq_prob_zero_all_fixed(const void *state, int n, int prec, uint64
     if (ws_bytes < dq_prob_ws_bytes(n)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: workspace too small");
     const size_t part_bytes = prob_part_bytes(n);
     double *d_out = (double *)((unsigned char *)d_ws + part_bytes);
-    const int rc = prob_launch(state, n, prec, fixed_mask, fixed_value, scale, d_out, d_ws, part_bytes, (hipStream_t)stream);
+    ResultSlot res((n + 1) * sizeof(double), d_out);
+    const int rc = prob_launch(state, n, prec, fixed_mask, fixed_value, scale, (double *)res.dst, d_ws, part_bytes, (hipStream_t)stream);
     if (rc) return rc;
-    HIPC(hipMemcpyAsync(out, d_out, (n + 1) * sizeof(double), hipMemcpyDeviceToHost, (hipStream_t)stream));
-    HIPC(hipStreamSynchronize((hipStream_t)stream));
-    return DQ_OK;
+    return res.collect(out, (n + 1) * sizeof(double), stream);
 }
 
 extern "C" int dq_prob_zero_all(const void *state, int n, int prec, double *out, void *d_ws, size_t ws_bytes, void *stream) {
@@ -2828,7 +3038,7 @@ extern "C" int dq_apply_dense_gates(int k, const dq_dense_block *blocks, uint32_
     if (ws_bytes < w.total) return fail(DQ_ERR_ARG, "dq_apply_dense_gates: workspace %zu < %zu bytes", ws_bytes, w.total);
     int rc = validate_dense(k, blocks, n_blocks, ops, n_ops, n_mats);
     if (rc) return rc;
-    std::vector<unsigned char> buf(w.upload, 0);
+    std::vector<unsigned char> buf(align_up(w.upload, 16), 0);  // the matrices begin at the next 256
     memcpy(buf.data(), blocks, n_blocks * sizeof(dq_dense_block));
     if (n_ops) memcpy(buf.data() + w.ops, ops, n_ops * sizeof(dq_dense_op));
     rc = dense_columns(k, blocks, n_blocks, ops, n_ops, reinterpret_cast<uint32_t *>(buf.data() + w.cols));
@@ -2878,29 +3088,26 @@ extern "C" int dq_read_amps(const void *state, int n, int prec, const int *l2p, 
     const uint64_t N = 1ull << n;
     if (start > N || count > N - start) return fail(DQ_ERR_ARG, "dq_read_amps: range out of bounds");
     if (count == 0) return DQ_OK;
-    int map[64];
+    QubitMap map;
+    memset(&map, 0, sizeof map);
     for (int q = 0; q < n; q++) {
-        map[q] = l2p ? l2p[q] : q;
-        if (map[q] < 0 || map[q] >= n) return fail(DQ_ERR_ARG, "dq_read_amps: bad qubit map");
+        const int p = l2p ? l2p[q] : q;
+        if (p < 0 || p >= n) return fail(DQ_ERR_ARG, "dq_read_amps: bad qubit map");
+        map.l2p[q] = (uint8_t)p;
     }
-    const size_t need = align_up(64 * sizeof(int), 256) + count * 2 * sizeof(double);
+    const size_t bytes = count * 2 * sizeof(double);
+    const size_t need = align_up(64 * sizeof(int), 256) + bytes;
     if (!d_ws || ws_bytes < need) return fail(DQ_ERR_ARG, "dq_read_amps: workspace %zu < %zu bytes", ws_bytes, need);
-    int *d_map = (int *)d_ws;
-    double *d_out = (double *)((unsigned char *)d_ws + align_up(64 * sizeof(int), 256));
-    std::vector<unsigned char> m((unsigned char *)map, (unsigned char *)map + 64 * sizeof(int));
-    int rc = stage_upload(d_map, m, stream);
-    if (rc) return rc;
+    ResultSlot res(bytes, (unsigned char *)d_ws + align_up(64 * sizeof(int), 256));
     const unsigned blocks = (unsigned)((count + 255) / 256);
     if (prec == DQ_F64)
         hipLaunchKernelGGL(read_kernel<double>, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
-                           (const V2<double>::type *)state, n, d_map, start, count, d_out);
+                           (const V2<double>::type *)state, n, map, start, count, (double *)res.dst);
     else
         hipLaunchKernelGGL(read_kernel<float>, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
-                           (const V2<float>::type *)state, n, d_map, start, count, d_out);
+                           (const V2<float>::type *)state, n, map, start, count, (double *)res.dst);
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(out, d_out, count * 2 * sizeof(double), hipMemcpyDeviceToHost, (hipStream_t)stream));
-    HIPC(hipStreamSynchronize((hipStream_t)stream));
-    return DQ_OK;
+    return res.collect(out, bytes, stream);
 }
 
 extern "C" int dq_write_amps(void *state, int n, int prec, uint64_t start, uint64_t count, const double *re,

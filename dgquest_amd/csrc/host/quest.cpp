@@ -363,7 +363,7 @@ void flush(QuregState *s) {
 // they keep and scale what they multiply the kept probabilities by.
 static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value, double &scale) {
     fixed = value = 0;
-    scale = 1.0;
+    long double product = 1.0L;  // one rounding, not one per measured qubit
     if (s->recorder || s->paged || s->init_kind != DQ_INIT_LOAD || s->pending.empty()) return false;
     for (const Gate &g : s->pending) {
         if (g.type != OP_COLLAPSE || g.cmask || popc64(g.tmask) != 1) return false;
@@ -371,8 +371,9 @@ static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value
         if ((fixed & g.tmask) && (value & g.tmask) != v) return false;
         fixed |= g.tmask;
         value |= v;
-        scale *= g.op[1] * g.op[1];
+        product *= (long double)g.op[1] * g.op[1];
     }
+    scale = (double)product;
     return true;
 }
 
@@ -883,10 +884,13 @@ static void compare_regs(QuregState *a, QuregState *b, double out[5]) {
     ENG(dq_stream_sync(b->stream));
     const size_t cw = (dq_compare_ws_bytes(a->n) + 255) / 256 * 256;
     ensure_ws(a, cw + 256);
-    double *d_out = (double *)((unsigned char *)a->d_ws + cw);
+    double *host = (double *)dq_result_acquire(5 * sizeof(double));
+    double *d_out = host ? host : (double *)((unsigned char *)a->d_ws + cw);
     ENG(dq_compare_states(a->d_state, a->prec, b->d_state, b->prec, a->n, d_out, a->d_ws, cw, a->stream));
-    ENG(dq_memcpy_async(out, d_out, 5 * sizeof(double), DQ_D2H, a->stream));
+    if (!host) ENG(dq_memcpy_async(out, d_out, 5 * sizeof(double), DQ_D2H, a->stream));
     ENG(dq_stream_sync(a->stream));
+    if (host) memcpy(out, host, 5 * sizeof(double));
+    dq_result_release(host);
 }
 
 Complex calcInnerProduct(Qureg bra, Qureg ket) {
@@ -1232,14 +1236,17 @@ int dgq_sample(Qureg q, int shots, const double *u, unsigned long long *out) {
     materialize_mapping(s);  // samples walk the CDF in logical index order
     const size_t res = (((size_t)shots * sizeof(uint64_t)) + 255) / 256 * 256;
     ensure_ws(s, res + dq_readout_ws_bytes(s->n, 1, (uint32_t)shots));
-    uint64_t *d_out = (uint64_t *)s->d_ws;
+    uint64_t *host = (uint64_t *)dq_result_acquire((size_t)shots * sizeof(uint64_t));
+    uint64_t *d_out = host ? host : (uint64_t *)s->d_ws;
     const void *st = s->d_state;
     ENG(dq_readout_many(s->prec, s->n, &st, 1, u, (uint32_t)shots, nullptr, d_out, (unsigned char *)s->d_ws + res,
                         s->ws_cap - res, s->stream));
-    std::vector<uint64_t> idx((size_t)shots);
-    ENG(dq_memcpy_async(idx.data(), d_out, (size_t)shots * sizeof(uint64_t), DQ_D2H, s->stream));
+    std::vector<uint64_t> idx(host ? 0 : (size_t)shots);
+    if (!host) ENG(dq_memcpy_async(idx.data(), d_out, (size_t)shots * sizeof(uint64_t), DQ_D2H, s->stream));
     ENG(dq_stream_sync(s->stream));
-    for (int i = 0; i < shots; i++) out[i] = idx[i];
+    const uint64_t *from = host ? host : idx.data();
+    for (int i = 0; i < shots; i++) out[i] = from[i];
+    dq_result_release(host);
     return 0;
 }
 
