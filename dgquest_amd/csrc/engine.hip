@@ -22,6 +22,7 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <string>
 #include <type_traits>
 #include <vector>
 
@@ -1972,22 +1973,76 @@ static bool block_runs(const dq_block &b, uint32_t *out) {
 // table fused with the shears after it, a WG op in front of each op with a
 // workgroup condition, END last.
 namespace {
+// Codes of the device ops for one R, looked up once.  Searching the table by
+// name for every op, and a heap block for every table, took most of a flush's
+// host time: the programs of a 30-qubit circuit (2426 ops in 106 phases)
+// 512 -> 104 us, of a 17-qubit one (507 ops in 94 phases) 100 -> 30 us.
+struct OpCodes {
+    const DevOpCode *tab;
+    int n;
+    int END, WG, SHEARS, TABLE_FULL, TABLE_GEN, TSH_FULL, TSH_GEN, FAN;
+    int TABLE_HALF[DQ_MAX_REG_BITS], TSH_HALF[DQ_MAX_REG_BITS], MAT[DQ_MAX_REG_BITS], SWAP[DQ_MAX_REG_BITS], RMAT[DQ_MAX_REG_BITS];
+    int FM_ALL, FM_B[DQ_MAX_REG_BITS][2];
+    struct Cond {  // variants of a conditioned op: every register, one bit, two bits (r1 < r2), a mask
+        int all, gen, b[DQ_MAX_REG_BITS][2], bb[DQ_MAX_REG_BITS][DQ_MAX_REG_BITS][2][2];
+    } NEG, PHASE;
+    int find(const char *name, int p0 = -1, int p1 = -1, int p2 = -1, int p3 = -1) const {
+        for (int c = 0; c < n; c++)
+            if (!strcmp(tab[c].name, name) && tab[c].p[0] == p0 && tab[c].p[1] == p1 && tab[c].p[2] == p2 && tab[c].p[3] == p3)
+                return c;
+        return -1;
+    }
+    void find_cond(Cond &d, const std::string &name, int R) const {
+        d.all = find((name + "_ALL").c_str());
+        d.gen = find((name + "_GEN").c_str());
+        for (int r = 0; r < R; r++)
+            for (int v = 0; v < 2; v++) {
+                d.b[r][v] = find((name + "_B").c_str(), r, v);
+                for (int r2 = r + 1; r2 < R; r2++)
+                    for (int v2 = 0; v2 < 2; v2++) d.bb[r][r2][v][v2] = find((name + "_BB").c_str(), r, r2, v, v2);
+            }
+    }
+    explicit OpCodes(int R) {
+        tab = dev_ops(R, n);
+        END = find("END");
+        WG = find("WG");
+        SHEARS = find("SHEARS");
+        TABLE_FULL = find("TABLE_FULL");
+        TABLE_GEN = find("TABLE_GEN");
+        TSH_FULL = find("TSH_FULL");
+        TSH_GEN = find("TSH_GEN");
+        FAN = find("FAN");
+        FM_ALL = find("FM_ALL");
+        for (int r = 0; r < R; r++) {
+            TABLE_HALF[r] = find("TABLE_HALF", r);
+            TSH_HALF[r] = find("TSH_HALF", r);
+            MAT[r] = find("MAT", r);
+            SWAP[r] = find("SWAP", r);
+            RMAT[r] = find("RMAT", r);
+            for (int v = 0; v < 2; v++) FM_B[r][v] = find("FM_B", r, v);
+        }
+        find_cond(NEG, "NEG", R);
+        find_cond(PHASE, "PHASE", R);
+    }
+    static const OpCodes &of(int R) {
+        static const OpCodes all[DQ_MAX_REG_BITS] = {OpCodes(1), OpCodes(2), OpCodes(3), OpCodes(4), OpCodes(5)};
+        return all[R - 1];
+    }
+};
+static_assert(DQ_MAX_REG_BITS == 5, "OpCodes::of lists every R");
+
 struct ProgBuilder {
     int prec, R, NR, ncodes;
     size_t ts;
+    const OpCodes &cd;
     const DevOpCode *tab;
     std::vector<unsigned char> &out;
+    bool gather;       // phases of one register condition become one FAN op
     bool bad = false;  // an op with no code (never sent to the device)
-    ProgBuilder(int prec_, int R_, std::vector<unsigned char> &o) : prec(prec_), R(R_), NR(1 << R_), out(o) {
-        ts = prec == DQ_F64 ? 8 : 4;
-        tab = dev_ops(R, ncodes);
-    }
-    int code(const char *name, int p0 = -1, int p1 = -1, int p2 = -1, int p3 = -1) const {
-        for (int c = 0; c < ncodes; c++)
-            if (!strcmp(tab[c].name, name) && tab[c].p[0] == p0 && tab[c].p[1] == p1 && tab[c].p[2] == p2 &&
-                tab[c].p[3] == p3)
-                return c;
-        return -1;
+    ProgBuilder(int prec_, int R_, std::vector<unsigned char> &o, bool gather_ = true)
+        : prec(prec_), R(R_), NR(1 << R_), ts(prec_ == DQ_F64 ? 8 : 4), cd(OpCodes::of(R_)), out(o), gather(gather_) {
+        tab = cd.tab;
+        ncodes = cd.n;
     }
     size_t size(int c) const { return (size_t)(prec == DQ_F64 ? tab[c].size64 : tab[c].size32); }
     // one op into `v`: header then coefficient bytes, zero padded to its size
@@ -2006,7 +2061,7 @@ struct ProgBuilder {
     void emit(const std::vector<unsigned char> &op, uint64_t c_wg, uint64_t v_wg) {
         if (c_wg) {
             const uint64_t cond[2] = {c_wg, v_wg};
-            encode(out, code("WG"), 0, 0, (uint32_t)op.size(), cond, 16);
+            encode(out, cd.WG, 0, 0, (uint32_t)op.size(), cond, 16);
         }
         out.insert(out.end(), op.begin(), op.end());
     }
@@ -2020,18 +2075,18 @@ struct ProgBuilder {
         return m;
     }
     // NEG / PHASE variant for the register condition (c, v)
-    int cond_variant(const char *all, const char *b, const char *bb, const char *gen, uint32_t c, uint32_t v) const {
+    static int cond_variant(const OpCodes::Cond &d, uint32_t c, uint32_t v) {
         const int pc = __builtin_popcount(c);
-        if (pc == 0) return code(all);
+        if (pc == 0) return d.all;
         if (pc == 1) {
             const int r = __builtin_ctz(c);
-            return code(b, r, (int)((v >> r) & 1));
+            return d.b[r][(v >> r) & 1];
         }
         if (pc == 2) {
             const int r1 = __builtin_ctz(c), r2 = 31 - __builtin_clz(c);
-            return code(bb, r1, r2, (int)((v >> r1) & 1), (int)((v >> r2) & 1));
+            return d.bb[r1][r2][(v >> r1) & 1][(v >> r2) & 1];
         }
-        return code(gen);
+        return d.gen;
     }
     // Value i of op o's coefficient array, in double.
     double val(const dq_op &o, int i) const {
@@ -2044,66 +2099,66 @@ struct ProgBuilder {
         memcpy(&v, reinterpret_cast<const unsigned char *>(o.m) + 4 * i, 4);
         return (double)v;
     }
-    void put(std::vector<unsigned char> &v, double x) const {
-        const size_t at = v.size();
-        v.resize(at + ts);
-        if (prec == DQ_F64) memcpy(v.data() + at, &x, 8);
-        else {
-            const float f = (float)x;
-            memcpy(v.data() + at, &f, 4);
+    // A diagonal over the register index, in double.
+    struct Diag {
+        double re[1 << DQ_MAX_REG_BITS], im[1 << DQ_MAX_REG_BITS];
+        Diag() { clear(); }
+        void clear() {
+            std::fill(re, re + (1 << DQ_MAX_REG_BITS), 1.0);
+            std::fill(im, im + (1 << DQ_MAX_REG_BITS), 0.0);
         }
-    }
+        void mul(int j, double fr, double fi) {
+            const double r = re[j] * fr - im[j] * fi, i = re[j] * fi + im[j] * fr;
+            re[j] = r;
+            im[j] = i;
+        }
+        void mul_cond(int NR, uint32_t c, uint32_t v, double fr, double fi) {
+            for (int j = 0; j < NR; j++)
+                if (((uint32_t)j & c) == v) mul(j, fr, fi);
+        }
+    };
     // A table op (or, with shear slots, a table+shears op) for the diagonal
-    // (tr, ti) over the register index: HALF when every factor that is not 1
+    // d over the register index: HALF when every factor that is not 1
     // has one register bit set, FULL when at least 3/4 of them are not 1, GEN
     // (a mask of the factors to apply) otherwise.  False if every factor is 1.
-    bool encode_table(std::vector<unsigned char> &op, const std::vector<double> &tr, const std::vector<double> &ti,
-                      const std::vector<unsigned char> *slots, uint32_t shear_mask) {
-        std::vector<unsigned char> table;
-        for (int e = 0; e < NR; e++) {
-            put(table, tr[e]);
-            put(table, ti[e]);
-        }
+    bool encode_table(std::vector<unsigned char> &op, const Diag &d, const unsigned char *slots, uint32_t shear_mask) {
+        unsigned char body[(2 << DQ_MAX_REG_BITS) * 8 + 2 * DQ_MAX_REG_BITS * 8];
+        size_t len = 0;
         uint32_t ne1 = 0;  // factors that are not exactly 1 in the state precision
         for (int e = 0; e < NR; e++) {
-            double r, i;
-            if (prec == DQ_F64) {
-                memcpy(&r, table.data() + e * 16, 8);
-                memcpy(&i, table.data() + e * 16 + 8, 8);
-            } else {
-                float fr, fi;
-                memcpy(&fr, table.data() + e * 8, 4);
-                memcpy(&fi, table.data() + e * 8 + 4, 4);
-                r = fr;
-                i = fi;
-            }
-            if (!(r == 1.0 && i == 0.0)) ne1 |= 1u << e;
+            const bool one = prec == DQ_F64 ? d.re[e] == 1.0 && d.im[e] == 0.0 : (float)d.re[e] == 1.0f && (float)d.im[e] == 0.0f;
+            if (!one) ne1 |= 1u << e;
         }
         if (!ne1) return false;
         int half = -1;
         for (int r = 0; r < R && half < 0; r++)
             if ((ne1 & ~jmask(1u << r, 1u << r, -1)) == 0) half = r;
-        std::vector<unsigned char> body;
         int c;
         uint32_t gen = 0;
         if (half >= 0) {
-            for (int e = 0; e < NR; e++)
-                if ((e >> half) & 1)
-                    body.insert(body.end(), table.begin() + (size_t)e * 2 * ts, table.begin() + (size_t)(e + 1) * 2 * ts);
-            c = slots ? code("TSH_HALF", half) : code("TABLE_HALF", half);
+            c = slots ? cd.TSH_HALF[half] : cd.TABLE_HALF[half];
         } else if (4 * __builtin_popcount(ne1) >= 3 * NR) {
-            body = table;
-            c = slots ? code("TSH_FULL") : code("TABLE_FULL");
+            c = slots ? cd.TSH_FULL : cd.TABLE_FULL;
         } else {
-            body = table;
             gen = ne1;
-            c = slots ? code("TSH_GEN") : code("TABLE_GEN");
+            c = slots ? cd.TSH_GEN : cd.TABLE_GEN;
+        }
+        for (int e = 0; e < NR; e++) {
+            if (half >= 0 && !((e >> half) & 1)) continue;
+            if (prec == DQ_F64) {
+                const double f[2] = {d.re[e], d.im[e]};
+                memcpy(body + len, f, 16);
+            } else {
+                const float f[2] = {(float)d.re[e], (float)d.im[e]};
+                memcpy(body + len, f, 8);
+            }
+            len += 2 * ts;
         }
         if (slots) {
-            body.insert(body.end(), slots->begin(), slots->end());
-            encode(op, c, shear_mask, gen, 0, body.data(), body.size());
+            memcpy(body + len, slots, 2 * (size_t)R * ts);
+            encode(op, c, shear_mask, gen, 0, body, len + 2 * (size_t)R * ts);
         } else {
-            encode(op, c, gen, 0, 0, body.data(), body.size());
+            encode(op, c, gen, 0, 0, body, len);
         }
         return true;
     }
@@ -2124,59 +2179,110 @@ struct ProgBuilder {
         uint32_t c_reg, v_reg;
         double fr, fi;
     };
+    // NEG / PHASE ops of a diagonal run with a lane or workgroup condition, kept
+    // by register condition (0: none, 1 + 2 r + v: bit r = v) until the run ends.
+    std::vector<const dq_op *> held[1 + 2 * DQ_MAX_REG_BITS];
+    static bool can_hold(const dq_op &o) {
+        return (o.c_thr || o.c_wg) && __builtin_popcountll(o.c_wg) <= 1 && __builtin_popcount(o.c_reg) <= 1;
+    }
+    void emit_single(const dq_op &o) {
+        std::vector<unsigned char> op;
+        if (o.kind == DQ_OP_NEG)
+            encode(op, cond_variant(cd.NEG, o.c_reg, o.v_reg), jmask(o.c_reg, o.v_reg, -1), o.c_thr, o.v_thr, nullptr, 0);
+        else
+            encode(op, cond_variant(cd.PHASE, o.c_reg, o.v_reg), jmask(o.c_reg, o.v_reg, -1), o.c_thr, o.v_thr, o.m, 2 * ts);
+        emit(op, o.c_wg, o.v_wg);
+    }
+    // The held ops of one register condition: a FAN op where that takes fewer
+    // vector instructions (a complex product of 4 on every selected register, and
+    // 6 a term, against 4 or, for a sign, 2 on every selected register and 2 a
+    // term; half of those with a workgroup condition are skipped).  A 27-qubit
+    // Fourier transform in FP32 ran 254 phases of 16 or 32 registers each.
+    void emit_held(uint32_t &n_out) {
+        for (int g = 0; g < 1 + 2 * R; g++) {
+            auto &h = held[g];
+            if (h.empty()) continue;
+            const int regs = g ? NR / 2 : NR;
+            double one = 0.0, fan = 4.0 * regs;
+            for (const dq_op *o : h) {
+                const double c = (o->kind == DQ_OP_NEG ? 2.0 : 4.0) * regs + 2.0;
+                one += o->c_wg ? 0.5 * c : c;
+                fan += o->c_wg ? 3.0 : 6.0;
+            }
+            if (h.size() < 2 || fan >= one) {
+                for (const dq_op *o : h) emit_single(*o);
+                n_out += (uint32_t)h.size();
+                h.clear();
+                continue;
+            }
+            const size_t at = out.size(), tb = ts == 8 ? 32 : 16;
+            out.resize(at + 16 + h.size() * tb, 0);
+            unsigned char *w = out.data() + at;
+            const uint32_t apply = (uint32_t)(g ? cd.FM_B[(g - 1) / 2][(g - 1) & 1] : cd.FM_ALL);
+            const uint32_t hdr[4] = {(uint32_t)cd.FAN, apply, 0, (uint32_t)(16 + h.size() * tb)};
+            memcpy(w, hdr, 16);
+            w += 16;
+            for (size_t i = 0; i < h.size(); i++, w += tb) {
+                const dq_op &o = *h[i];
+                uint32_t c[2] = {o.c_thr | (o.v_thr << 16), 0};
+                if (o.c_wg) c[1] = (uint32_t)__builtin_ctzll(o.c_wg) | 0x100u | (o.v_wg ? 0x200u : 0u);
+                if (i + 1 == h.size()) c[1] |= 0x400u;
+                memcpy(w, c, 8);
+                const double f[2] = {o.kind == DQ_OP_NEG ? -1.0 : val(o, 0), o.kind == DQ_OP_NEG ? 0.0 : val(o, 1)};
+                if (ts == 8) {
+                    memcpy(w + 16, f, 16);
+                } else {
+                    const float f4[2] = {(float)f[0], (float)f[1]};
+                    memcpy(w + 8, f4, 8);
+                }
+            }
+            h.clear();
+            n_out++;
+        }
+    }
     void build(const dq_op *ops, uint32_t count, uint32_t &n_out) {
         n_out = 0;
         std::vector<unsigned char> op;
-        std::vector<double> tr(NR, 1.0), ti(NR, 0.0);
-        bool pending = false;  // tr/ti hold a table not yet emitted
+        const size_t nslot = 2 * (size_t)R * ts;  // bytes of the shear slots
+        Diag tab_;
+        bool pending = false;  // tab_ holds a table not yet emitted
         std::vector<WgDiag> wgd;  // workgroup-conditioned factors of the pending table
         uint64_t wg_bits = 0;     // their workgroup bits
         auto is_diag = [](const dq_op &o) {
             return o.kind == DQ_OP_NEG || o.kind == DQ_OP_PHASE || o.kind == DQ_OP_DIAGR;
         };
-        auto mul_into = [&](std::vector<double> &xr, std::vector<double> &xi, uint32_t c, uint32_t v, double fr,
-                            double fi) {
-            for (int j = 0; j < NR; j++)
-                if (((uint32_t)j & c) == v) {
-                    const double r = xr[j] * fr - xi[j] * fi, i = xr[j] * fi + xi[j] * fr;
-                    xr[j] = r;
-                    xi[j] = i;
-                }
-        };
-        auto mul = [&](uint32_t c, uint32_t v, double fr, double fi) { mul_into(tr, ti, c, v, fr, fi); };
-        auto flush = [&](const std::vector<unsigned char> *slots, uint32_t shear_mask) {
+        auto flush = [&](const unsigned char *slots, uint32_t shear_mask) {
             if (pending && wg_bits) {
                 const int nb = __builtin_popcountll(wg_bits);
                 for (uint32_t a = 0; a < (1u << nb); a++) {
                     uint64_t val = 0, m = wg_bits;  // assignment a deposited on the bits
                     for (int i = 0; m; i++, m &= m - 1)
                         if ((a >> i) & 1) val |= m & (~m + 1);
-                    std::vector<double> vr = tr, vi = ti;
+                    Diag v = tab_;
                     for (const WgDiag &d : wgd)
-                        if ((val & d.c_wg) == d.v_wg) mul_into(vr, vi, d.c_reg, d.v_reg, d.fr, d.fi);
+                        if ((val & d.c_wg) == d.v_wg) v.mul_cond(NR, d.c_reg, d.v_reg, d.fr, d.fi);
                     op.clear();
-                    if (!encode_table(op, vr, vi, slots, shear_mask)) {
+                    if (!encode_table(op, v, slots, shear_mask)) {
                         if (!slots) continue;  // nothing to do for these workgroups
                         op.clear();
-                        encode(op, code("SHEARS"), shear_mask, 0, 0, slots->data(), slots->size());
+                        encode(op, cd.SHEARS, shear_mask, 0, 0, slots, nslot);
                     }
                     emit(op, wg_bits, val);
                     n_out++;
                 }
             } else {
                 op.clear();
-                const bool any = pending && encode_table(op, tr, ti, slots, shear_mask);
+                const bool any = pending && encode_table(op, tab_, slots, shear_mask);
                 if (any || slots) {
                     if (!any) {
                         op.clear();
-                        encode(op, code("SHEARS"), shear_mask, 0, 0, slots->data(), slots->size());
+                        encode(op, cd.SHEARS, shear_mask, 0, 0, slots, nslot);
                     }
                     emit(op, 0, 0);
                     n_out++;
                 }
             }
-            std::fill(tr.begin(), tr.end(), 1.0);
-            std::fill(ti.begin(), ti.end(), 0.0);
+            if (pending) tab_.clear();
             pending = false;
             wgd.clear();
             wg_bits = 0;
@@ -2190,6 +2296,11 @@ struct ProgBuilder {
             pending = true;
             return true;
         };
+        auto hold = [&](const dq_op &o) {
+            if (!gather || !can_hold(o)) return false;
+            held[o.c_reg ? 1 + 2 * __builtin_ctz(o.c_reg) + (o.v_reg ? 1 : 0) : 0].push_back(&o);
+            return true;
+        };
         bool fold_run = false;  // the current run of diagonal ops holds an unconditioned table
         bool in_run = false;
         for (uint32_t k = 0; k < count; k++) {
@@ -2197,33 +2308,39 @@ struct ProgBuilder {
             const unsigned char *m = reinterpret_cast<const unsigned char *>(o.m);
             if (is_diag(o) && !in_run) {
                 fold_run = false;
-                for (uint32_t k2 = k; k2 < count && is_diag(ops[k2]); k2 += ops[k2].kind == DQ_OP_DIAGR ? 1 + ops[k2].tbit : 1)
-                    if (ops[k2].kind == DQ_OP_DIAGR && !ops[k2].c_wg) fold_run = true;
+                double plain = 0.0;  // vector instructions of the run's unconditioned ops, each on its own
+                for (uint32_t k2 = k; k2 < count && is_diag(ops[k2]); k2 += ops[k2].kind == DQ_OP_DIAGR ? 1 + ops[k2].tbit : 1) {
+                    const dq_op &d = ops[k2];
+                    if (d.kind == DQ_OP_DIAGR) fold_run |= !d.c_wg;
+                    else if (!d.c_thr && !d.c_wg) plain += (d.kind == DQ_OP_NEG ? 2.0 : 4.0) * (NR >> __builtin_popcount(d.c_reg));
+                }
+                if (gather && plain > 4.0 * NR) fold_run = true;  // a table of their own takes less
             }
             in_run = is_diag(o);
+            if (!in_run) emit_held(n_out);
             op.clear();
             switch (o.kind) {
                 case DQ_OP_SHEAR: {
                     // merge the run of unconditioned shears on distinct bits
-                    std::vector<unsigned char> slots(2 * (size_t)R * ts, 0);
+                    unsigned char slots[2 * DQ_MAX_REG_BITS * 8] = {};
                     uint32_t mask = 0;
                     uint32_t k2 = k;
                     while (k2 < count && ops[k2].kind == DQ_OP_SHEAR && !ops[k2].c_wg && !((mask >> ops[k2].tbit) & 1)) {
                         mask |= 1u << ops[k2].tbit;
-                        memcpy(slots.data() + 2 * ops[k2].tbit * ts, ops[k2].m, 2 * ts);
+                        memcpy(slots + 2 * ops[k2].tbit * ts, ops[k2].m, 2 * ts);
                         k2++;
                     }
                     if (k2 == k) {  // a shear with a workgroup condition: on its own
                         flush(nullptr, 0);
                         op.clear();
                         mask = 1u << o.tbit;
-                        memcpy(slots.data() + 2 * o.tbit * ts, o.m, 2 * ts);
-                        encode(op, code("SHEARS"), mask, 0, 0, slots.data(), slots.size());
+                        memcpy(slots + 2 * o.tbit * ts, o.m, 2 * ts);
+                        encode(op, cd.SHEARS, mask, 0, 0, slots, nslot);
                         emit(op, o.c_wg, o.v_wg);
                         n_out++;
                         continue;
                     }
-                    flush(&slots, mask);
+                    flush(slots, mask);
                     k = k2 - 1;
                     continue;
                 }
@@ -2231,17 +2348,17 @@ struct ProgBuilder {
                     if (!o.c_wg) {
                         for (int e = 0; e < NR; e++) {
                             const dq_op &d = ops[k + 1 + e / 4];
-                            mul((uint32_t)(NR - 1), (uint32_t)e, val(d, 2 * (e % 4)), val(d, 2 * (e % 4) + 1));
+                            tab_.mul(e, val(d, 2 * (e % 4)), val(d, 2 * (e % 4) + 1));
                         }
                         pending = true;
                     } else {  // a table under a workgroup condition: its own op (it commutes with the pending one)
-                        std::vector<double> wr(NR), wi(NR);
+                        Diag w;
                         for (int e = 0; e < NR; e++) {
                             const dq_op &d = ops[k + 1 + e / 4];
-                            wr[e] = val(d, 2 * (e % 4));
-                            wi[e] = val(d, 2 * (e % 4) + 1);
+                            w.re[e] = val(d, 2 * (e % 4));
+                            w.im[e] = val(d, 2 * (e % 4) + 1);
                         }
-                        if (encode_table(op, wr, wi, nullptr, 0)) {
+                        if (encode_table(op, w, nullptr, 0)) {
                             emit(op, o.c_wg, o.v_wg);
                             n_out++;
                         }
@@ -2251,38 +2368,40 @@ struct ProgBuilder {
                 }
                 case DQ_OP_NEG:
                     if (fold_run && !o.c_thr && !o.c_wg) {
-                        mul(o.c_reg, o.v_reg, -1.0, 0.0);
+                        tab_.mul_cond(NR, o.c_reg, o.v_reg, -1.0, 0.0);
                         pending = true;
                         continue;
                     }
                     if (fold_run && o.c_wg && fold_wg(o, -1.0, 0.0)) continue;
-                    encode(op, cond_variant("NEG_ALL", "NEG_B", "NEG_BB", "NEG_GEN", o.c_reg, o.v_reg),
-                           jmask(o.c_reg, o.v_reg, -1), o.c_thr, o.v_thr, nullptr, 0);
-                    break;
+                    if (hold(o)) continue;
+                    emit_single(o);
+                    n_out++;
+                    continue;
                 case DQ_OP_PHASE:
                     if (fold_run && !o.c_thr && !o.c_wg) {
-                        mul(o.c_reg, o.v_reg, val(o, 0), val(o, 1));
+                        tab_.mul_cond(NR, o.c_reg, o.v_reg, val(o, 0), val(o, 1));
                         pending = true;
                         continue;
                     }
                     if (fold_run && o.c_wg && fold_wg(o, val(o, 0), val(o, 1))) continue;
-                    encode(op, cond_variant("PHASE_ALL", "PHASE_B", "PHASE_BB", "PHASE_GEN", o.c_reg, o.v_reg),
-                           jmask(o.c_reg, o.v_reg, -1), o.c_thr, o.v_thr, m, 2 * ts);
-                    break;
+                    if (hold(o)) continue;
+                    emit_single(o);
+                    n_out++;
+                    continue;
                 case DQ_OP_MAT:
                     flush(nullptr, 0);
                     op.clear();
-                    encode(op, code("MAT", (int)o.tbit), jmask(o.c_reg, o.v_reg, (int)o.tbit), o.c_thr, o.v_thr, m, 8 * ts);
+                    encode(op, cd.MAT[o.tbit], jmask(o.c_reg, o.v_reg, (int)o.tbit), o.c_thr, o.v_thr, m, 8 * ts);
                     break;
                 case DQ_OP_SWAP:
                     flush(nullptr, 0);
                     op.clear();
-                    encode(op, code("SWAP", (int)o.tbit), jmask(o.c_reg, o.v_reg, (int)o.tbit), o.c_thr, o.v_thr, nullptr, 0);
+                    encode(op, cd.SWAP[o.tbit], jmask(o.c_reg, o.v_reg, (int)o.tbit), o.c_thr, o.v_thr, nullptr, 0);
                     break;
                 case DQ_OP_RMAT:
                     flush(nullptr, 0);
                     op.clear();
-                    encode(op, code("RMAT", (int)o.tbit), 0, 0, 0, m, 4 * ts);
+                    encode(op, cd.RMAT[o.tbit], 0, 0, 0, m, 4 * ts);
                     break;
                 default:
                     continue;
@@ -2290,9 +2409,10 @@ struct ProgBuilder {
             emit(op, o.c_wg, o.v_wg);
             n_out++;
         }
+        emit_held(n_out);
         flush(nullptr, 0);
         op.clear();
-        encode(op, code("END"), 0, 0, 0, nullptr, 0);
+        encode(op, cd.END, 0, 0, 0, nullptr, 0);
         out.insert(out.end(), op.begin(), op.end());
     }
     // Walk a built program: every code in range, sizes chaining to END at the
@@ -2303,23 +2423,34 @@ struct ProgBuilder {
             uint32_t c;
             memcpy(&c, out.data() + at, 4);
             if (c >= (uint32_t)ncodes) return false;
-            if (!strcmp(tab[c].name, "END")) return at + size(c) == out.size();
-            at += size(c);
+            if (c == (uint32_t)cd.END) return at + size(c) == out.size();
+            if (c >= (uint32_t)cd.FM_ALL) return false;  // reached through a FAN's header only
+            uint32_t fan[4];
+            memcpy(fan, out.data() + at, 16);
+            if (c == (uint32_t)cd.FAN) {  // whole terms, the last one marked: the handler's loop ends there
+                const size_t tb = ts == 8 ? 32 : 16;
+                if (fan[1] < (uint32_t)cd.FM_ALL || fan[1] >= (uint32_t)ncodes || fan[3] <= 16 || (fan[3] - 16) % tb ||
+                    at + fan[3] > out.size())
+                    return false;
+                uint32_t last;
+                memcpy(&last, out.data() + at + fan[3] - tb + 4, 4);
+                if (!(last & 0x400u)) return false;
+                at += fan[3];
+            } else {
+                at += size(c);
+            }
         }
         return false;
     }
 };
 }  // namespace
 
-// The device program of one phase's ops, built on the host as
-// dq_apply_blocks builds it (no GPU needed): lets the program encoding be
-// checked against the op semantics on any host.
-extern "C" int dq_build_program(int prec, int reg_bits, const dq_op *ops, uint32_t n_ops, unsigned char *out,
-                                size_t cap, size_t *len) {
+static int build_program(int prec, int reg_bits, const dq_op *ops, uint32_t n_ops, unsigned char *out, size_t cap, size_t *len,
+                         bool gather) {
     if ((prec != DQ_F32 && prec != DQ_F64) || reg_bits < 1 || reg_bits > DQ_MAX_REG_BITS || !len || (n_ops && !ops))
         return fail(DQ_ERR_ARG, "dq_build_program: bad arguments");
     std::vector<unsigned char> prog;
-    ProgBuilder pb(prec, reg_bits, prog);
+    ProgBuilder pb(prec, reg_bits, prog, gather);
     uint32_t n_out = 0;
     pb.build(ops, n_ops, n_out);
     if (pb.bad || !pb.check(0)) return fail(DQ_ERR_ARG, "dq_build_program: op not expressible as a device op");
@@ -2329,6 +2460,18 @@ extern "C" int dq_build_program(int prec, int reg_bits, const dq_op *ops, uint32
         memcpy(out, prog.data(), prog.size());
     }
     return DQ_OK;
+}
+
+// The device program of one phase's ops, built on the host (no GPU needed): lets
+// the program encoding be checked against the op semantics on any host.
+extern "C" int dq_build_program(int prec, int reg_bits, const dq_op *ops, uint32_t n_ops, unsigned char *out,
+                                size_t cap, size_t *len) {
+    return build_program(prec, reg_bits, ops, n_ops, out, cap, len, false);
+}
+
+extern "C" int dq_build_program_gathered(int prec, int reg_bits, const dq_op *ops, uint32_t n_ops, unsigned char *out,
+                                         size_t cap, size_t *len) {
+    return build_program(prec, reg_bits, ops, n_ops, out, cap, len, true);
 }
 
 extern "C" int dq_init_state(void *state, int n, int prec, int kind, uint64_t index, double value, void *stream) {

@@ -36,6 +36,14 @@ size of each op code is fixed (op_size below).
       TSH_*     a TABLE_* table, then the SHEARS slots: the diagonal, then the
                 shears, in one op
       PHASE_*   re, im          MAT  u00 u01 u10 u11 (re, im)     RMAT m0..m3
+      FAN       terms (FAN_TERM): the product of the phases of the terms whose
+                condition holds, formed once per thread, multiplies the
+                registers that the op's FM_* code selects.  Header: mask = the
+                FM_* code (never an op of its own), v_thr = bytes of the op.
+                Term: u32 lane condition (mask | value << 16, 0: every lane),
+                u32 workgroup condition (0: none; bit number | 1 << 8 | value
+                << 9) | 1 << 10 on the last term, [8 bytes of padding in FP64,]
+                re, im
 Scalar registers s36..s71 are reserved by the asm (clobbered; the compiler
 keeps the SGPRs above s71 for itself, and at 8 waves per SIMD it may not use
 any above s71):
@@ -52,6 +60,7 @@ import itertools
 import sys
 
 BUF2, HDR, OFF, SCR, TAB = 36, 52, 68, 69, 70
+FAN_TERM = {4: 16, 8: 32}  # bytes of a FAN term by sizeof(T)
 EXEC = BUF2             # saved exec of a lane-conditioned op (s[36:37])
 COEF = HDR + 4          # coefficients start right after the 16-byte header
 CLOBBER = range(36, 72)
@@ -76,13 +85,15 @@ def op_codes(R):
     codes += [("RMAT", (b,)) for b in range(R)]
     codes += [("TSH_FULL", ()), ("TSH_GEN", ())]
     codes += [("TSH_HALF", (r,)) for r in range(R)]
+    codes += [("FAN", ()), ("FM_ALL", ())]
+    codes += [("FM_B", (r, v)) for r in range(R) for v in (0, 1)]
     return codes
 
 
 def op_size(name, R, ts):
-    """Bytes of an op (a multiple of 16)."""
+    """Bytes of an op (a multiple of 16); of a FAN, of its header (the op's size is in it)."""
     base = name.split("_")[0]
-    if name in ("END", "SWAP") or base == "NEG":
+    if name in ("END", "SWAP", "FAN") or base in ("NEG", "FM"):
         b = 0
     elif name == "WG":
         b = 16
@@ -447,6 +458,78 @@ class Gen:
             self.e(f"{self.mov} {xi}, %[t1]")
         self.tail("RMAT")
 
+    # --- phases of one register condition, gathered -----------------------------
+    # Controlled phases between a register bit and lane, wave or workgroup bits
+    # (a Fourier transform has one for every pair of qubits) multiplied every
+    # selected register each: 2^R / 2 complex products and a dispatch per phase.
+    # Here a term is one complex product on the thread's factor (t0, t1), under
+    # its condition, and the registers are multiplied once for all terms.
+    def fan_term(self, b, tag, done):
+        f = self.f
+        self.e(f"s_bitcmp1_b32 s{b + 1}, 8")
+        self.e(f"s_cbranch_scc0 {self.lbl(tag + 'n')}")
+        self.e(f"s_lshr_b64 vcc, %[base], s{b + 1}")   # the shift is the low 6 bits, the bit number
+        self.e(f"s_lshr_b32 vcc_hi, s{b + 1}, 9")
+        self.e("s_xor_b32 vcc_lo, vcc_lo, vcc_hi")
+        self.e("s_bitcmp1_b32 vcc_lo, 0")
+        self.e(f"s_cbranch_scc1 {self.lbl(tag + 's')}")
+        self.e(f"{self.lbl(tag + 'n')}:")
+        self.e(f"s_mov_b64 exec, {sp(HDR)}")           # a compare leaves 0 for lanes that are off
+        self.e(f"s_and_b32 vcc_lo, s{b}, 0xffff")
+        self.e("v_and_b32 %[vt], vcc_lo, %[tid]")
+        self.e(f"s_lshr_b32 vcc_lo, s{b}, 16")
+        self.e("v_cmp_eq_u32 vcc, vcc_lo, %[vt]")
+        self.e(f"s_and_b64 exec, {sp(HDR)}, vcc")
+        v = b + 2 if self.ts == 4 else b + 4
+        pr, pi = self.sval(v, 0), self.sval(v, 1)
+        self.e(f"v_mul_{f} %[t2], {pi}, %[t1]")
+        self.e(f"v_mul_{f} %[t3], {pi}, %[t0]")
+        self.e(f"v_fma_{f} %[t0], {pr}, %[t0], -%[t2]")
+        self.e(f"v_fma_{f} %[t1], {pr}, %[t1], %[t3]")
+        self.e(f"{self.lbl(tag + 's')}:")
+        self.e(f"s_bitcmp1_b32 s{b + 1}, 10")
+        self.e(f"s_cbranch_scc1 {self.lbl(done)}")
+
+    def h_fan(self):
+        tw = FAN_TERM[self.ts] // 4
+        first = 12 // tw                              # whole terms in the header's 64 bytes
+        ptr = HDR + 2
+        self.e(f"s_mov_b32 s{SCR}, s{HDR + 1}")       # the FM_* code
+        self.e(f"s_mov_b64 {sp(HDR)}, exec")
+        self.e(f"s_add_u32 s{ptr}, s{OFF}, {16 + first * FAN_TERM[self.ts]}")
+        self.e(f"s_load_dwordx16 s[{BUF2}:{BUF2 + 15}], %[prog], s{ptr}")
+        if self.d:
+            self.e("v_cvt_f64_i32 %[t0], 1")
+            self.e("v_cvt_f64_i32 %[t1], 0")
+        else:
+            self.e("v_mov_b32 %[t0], 1.0")
+            self.e("v_mov_b32 %[t1], 0")
+        for i in range(first):
+            self.fan_term(COEF + tw * i, f"fh{i}", "fandone")
+        self.e(f"{self.lbl('fanloop')}:")
+        self.e("s_waitcnt lgkmcnt(0)")
+        for i in range(16 // tw):
+            self.fan_term(BUF2 + tw * i, f"fb{i}", "fandone")
+        self.e(f"s_add_u32 s{ptr}, s{ptr}, 64")
+        self.e(f"s_load_dwordx16 s[{BUF2}:{BUF2 + 15}], %[prog], s{ptr}")
+        self.e(f"s_branch {self.lbl('fanloop')}")
+        self.e(f"{self.lbl('fandone')}:")
+        self.e(f"s_mov_b64 exec, {sp(HDR)}")
+        self.e("s_waitcnt lgkmcnt(0)")                # a load ahead may still be on its way
+        self.e(f"s_lshl2_add_u32 s36, s{SCR}, s{TAB}")
+        self.e(f"s_addc_u32 s37, s{TAB + 1}, 0")
+        self.e("s_setpc_b64 s[36:37]")
+
+    def h_fm(self, name, params):
+        f = self.f
+        for j in self.sel(name, params):
+            self.e(f"v_mul_{f} %[t2], %[t1], {self.im(j)}")
+            self.e(f"v_mul_{f} %[t3], %[t1], {self.re(j)}")
+            self.e(f"v_fma_{f} {self.re(j)}, %[t0], {self.re(j)}, -%[t2]")
+            self.e(f"v_fma_{f} {self.im(j)}, %[t0], {self.im(j)}, %[t3]")
+        self.e(f"s_add_u32 s{OFF}, s{OFF}, s{HDR + 3}")
+        self.dispatch()
+
     # --- the whole interpreter -----------------------------------------------
     def build(self):
         e = self.e
@@ -483,6 +566,10 @@ class Gen:
                 self.h_rmat(params)
             elif name.startswith("TSH"):
                 self.h_tsh(name, params, tag)
+            elif name == "FAN":
+                self.h_fan()
+            elif name.startswith("FM"):
+                self.h_fm(name, params)
         e(f"{self.lbl('end')}:")
         return self.L
 

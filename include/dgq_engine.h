@@ -208,6 +208,10 @@ size_t dq_apply_ws_bytes(uint32_t n_blocks, uint32_t n_phases, uint32_t n_ops, u
  * src/cpp/QuEST_gpu_kernel.cu:175-359). */
 int dq_build_program(int prec, int reg_bits, const dq_op *ops, uint32_t n_ops, unsigned char *out, size_t cap,
                      size_t *len);
+/* The program as dq_apply_blocks uploads it: conditioned phases of one
+ * register condition gathered into one op where that is less work (op FAN). */
+int dq_build_program_gathered(int prec, int reg_bits, const dq_op *ops, uint32_t n_ops, unsigned char *out, size_t cap,
+                              size_t *len);
 
 /* P(qubit q = 0) for every qubit q < n, and the total probability in
  * out[n] (n + 1 doubles, host memory).  One read of the state plus a small
