@@ -2179,6 +2179,7 @@ struct ProgBuilder {
         uint32_t c_reg, v_reg;
         double fr, fi;
     };
+    static constexpr size_t kFanTerm = 32;  // bytes
     // NEG / PHASE ops of a diagonal run with a lane or workgroup condition, kept
     // by register condition (0: none, 1 + 2 r + v: bit r = v) until the run ends.
     std::vector<const dq_op *> held[1 + 2 * DQ_MAX_REG_BITS];
@@ -2215,7 +2216,7 @@ struct ProgBuilder {
                 h.clear();
                 continue;
             }
-            const size_t at = out.size(), tb = ts == 8 ? 32 : 16;
+            const size_t at = out.size(), tb = kFanTerm;
             out.resize(at + 16 + h.size() * tb, 0);
             unsigned char *w = out.data() + at;
             const uint32_t apply = (uint32_t)(g ? cd.FM_B[(g - 1) / 2][(g - 1) & 1] : cd.FM_ALL);
@@ -2229,12 +2230,7 @@ struct ProgBuilder {
                 if (i + 1 == h.size()) c[1] |= 0x400u;
                 memcpy(w, c, 8);
                 const double f[2] = {o.kind == DQ_OP_NEG ? -1.0 : val(o, 0), o.kind == DQ_OP_NEG ? 0.0 : val(o, 1)};
-                if (ts == 8) {
-                    memcpy(w + 16, f, 16);
-                } else {
-                    const float f4[2] = {(float)f[0], (float)f[1]};
-                    memcpy(w + 8, f4, 8);
-                }
+                memcpy(w + 16, f, 16);
             }
             h.clear();
             n_out++;
@@ -2428,7 +2424,7 @@ struct ProgBuilder {
             uint32_t fan[4];
             memcpy(fan, out.data() + at, 16);
             if (c == (uint32_t)cd.FAN) {  // whole terms, the last one marked: the handler's loop ends there
-                const size_t tb = ts == 8 ? 32 : 16;
+                const size_t tb = kFanTerm;
                 if (fan[1] < (uint32_t)cd.FM_ALL || fan[1] >= (uint32_t)ncodes || fan[3] <= 16 || (fan[3] - 16) % tb ||
                     at + fan[3] > out.size())
                     return false;

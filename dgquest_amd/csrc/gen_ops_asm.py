@@ -60,7 +60,7 @@ import itertools
 import sys
 
 BUF2, HDR, OFF, SCR, TAB = 36, 52, 68, 69, 70
-FAN_TERM = {4: 16, 8: 32}  # bytes of a FAN term by sizeof(T)
+FAN_TERM = 32           # bytes of a FAN term
 EXEC = BUF2             # saved exec of a lane-conditioned op (s[36:37])
 COEF = HDR + 4          # coefficients start right after the 16-byte header
 CLOBBER = range(36, 72)
@@ -462,10 +462,14 @@ class Gen:
     # Controlled phases between a register bit and lane, wave or workgroup bits
     # (a Fourier transform has one for every pair of qubits) multiplied every
     # selected register each: 2^R / 2 complex products and a dispatch per phase.
-    # Here a term is one complex product on the thread's factor (t0, t1), under
-    # its condition, and the registers are multiplied once for all terms.
+    # Here a term is one complex product on the thread's factor, under its
+    # condition, and the registers are multiplied once for all terms.  The
+    # factor is formed in FP64 in either precision: its rounding is common to all
+    # registers of a thread, so in FP32 it would add up in probabilities where
+    # the amplitudes' own roundings average out.  (FP64 multiplies issue at the
+    # rate of FP32 ones.)  FP64 keeps it in t0, t1, FP32 in f0, f1 until the end.
     def fan_term(self, b, tag, done):
-        f = self.f
+        f0, f1, f2, f3 = (f"%[{'t' if self.d else 'f'}{i}]" for i in range(4))
         self.e(f"s_bitcmp1_b32 s{b + 1}, 8")
         self.e(f"s_cbranch_scc0 {self.lbl(tag + 'n')}")
         self.e(f"s_lshr_b64 vcc, %[base], s{b + 1}")   # the shift is the low 6 bits, the bit number
@@ -480,41 +484,36 @@ class Gen:
         self.e(f"s_lshr_b32 vcc_lo, s{b}, 16")
         self.e("v_cmp_eq_u32 vcc, vcc_lo, %[vt]")
         self.e(f"s_and_b64 exec, {sp(HDR)}, vcc")
-        v = b + 2 if self.ts == 4 else b + 4
-        pr, pi = self.sval(v, 0), self.sval(v, 1)
-        self.e(f"v_mul_{f} %[t2], {pi}, %[t1]")
-        self.e(f"v_mul_{f} %[t3], {pi}, %[t0]")
-        self.e(f"v_fma_{f} %[t0], {pr}, %[t0], -%[t2]")
-        self.e(f"v_fma_{f} %[t1], {pr}, %[t1], %[t3]")
+        self.e(f"v_mul_f64 {f2}, {sp(b + 6)}, {f1}")
+        self.e(f"v_mul_f64 {f3}, {sp(b + 6)}, {f0}")
+        self.e(f"v_fma_f64 {f0}, {sp(b + 4)}, {f0}, -{f2}")
+        self.e(f"v_fma_f64 {f1}, {sp(b + 4)}, {f1}, {f3}")
         self.e(f"{self.lbl(tag + 's')}:")
         self.e(f"s_bitcmp1_b32 s{b + 1}, 10")
         self.e(f"s_cbranch_scc1 {self.lbl(done)}")
 
     def h_fan(self):
-        tw = FAN_TERM[self.ts] // 4
-        first = 12 // tw                              # whole terms in the header's 64 bytes
         ptr = HDR + 2
+        f0, f1 = ("%[t0]", "%[t1]") if self.d else ("%[f0]", "%[f1]")
         self.e(f"s_mov_b32 s{SCR}, s{HDR + 1}")       # the FM_* code
         self.e(f"s_mov_b64 {sp(HDR)}, exec")
-        self.e(f"s_add_u32 s{ptr}, s{OFF}, {16 + first * FAN_TERM[self.ts]}")
+        self.e(f"s_add_u32 s{ptr}, s{OFF}, {16 + FAN_TERM}")
         self.e(f"s_load_dwordx16 s[{BUF2}:{BUF2 + 15}], %[prog], s{ptr}")
-        if self.d:
-            self.e("v_cvt_f64_i32 %[t0], 1")
-            self.e("v_cvt_f64_i32 %[t1], 0")
-        else:
-            self.e("v_mov_b32 %[t0], 1.0")
-            self.e("v_mov_b32 %[t1], 0")
-        for i in range(first):
-            self.fan_term(COEF + tw * i, f"fh{i}", "fandone")
+        self.e(f"v_cvt_f64_i32 {f0}, 1")
+        self.e(f"v_cvt_f64_i32 {f1}, 0")
+        self.fan_term(COEF, "fh", "fandone")          # the header's load holds the first term
         self.e(f"{self.lbl('fanloop')}:")
         self.e("s_waitcnt lgkmcnt(0)")
-        for i in range(16 // tw):
-            self.fan_term(BUF2 + tw * i, f"fb{i}", "fandone")
+        for i in range(2):
+            self.fan_term(BUF2 + 8 * i, f"fb{i}", "fandone")
         self.e(f"s_add_u32 s{ptr}, s{ptr}, 64")
         self.e(f"s_load_dwordx16 s[{BUF2}:{BUF2 + 15}], %[prog], s{ptr}")
         self.e(f"s_branch {self.lbl('fanloop')}")
         self.e(f"{self.lbl('fandone')}:")
         self.e(f"s_mov_b64 exec, {sp(HDR)}")
+        if not self.d:
+            self.e("v_cvt_f32_f64 %[t0], %[f0]")
+            self.e("v_cvt_f32_f64 %[t1], %[f1]")
         self.e("s_waitcnt lgkmcnt(0)")                # a load ahead may still be on its way
         self.e(f"s_lshl2_add_u32 s36, s{SCR}, s{TAB}")
         self.e(f"s_addc_u32 s37, s{TAB + 1}, 0")
@@ -580,6 +579,8 @@ class Gen:
         out.append(f"    __device__ __forceinline__ static void run(Regs<{self.T}, {self.R}> &a, const void *prog,")
         out.append("                                               uint64_t base, uint32_t tid) {")
         out.append(f"        {self.T} t0, t1, t2, t3;")
+        if not self.d:
+            out.append("        double f0, f1, f2, f3;")
         out.append("        uint32_t vt;")
         out.append("        asm volatile(")
         for ln in body:
@@ -587,6 +588,7 @@ class Gen:
             out.append(f'            "{pre}{ln}\\n"')
         outs = [f'[re{j}] "+v"(a.re[{j}])' for j in range(self.NR)] + \
                [f'[im{j}] "+v"(a.im[{j}])' for j in range(self.NR)] + \
+               ([] if self.d else [f'[f{i}] "=&v"(f{i})' for i in range(4)]) + \
                ['[t0] "=&v"(t0)', '[t1] "=&v"(t1)', '[t2] "=&v"(t2)', '[t3] "=&v"(t3)', '[vt] "=&v"(vt)']
         ins = ['[prog] "s"(prog)', '[base] "s"(base)', '[tid] "v"(tid)']
         out.append("            : " + ",\n              ".join(outs))

@@ -34,7 +34,7 @@ def build(eng, prec, R, ops):
 
 def run_gathered(A, prog, prec, R, base):
     """Returns the number of FAN terms run."""
-    ts, ft = (8, np.float64) if prec == 2 else (4, np.float32)
+    ts = 8 if prec == 2 else 4
     codes = GEN.op_codes(R)
     end = np.array([codes.index(("END", ())), 0, 0, 0], dtype=np.uint32).tobytes()
     tid = np.arange(A.shape[0])
@@ -55,13 +55,13 @@ def run_gathered(A, prog, prec, R, base):
             M.run_program(A, prog[at:at + size] + end, prec, R, base)
             at += size
             continue
-        tb = GEN.FAN_TERM[ts]
+        tb = GEN.FAN_TERM
         f = np.ones(A.shape[0], dtype=np.complex128)
         assert (size - 16) % tb == 0 and size > 16
         for k in range((size - 16) // tb):
             p = at + 16 + k * tb
             lane, wg = (int(x) for x in np.frombuffer(prog, dtype=np.uint32, count=2, offset=p))
-            re, im = np.frombuffer(prog, dtype=ft, count=2, offset=p + tb - 2 * ts).astype(np.float64)
+            re, im = np.frombuffer(prog, dtype=np.float64, count=2, offset=p + 16)
             assert bool(wg & 0x400) == (p + tb == at + size)  # only the last term is marked
             terms += 1
             if wg & 0x100 and ((base >> (wg & 63)) ^ (wg >> 9)) & 1:
