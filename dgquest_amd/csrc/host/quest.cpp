@@ -412,14 +412,35 @@ void ensure_probs(QuregState *s) {
     s->det_base = true;
 }
 
-// Move every logical qubit back to its own physical position with
-// permutation sweeps (each moves at most one tile's worth of qubits).
+// Registers of at most this many qubits (the small kernel's) swap by gates.
+static const int kPermuteMin = 6;
+
+// Move every logical qubit back to its own physical position: one or two
+// passes over the state, or one permutation sweep where the qubits that move fit
+// its tile.
 void materialize_mapping(QuregState *s) {
     flush(s);
     const int n = s->n;
     bool ident = true;
     for (int q = 0; q < n; q++) ident &= s->l2p[q] == q;
     if (ident) return;
+    if (n > kPermuteMin) {
+        // a sweep's tile moves a few qubits more than the permutation kernel's: one
+        // pass of it where that is enough and the kernel would take two
+        int dest[64], high = 0;
+        for (int q = 0; q < n; q++) {
+            dest[s->l2p[q]] = q;
+            high += q >= 6 && s->l2p[q] != q;
+        }
+        const TuneParams t = fit_shape(s->tune, n, s->prec);
+        if (dq_permute_launches(n, s->prec, dest) == 1 || high > t.R + t.W) {
+            ENG(dq_permute_qubits(s->d_state, n, s->prec, dest, s->stream));
+            for (int q = 0; q < n; q++) s->l2p[q] = s->p2l[q] = q;
+            s->probs_dirty = true;
+            s->det_base = false;
+            return;
+        }
+    }
     std::vector<Plan> passes;
     std::vector<Gate> gates;
     std::string err;

@@ -323,6 +323,14 @@ int dq_compare_states(const void *a, int prec_a, const void *b, int prec_b, int 
 size_t dq_compare_ws_bytes(int n_qubits);
 
 /* 0 if all work recorded before `ev` has completed, 1 if not yet (no wait). */
+/* The qubits of a state permuted in place: the amplitude at index x moves to
+ * the index whose bit dest[p] is bit p of x.  One pass over the state if dest
+ * is an involution or moves few bits, two otherwise; no workspace, no sync.
+ * dq_permute_launches: that number of passes (0 for the identity), or a
+ * negative error code.  Takes the place of the reference's reorder_data_kernel
+ * (src/cpp/QuEST_gpu_kernel.cu:589-636) for a whole register. */
+int dq_permute_qubits(void *state, int n_qubits, int prec, const int *dest, void *stream);
+int dq_permute_launches(int n_qubits, int prec, const int *dest);
 int dq_event_query(void *ev);
 /* Wait for the work recorded before `ev`. */
 int dq_event_sync(void *ev);
