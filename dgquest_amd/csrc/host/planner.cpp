@@ -772,6 +772,20 @@ void hand_over_lanes(uint64_t from, uint64_t next, std::vector<int> &pos) {
     for (size_t j = 0; j < out.size() && j < in.size(); j++) std::swap(pos[out[j]], pos[in[j]]);
 }
 
+// Positions after a last block whose store brings the labels end_lanes[0..5] to
+// positions 0..5, each swapping with the label there; unchanged unless all of
+// them lie in the block's tile (positions ptile).
+std::vector<int> home_lanes(uint64_t ptile, const int *end_lanes, std::vector<int> pos) {
+    for (int l = 0; l < 6; l++)
+        if (!((ptile >> pos[end_lanes[l]]) & 1)) return pos;
+    for (int l = 0; l < 6; l++) {
+        const int a = end_lanes[l];
+        const int b = (int)(std::find(pos.begin(), pos.end(), l) - pos.begin());
+        std::swap(pos[a], pos[b]);
+    }
+    return pos;
+}
+
 uint64_t to_positions(uint64_t labels, const std::vector<int> &pos) {
     uint64_t m = 0;
     for (; labels; labels &= labels - 1) m |= 1ull << pos[ctz64(labels)];
@@ -781,11 +795,13 @@ uint64_t to_positions(uint64_t labels, const std::vector<int> &pos) {
 }  // namespace
 
 void plan_circuit(const std::vector<Gate> &gates, int n, int prec, int init_kind, uint64_t init_index,
-                  double init_value, const TuneParams &tp, Plan &P, int n_local, bool rotate_lanes) {
+                  double init_value, const TuneParams &tp, Plan &P, int n_local, bool rotate_lanes, const int *end_lanes) {
     if (n_local < 0 || n_local > n) n_local = n;
+    if (n_local != n) end_lanes = nullptr;
     P.blocks.clear();
     P.phases.clear();
     P.ops.clear();
+    P.moved.clear();
     P.st = PlanStats();
     P.st.gates_in = (int)gates.size();
 
@@ -905,6 +921,9 @@ void plan_circuit(const std::vector<Gate> &gates, int n, int prec, int init_kind
             const uint64_t next = i + 1 < rbg.size() ? rlanes[i + 1] : rlanes[i];
             std::vector<int> pos2 = pos;
             hand_over_lanes(rlanes[i], next, pos2);
+            const bool end = i + 1 == rbg.size();
+            if (end && end_lanes) pos2 = home_lanes(ptile, end_lanes, pos);
+            const bool moves = pos2 != pos;
             std::vector<int> at(n);
             for (int q = 0; q < n; q++) at[pos[q]] = q;
             uint8_t store_pos[DQ_MAX_TILE_BITS];
@@ -912,8 +931,8 @@ void plan_circuit(const std::vector<Gate> &gates, int n, int prec, int init_kind
             for (int p = 0; p < n; p++)
                 if ((ptile >> p) & 1) store_pos[b++] = (uint8_t)pos2[at[p]];
             emit_block(hg, ptile, n, n_local, t, prec, i == 0 ? init_kind : DQ_INIT_LOAD, init_index, init_value, F,
-                       i + 1 == rbg.size(), P, next != rlanes[i] ? store_pos : nullptr);
-            if (next != rlanes[i]) {
+                       end, P, moves ? store_pos : nullptr);
+            if (moves) {
                 std::vector<int> to(n);
                 for (int q = 0; q < n; q++) to[pos[q]] = pos2[q];
                 F.permute(to);
@@ -934,10 +953,87 @@ void plan_circuit(const std::vector<Gate> &gates, int n, int prec, int init_kind
     for (const auto &bg : bgs)
         for (const Gate &g : bg)
             if (!gate_is_diagonal(g.type)) F.left[ctz64(g.tmask)]++;
-    for (size_t i = 0; i < bgs.size(); i++)
-        emit_block(bgs[i], tms[i], n, n_local, t, prec, i == 0 ? init_kind : DQ_INIT_LOAD, init_index, init_value, F,
-                   i + 1 == bgs.size(), P);
+    for (size_t i = 0; i < bgs.size(); i++) {
+        const bool end = i + 1 == bgs.size();
+        uint8_t store_pos[DQ_MAX_TILE_BITS];
+        bool moves = false;
+        if (end && end_lanes) {
+            uint64_t tile = tms[i] | 0x3Full;  // as emit_block pads it
+            for (int q = 6; q < n && popc64(tile) < T; q++) tile |= 1ull << q;
+            std::vector<int> pos(n);
+            for (int q = 0; q < n; q++) pos[q] = q;
+            const std::vector<int> pos2 = home_lanes(tile, end_lanes, pos);
+            moves = pos2 != pos;
+            int b = 0;
+            for (int q = 0; q < n; q++)
+                if ((tile >> q) & 1) store_pos[b++] = (uint8_t)pos2[q];
+            if (moves) P.moved = pos2;
+        }
+        emit_block(bgs[i], tms[i], n, n_local, t, prec, i == 0 ? init_kind : DQ_INIT_LOAD, init_index, init_value, F, end, P,
+                   moves ? store_pos : nullptr);
+    }
     P.st.ops = (int)P.ops.size();
+}
+
+void rename_to_home(Plan &P, int n, const std::vector<int> &l2p) {
+    if (P.blocks.empty() || P.blocks[0].init_kind == DQ_INIT_LOAD) return;
+    if (P.moved.empty()) {
+        P.moved.resize(n);
+        for (int q = 0; q < n; q++) P.moved[q] = q;
+    }
+    // rho: new name of each position; 0..5 keep theirs
+    std::vector<int> rho(n, -1);
+    uint64_t taken = 0x3Full;
+    for (int p = 0; p < n && p < 6; p++) rho[p] = p;
+    for (int q = 6; q < n; q++) {
+        const int f = P.moved[l2p[q]];
+        if (f < 6) continue;
+        rho[f] = q;
+        taken |= 1ull << q;
+    }
+    // lane l holds x, the qubit l is at a position above: give that position the
+    // name x, so that undoing the rest swaps the two (an involution is one pass)
+    for (int x = 6; x < n; x++) {
+        const int l = P.moved[l2p[x]];
+        if (l >= 6) continue;
+        const int f = P.moved[l2p[l]];
+        if (f < 6) continue;
+        rho[f] = x;
+        taken |= 1ull << x;
+    }
+    for (int p = 6, f = 6; p < n; p++) {
+        if (rho[p] >= 0) continue;
+        while ((taken >> f) & 1) f++;
+        rho[p] = f;
+        taken |= 1ull << f;
+    }
+    bool same = true;
+    for (int p = 0; p < n; p++) same &= rho[p] == p;
+    if (!same) {
+        auto map = [&](uint64_t m) {
+            uint64_t o = 0;
+            for (; m; m &= m - 1) o |= 1ull << rho[ctz64(m)];
+            return o;
+        };
+        for (dq_block &b : P.blocks) {
+            b.nontile_mask = map(b.nontile_mask);
+            if (b.init_kind == DQ_INIT_CLASSICAL) b.init_index = map(b.init_index);
+            for (uint32_t r = 0; r < b.reg_bits; r++) {
+                b.ld_reg[r] = map(b.ld_reg[r]);
+                b.st_reg[r] = map(b.st_reg[r]);
+            }
+            for (uint32_t w = 0; w < b.wave_bits; w++) {
+                b.ld_wave[w] = map(b.ld_wave[w]);
+                b.st_wave[w] = map(b.st_wave[w]);
+            }
+        }
+        for (dq_op &o : P.ops)
+            if (o.c_wg) {
+                o.c_wg = map(o.c_wg);
+                o.v_wg = map(o.v_wg);
+            }
+        for (int q = 0; q < n; q++) P.moved[q] = rho[P.moved[q]];
+    }
 }
 
 bool plan_permutation(int n, int prec, const std::vector<int> &src, const std::vector<int> &dst,

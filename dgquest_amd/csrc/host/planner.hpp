@@ -65,8 +65,21 @@ struct Plan {
 // has 13 useful tile qubits rather than 7 and the six fixed ones.  The
 // partition is kept only when it needs fewer sweeps than fixed lanes; the
 // caller composes out.moved into its qubit map.
+//
+// end_lanes (or null; whole registers only): the last block stores the qubits at
+// start positions end_lanes[0..5] to positions 0..5, in order, when they all lie
+// in its tile.
 void plan_circuit(const std::vector<Gate> &gates, int n, int prec, int init_kind, uint64_t init_index,
-                  double init_value, const TuneParams &tp, Plan &out, int n_local = -1, bool rotate_lanes = false);
+                  double init_value, const TuneParams &tp, Plan &out, int n_local = -1, bool rotate_lanes = false,
+                  const int *end_lanes = nullptr);
+
+// Rename the positions 6 and up of a plan that generates its own state (basis or
+// plus state), so that as many of them as possible end at home: the qubit at
+// start position l2p[q] at position q.  Where a generated state begins is free,
+// so this costs nothing on the device, and a map that the plan's own moves and
+// the recorded relabellings leave needs no pass to be undone (or a smaller one,
+// where lanes are not at home).  out.moved then includes the renaming.
+void rename_to_home(Plan &P, int n, const std::vector<int> &l2p);
 
 // A pass that only moves qubits: afterwards physical qubit dst[i] holds what
 // physical qubit src[i] held.  All moved qubits must fit one tile.

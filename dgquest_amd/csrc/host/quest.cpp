@@ -260,8 +260,12 @@ static bool same_gate(const Gate &a, const Gate &b) {
 }
 
 // Was the register's last plan made from exactly what it now holds?
-static bool plan_is_cached(const QuregState *s, const TuneParams &t, bool rot) {
+// A plan that ends with other lanes than wanted runs the same gates; only for a
+// state that is handed out next is one with the wanted lanes made (unless the
+// search picked the plan).
+static bool plan_is_cached(const QuregState *s, const TuneParams &t, bool rot, const std::vector<int> &end_lanes) {
     const auto &c = s->cache;
+    if (!end_lanes.empty() && !c.searched && c.end_lanes != end_lanes) return false;
     if (!c.valid || c.rotate != rot || !same_shape(c.tune, t) || c.init_kind != s->init_kind ||
         c.init_index != s->init_index || c.init_value != s->init_value || c.gates.size() != s->pending.size())
         return false;
@@ -270,9 +274,12 @@ static bool plan_is_cached(const QuregState *s, const TuneParams &t, bool rot) {
     return true;
 }
 
-static void cache_plan(QuregState *s, const TuneParams &t, bool rot, const Plan &P) {
+static void cache_plan(QuregState *s, const TuneParams &t, bool rot, const Plan &P, bool searched,
+                       const std::vector<int> &end_lanes) {
     auto &c = s->cache;
     c.valid = true;
+    c.searched = searched;
+    c.end_lanes = end_lanes;
     c.gates = s->pending;
     c.init_kind = s->init_kind;
     c.init_index = s->init_index;
@@ -282,13 +289,16 @@ static void cache_plan(QuregState *s, const TuneParams &t, bool rot, const Plan 
     c.plan = P;
 }
 
+// Registers of at most this many qubits (the small kernel's) swap by gates.
+static const int kPermuteMin = 6;
+
 static bool rotation_allowed(const QuregState *s) { return s->rotate >= 0 ? s->rotate != 0 : rotate_lanes(); }
 static bool rotation_for(const QuregState *s) {
     if (s->rotate < 0 && s->rotate_pick >= 0) return s->rotate_pick != 0;
     return rotation_allowed(s);
 }
 
-void flush(QuregState *s) {
+void flush(QuregState *s, bool home) {
     if (s->recorder) engine_fatal("a recording register cannot execute or read its state", DQ_ERR_UNSUPPORTED);
     if (s->pending.empty() && s->init_kind == DQ_INIT_LOAD) return;
     s->det_base = false;
@@ -336,12 +346,16 @@ void flush(QuregState *s) {
     } else {
         Plan P;
         const bool rot = rotation_for(s);
-        if (plan_is_cached(s, s->tune, rot)) {
+        home = home && s->init_kind != DQ_INIT_LOAD && s->n > kPermuteMin;
+        const std::vector<int> end_lanes(s->l2p.begin(), s->l2p.begin() + (home ? 6 : 0));
+        if (plan_is_cached(s, s->tune, rot, end_lanes)) {
             P = s->cache.plan;
         } else {
-            plan_circuit(s->pending, s->n, s->prec, s->init_kind, s->init_index, s->init_value, s->tune, P, -1, rot);
-            cache_plan(s, s->tune, rot, P);
+            plan_circuit(s->pending, s->n, s->prec, s->init_kind, s->init_index, s->init_value, s->tune, P, -1, rot,
+                         home ? end_lanes.data() : nullptr);
+            cache_plan(s, s->tune, rot, P, false, end_lanes);
         }
+        if (home) rename_to_home(P, s->n, s->l2p);
         run_plan(s, P);
         if (!P.moved.empty()) {  // the plan moved qubits: logical q now sits at moved[l2p[q]]
             for (int q = 0; q < s->n; q++) s->l2p[q] = P.moved[s->l2p[q]];
@@ -412,14 +426,11 @@ void ensure_probs(QuregState *s) {
     s->det_base = true;
 }
 
-// Registers of at most this many qubits (the small kernel's) swap by gates.
-static const int kPermuteMin = 6;
-
 // Move every logical qubit back to its own physical position: one or two
 // passes over the state, or one permutation sweep where the qubits that move fit
 // its tile.
 void materialize_mapping(QuregState *s) {
-    flush(s);
+    flush(s, true);
     const int n = s->n;
     bool ident = true;
     for (int q = 0; q < n; q++) ident &= s->l2p[q] == q;
@@ -628,7 +639,7 @@ void searchQuregTaskPartitions(Qureg qureg, QuESTEnv env) {
         }
     }
     if (have) {
-        cache_plan(s, s->tune, rotation_for(s), pick);
+        cache_plan(s, s->tune, rotation_for(s), pick, true, {});
         s->predicted_ms = best;
     }
 }
@@ -1199,8 +1210,8 @@ Qureg dgq_create_recorder(int numQubits) {
 
 void dgq_destroy_recorder(Qureg q) { destroyQureg(q, q.env); }
 
-int dgq_recorder_plan(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_block *blocks, int cap_blocks,
-                      dq_phase *phases, int cap_phases, dq_op *ops, int cap_ops, int counts[3], int *l2p) {
+static int recorder_plan(Qureg q, bool home, int k, int R, int W, int max_ops, int fuse, dq_block *blocks, int cap_blocks,
+                         dq_phase *phases, int cap_phases, dq_op *ops, int cap_ops, int counts[3], int *l2p) {
     QuregState *s = q.state;
     if (!s || !s->recorder || !counts) return -1;
     TuneParams tp;
@@ -1210,7 +1221,10 @@ int dgq_recorder_plan(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_bl
     tp.max_ops = max_ops;
     tp.fuse_diagonals = fuse != 0;
     Plan P;
-    plan_circuit(s->pending, s->n, s->prec, s->init_kind, s->init_index, s->init_value, tp, P, -1, rotation_for(s));
+    home = home && s->init_kind != DQ_INIT_LOAD && s->n > kPermuteMin;
+    plan_circuit(s->pending, s->n, s->prec, s->init_kind, s->init_index, s->init_value, tp, P, -1, rotation_for(s),
+                 home ? s->l2p.data() : nullptr);
+    if (home) rename_to_home(P, s->n, s->l2p);
     counts[0] = (int)P.blocks.size();
     counts[1] = (int)P.phases.size();
     counts[2] = (int)P.ops.size();
@@ -1221,6 +1235,16 @@ int dgq_recorder_plan(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_bl
     if (counts[1]) memcpy(phases, P.phases.data(), P.phases.size() * sizeof(dq_phase));
     if (counts[2]) memcpy(ops, P.ops.data(), P.ops.size() * sizeof(dq_op));
     return 0;
+}
+
+int dgq_recorder_plan(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_block *blocks, int cap_blocks,
+                      dq_phase *phases, int cap_phases, dq_op *ops, int cap_ops, int counts[3], int *l2p) {
+    return recorder_plan(q, false, k, R, W, max_ops, fuse, blocks, cap_blocks, phases, cap_phases, ops, cap_ops, counts, l2p);
+}
+
+int dgq_recorder_plan_home(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_block *blocks, int cap_blocks,
+                           dq_phase *phases, int cap_phases, dq_op *ops, int cap_ops, int counts[3], int *l2p) {
+    return recorder_plan(q, true, k, R, W, max_ops, fuse, blocks, cap_blocks, phases, cap_phases, ops, cap_ops, counts, l2p);
 }
 
 int dgq_recorder_export(Qureg q, dgq_gate_rec *gates, int cap, int *n_gates, int *l2p, int *init_kind,

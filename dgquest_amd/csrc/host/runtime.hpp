@@ -59,6 +59,8 @@ struct QuregState {
         double init_value = 0.0;
         dgq::TuneParams tune;
         bool rotate = false;
+        bool searched = false;         // searchQuregTaskPartitions' pick
+        std::vector<int> end_lanes;    // plan_circuit's end_lanes (empty: none)
         dgq::Plan plan;
     } cache;
     double predicted_ms = 0.0;        // searchQuregTaskPartitions' predicted device ms (0: no search)
@@ -75,7 +77,9 @@ namespace dgq {
 
 [[noreturn]] void engine_fatal(const char *what, int rc);
 void ensure_ws(QuregState *s, size_t bytes);
-void flush(QuregState *s);
+// home: the caller wants the state in logical qubit order next; a plan that
+// generates its state then ends there as far as it can (rename_to_home).
+void flush(QuregState *s, bool home = false);
 void ensure_probs(QuregState *s);
 void materialize_mapping(QuregState *s);
 

@@ -106,6 +106,12 @@ void dgq_destroy_recorder(Qureg q);
 int dgq_recorder_plan(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_block *blocks, int cap_blocks,
                       dq_phase *phases, int cap_phases, dq_op *ops, int cap_ops, int counts[3], int *l2p);
 
+/* The same for a flush whose state is handed out in logical qubit order next
+ * (dgq_state_pointer, sampling, overlaps, setAmps): a plan that generates its
+ * state ends with the qubits at home as far as it can. */
+int dgq_recorder_plan_home(Qureg q, int k, int R, int W, int max_ops, int fuse, dq_block *blocks, int cap_blocks,
+                           dq_phase *phases, int cap_phases, dq_op *ops, int cap_ops, int counts[3], int *l2p);
+
 /* The recording of q as gate records (physical qubit positions, the encoding
  * of src/cpp/QuEST_backend.h:160-178) for another executor such as the
  * request server of dgq_serve.h: *n_gates receives the count; gates (cap
