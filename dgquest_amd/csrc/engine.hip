@@ -963,28 +963,64 @@ readout_sample(const void *const *__restrict__ states, int n, RoLevels lv, const
 // comparison of two states of one size (any precisions): <a|b>, <a|a>, <b|b>
 // and max |a_i - b_i|
 // ----------------------------------------------------------------------------
+// Bound: HBM, one read of each state.  A thread has 8 amplitudes of either state in
+// flight, sums those first and adds the sums to its totals (short chains of
+// additions); workgroups are added up to 2^CMP_GROUPS_LOG, from shares of one such
+// step.  One amplitude per loop step and 2^16 amplitudes per workgroup left a
+// state of up to 16 qubits on one workgroup and large ones waiting
+// for loads.  27 qubits FP64, both stages: 741 -> 627 us (5.8 -> 6.9 TB/s).
 #define CMP_SLOTS 5
+#define CMP_LOADS_LOG 3    // amplitudes of either state in flight per thread
+#define CMP_GROUPS_LOG 13
+
+// qubits of a workgroup's share of an n-qubit state (>= 8 + CMP_LOADS_LOG, fewer for a smaller state)
+static int cmp_share(int n) { return std::min(n, std::max(8 + CMP_LOADS_LOG, n - CMP_GROUPS_LOG)); }
 
 template <typename TA, typename TB>
 __global__ void __launch_bounds__(256)
-compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB>::type *__restrict__ b, int n,
+compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB>::type *__restrict__ b, int share,
                double *__restrict__ part) {
+    constexpr uint32_t J = 1u << CMP_LOADS_LOG;
     __shared__ double red[4][CMP_SLOTS];
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int cb = n < PROB_WG_BITS ? n : PROB_WG_BITS;
-    const uint64_t g0 = (uint64_t)blockIdx.x << cb;
-    const uint32_t cnt = 1u << cb;
+    const uint64_t cnt = 1ull << share;
+    a += (uint64_t)blockIdx.x << share;
+    b += (uint64_t)blockIdx.x << share;
     double re = 0.0, im = 0.0, aa = 0.0, bb = 0.0, mx = 0.0;
-    for (uint32_t i = tid; i < cnt; i += 256) {
-        const typename V2<TA>::type x = a[g0 + i];
-        const typename V2<TB>::type y = b[g0 + i];
-        const double xr = x.x, xi = x.y, yr = y.x, yi = y.y;
-        re += xr * yr + xi * yi;
-        im += xr * yi - xi * yr;
-        aa += xr * xr + xi * xi;
-        bb += yr * yr + yi * yi;
-        const double dr = xr - yr, di = xi - yi;
-        mx = fmax(mx, dr * dr + di * di);
+    auto step = [&](const typename V2<TA>::type *x, const typename V2<TB>::type *y, uint32_t count) {
+        double r = 0.0, i = 0.0, p = 0.0, q = 0.0;
+#pragma unroll
+        for (uint32_t j = 0; j < count; j++) {
+            const double xr = x[j].x, xi = x[j].y, yr = y[j].x, yi = y[j].y;
+            r += xr * yr + xi * yi;
+            i += xr * yi - xi * yr;
+            p += xr * xr + xi * xi;
+            q += yr * yr + yi * yi;
+            const double dr = xr - yr, di = xi - yi;
+            mx = fmax(mx, dr * dr + di * di);
+        }
+        re += r;
+        im += i;
+        aa += p;
+        bb += q;
+    };
+    if (cnt >= 256 * J) {  // a multiple of it: both are powers of two
+        for (uint64_t i = tid; i < cnt; i += 256 * J) {
+            typename V2<TA>::type x[J];
+            typename V2<TB>::type y[J];
+#pragma unroll
+            for (uint32_t j = 0; j < J; j++) {
+                x[j] = __builtin_nontemporal_load(a + i + j * 256);
+                y[j] = __builtin_nontemporal_load(b + i + j * 256);
+            }
+            step(x, y, J);
+        }
+    } else {
+        for (uint64_t i = tid; i < cnt; i += 256) {
+            const typename V2<TA>::type x = a[i];
+            const typename V2<TB>::type y = b[i];
+            step(&x, &y, 1);
+        }
     }
     double v[CMP_SLOTS] = {wave_sum(re), wave_sum(im), wave_sum(aa), wave_sum(bb), wave_max(mx)};
     if (lane == 0)
@@ -993,7 +1029,7 @@ compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB
     if (tid < CMP_SLOTS) {
         const double r = tid == 4 ? fmax(fmax(red[0][4], red[1][4]), fmax(red[2][4], red[3][4]))
                                   : (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
-        part[(uint64_t)blockIdx.x * CMP_SLOTS + tid] = r;
+        part[(uint64_t)tid * gridDim.x + blockIdx.x] = r;
     }
 }
 
@@ -1310,24 +1346,20 @@ dense_form(const dq_small_gate *__restrict__ gates, const uint32_t *__restrict__
 }
 
 // one workgroup: out = {re <a|b>, im <a|b>, <a|a>, <b|b>, max |a_i - b_i|}
+// One workgroup per slot.
 __global__ void __launch_bounds__(256) compare_stage2(const double *__restrict__ part, uint32_t ngroups, double *__restrict__ out) {
-    __shared__ double red[4][CMP_SLOTS];
+    __shared__ double red[4];
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    double v[CMP_SLOTS] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (uint32_t g = tid; g < ngroups; g += 256) {
-        for (int k = 0; k < 4; k++) v[k] += part[(uint64_t)g * CMP_SLOTS + k];
-        v[4] = fmax(v[4], part[(uint64_t)g * CMP_SLOTS + 4]);
-    }
-    for (int k = 0; k < 4; k++) v[k] = wave_sum(v[k]);
-    v[4] = wave_max(v[4]);
-    if (lane == 0)
-        for (int k = 0; k < CMP_SLOTS; k++) red[w][k] = v[k];
+    const int k = blockIdx.x;
+    const double *__restrict__ src = part + (uint64_t)k * ngroups;
+    double v = 0.0;
+#pragma unroll 8
+    for (uint32_t g = tid; g < ngroups; g += 256) v = k == 4 ? fmax(v, src[g]) : v + src[g];
+    v = k == 4 ? wave_max(v) : wave_sum(v);
+    if (lane == 0) red[w] = v;
     __syncthreads();
-    if (tid < CMP_SLOTS) {
-        const double r = tid == 4 ? sqrt(fmax(fmax(red[0][4], red[1][4]), fmax(red[2][4], red[3][4])))
-                                  : (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]);
-        out[tid] = r;
-    }
+    if (tid == 0)
+        out[k] = k == 4 ? sqrt(fmax(fmax(red[0], red[1]), fmax(red[2], red[3]))) : (red[0] + red[1]) + (red[2] + red[3]);
 }
 
 // ----------------------------------------------------------------------------
@@ -3086,14 +3118,13 @@ extern "C" int dq_readout_many(int prec, int n, const void *const *states, uint3
 // ---- comparison of two states -------------------------------------------------
 extern "C" size_t dq_compare_ws_bytes(int n) {
     if (n < 1 || n > 40) return 0;
-    const int cb = n < PROB_WG_BITS ? n : PROB_WG_BITS;
-    return align_up(((size_t)1 << (n - cb)) * CMP_SLOTS * sizeof(double), 256);
+    return align_up(((size_t)1 << (n - cmp_share(n))) * CMP_SLOTS * sizeof(double), 256);
 }
 
 template <typename TA, typename TB>
-static void launch_compare(const void *a, const void *b, int n, unsigned groups, double *part, hipStream_t s) {
+static void launch_compare(const void *a, const void *b, int share, unsigned groups, double *part, hipStream_t s) {
     hipLaunchKernelGGL((compare_stage1<TA, TB>), dim3(groups), dim3(256), 0, s, (const typename V2<TA>::type *)a,
-                       (const typename V2<TB>::type *)b, n, part);
+                       (const typename V2<TB>::type *)b, share, part);
 }
 
 extern "C" int dq_compare_states(const void *a, int prec_a, const void *b, int prec_b, int n, double *d_out,
@@ -3101,16 +3132,16 @@ extern "C" int dq_compare_states(const void *a, int prec_a, const void *b, int p
     const bool pa = prec_a == DQ_F32 || prec_a == DQ_F64, pb = prec_b == DQ_F32 || prec_b == DQ_F64;
     if (!a || !b || !d_out || !pa || !pb || n < 1 || n > 40) return fail(DQ_ERR_ARG, "dq_compare_states: bad arguments");
     if (!d_ws || ws_bytes < dq_compare_ws_bytes(n)) return fail(DQ_ERR_ARG, "dq_compare_states: workspace too small");
-    const int cb = n < PROB_WG_BITS ? n : PROB_WG_BITS;
-    const uint64_t groups = 1ull << (n - cb);
+    const int share = cmp_share(n);
+    const uint64_t groups = 1ull << (n - share);
     double *part = (double *)d_ws;
     hipStream_t s = (hipStream_t)stream;
-    if (prec_a == DQ_F64 && prec_b == DQ_F64) launch_compare<double, double>(a, b, n, (unsigned)groups, part, s);
-    else if (prec_a == DQ_F64) launch_compare<double, float>(a, b, n, (unsigned)groups, part, s);
-    else if (prec_b == DQ_F64) launch_compare<float, double>(a, b, n, (unsigned)groups, part, s);
-    else launch_compare<float, float>(a, b, n, (unsigned)groups, part, s);
+    if (prec_a == DQ_F64 && prec_b == DQ_F64) launch_compare<double, double>(a, b, share, (unsigned)groups, part, s);
+    else if (prec_a == DQ_F64) launch_compare<double, float>(a, b, share, (unsigned)groups, part, s);
+    else if (prec_b == DQ_F64) launch_compare<float, double>(a, b, share, (unsigned)groups, part, s);
+    else launch_compare<float, float>(a, b, share, (unsigned)groups, part, s);
     HIPC(hipGetLastError());
-    hipLaunchKernelGGL(compare_stage2, dim3(1), dim3(256), 0, s, part, (uint32_t)groups, d_out);
+    hipLaunchKernelGGL(compare_stage2, dim3(CMP_SLOTS), dim3(256), 0, s, part, (uint32_t)groups, d_out);
     HIPC(hipGetLastError());
     return DQ_OK;
 }
