@@ -919,10 +919,13 @@ static void compare_regs(QuregState *a, QuregState *b, double out[5]) {
     double *host = (double *)dq_result_acquire(5 * sizeof(double));
     double *d_out = host ? host : (double *)((unsigned char *)a->d_ws + cw);
     ENG(dq_compare_states(a->d_state, a->prec, b->d_state, b->prec, a->n, d_out, a->d_ws, cw, a->stream));
-    if (!host) ENG(dq_memcpy_async(out, d_out, 5 * sizeof(double), DQ_D2H, a->stream));
-    ENG(dq_stream_sync(a->stream));
-    if (host) memcpy(out, host, 5 * sizeof(double));
-    dq_result_release(host);
+    if (host) {
+        ENG(dq_result_wait(host, out, 5 * sizeof(double), a->stream));
+        dq_result_release(host);
+    } else {
+        ENG(dq_memcpy_async(out, d_out, 5 * sizeof(double), DQ_D2H, a->stream));
+        ENG(dq_stream_sync(a->stream));
+    }
 }
 
 Complex calcInnerProduct(Qureg bra, Qureg ket) {
@@ -1286,12 +1289,14 @@ int dgq_sample(Qureg q, int shots, const double *u, unsigned long long *out) {
     const void *st = s->d_state;
     ENG(dq_readout_many(s->prec, s->n, &st, 1, u, (uint32_t)shots, nullptr, d_out, (unsigned char *)s->d_ws + res,
                         s->ws_cap - res, s->stream));
-    std::vector<uint64_t> idx(host ? 0 : (size_t)shots);
-    if (!host) ENG(dq_memcpy_async(idx.data(), d_out, (size_t)shots * sizeof(uint64_t), DQ_D2H, s->stream));
-    ENG(dq_stream_sync(s->stream));
-    const uint64_t *from = host ? host : idx.data();
-    for (int i = 0; i < shots; i++) out[i] = from[i];
-    dq_result_release(host);
+    static_assert(sizeof *out == sizeof(uint64_t), "samples are 64-bit words");
+    if (host) {
+        ENG(dq_result_wait(host, out, (size_t)shots * sizeof(uint64_t), s->stream));
+        dq_result_release(host);
+    } else {
+        ENG(dq_memcpy_async(out, d_out, (size_t)shots * sizeof(uint64_t), DQ_D2H, s->stream));
+        ENG(dq_stream_sync(s->stream));
+    }
     return 0;
 }
 

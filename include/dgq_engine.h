@@ -164,11 +164,14 @@ int dq_device_sync(void);
 #define DQ_D2D 3
 int dq_memcpy_async(void *dst, const void *src, size_t bytes, int kind, void *stream);
 /* A pinned host slot for the results of one synchronous read-out: a kernel
- * may store to it like to device memory, and the host reads it once the
- * stream is synchronised.  NULL when `bytes` is above 128 KiB or all 16 slots
- * are in use (results then go through device memory).  Release it after
- * reading; slots are shared by all threads and streams. */
+ * may store to it like to device memory, every 8-byte word once.  NULL when
+ * `bytes` is above 128 KiB or all 16 slots are in use (results then go through
+ * device memory).  Slots are shared by all threads and streams.
+ * dq_result_wait waits until kernels enqueued on `stream` have stored all
+ * `bytes` (a multiple of 8) and copies them to `out`; release the slot after
+ * it. */
 void *dq_result_acquire(size_t bytes);
+int dq_result_wait(const void *slot, void *out, size_t bytes, void *stream);
 void dq_result_release(void *slot);
 int dq_event_create(void **ev);
 int dq_event_destroy(void *ev);

@@ -111,3 +111,21 @@ def test_more_threads_than_slots(quest, env):
     for t in ts:
         t.join()
     assert not errs
+
+
+def test_read_of_the_unwritten_word(quest, env):
+    """An amplitude whose bits are those of a word that no kernel has stored is still read."""
+    n = 4
+    bits = np.array([0x7FF4DEAD00BEEF01], dtype=np.uint64)
+    re, im = np.zeros(1 << n), np.zeros(1 << n)
+    re[3:4], im[5:6] = bits.view(np.float64), bits.view(np.float64)
+    q = quest.createQureg(n, env)
+    ptr = C.POINTER(quest.qreal)
+    try:
+        quest.initStateFromAmps(q, re.ctypes.data_as(ptr), im.ctypes.data_as(ptr))
+        for _ in range(2):
+            v = quest.state_vector(q)
+            assert v.real.copy().view(np.uint64)[3] == bits[0] and v.imag.copy().view(np.uint64)[5] == bits[0]
+            assert np.count_nonzero(v.real.copy().view(np.uint64)) == 1
+    finally:
+        quest.destroyQureg(q, env)
