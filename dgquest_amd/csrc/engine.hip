@@ -1036,160 +1036,190 @@ compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB
 // ----------------------------------------------------------------------------
 // dense sweeps: FP32 tile in LDS, dense 2^k x 2^k complex blocks on MFMA
 // ----------------------------------------------------------------------------
-// A dense op on k tile bits is one real GEMM per tile:
-//   [Re y; Im y] = [[Ur, -Ui], [Ui, Ur]] [Re x; Im x],
-// rows and the contraction index both of size M = 2^(k+1), one column per
-// assignment of the other T - k tile bits (NC = 2^(T-k) columns).
-// v_mfma_f32_32x32x2f32: lane l supplies A[l % 32][l / 32] and
-// B[l / 32][l % 32]; result register v of lane l is
-// C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].  The host lays every real
-// matrix out so that a lane's A operands of four consecutive MFMAs (p = 4q ..
-// 4q + 3 over the contraction pairs) are 16 contiguous bytes:
-//   mat[((rb * M/8 + q) * 64 + l) * 4 + i] = A[32 rb + l % 32][2 (4q + i) + l / 32].
+// A dense op on k tile bits is one complex GEMM per tile, rows and the contraction
+// index of size K = 2^k, one column per assignment of the other T - k tile bits
+// (NC = 2^(T-k) columns): Yr = Ur Xr - Ui Xi, Yi = Ui Xr + Ur Xi.
+//
+// Each FP32 factor is the sum of three bf16 numbers (8 significant bits each, 24 in
+// all: the split of an FP32 amplitude is exact), and a real product is the six
+// piece products of order up to 2^-16, on v_mfma_f32_32x32x16_bf16 with FP32
+// sums: 16 times the rate of v_mfma_f32_32x32x2f32, so 2.7 times for a product.
+// The leading products have accumulators of their own (their sums take 2 K / 16
+// roundings instead of 2 K), the other five share the second ones.  What is left out is at most
+// 3 * 2^-25 of a product's magnitude, less than the rounding of its two FP32 factors.
+// Measured over 15 to 25 qubits, depth 20: error against 64 bits 1.9e-7 .. 3.4e-7 (FP32 MFMA
+// 7.4e-7 .. 1.3e-6); 25 qubits, k = 7, 42 ops in 26 blocks: 13.9 -> 8.5 ms of kernels.
+//
+// v_mfma_f32_32x32x16_bf16: lane l supplies A[l % 32][8 (l / 32) + i] and
+// B[8 (l / 32) + i][l % 32], i = 0..7 in 16 bytes; result register v of lane l is
+// C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].  A matrix is stored as those 16 bytes:
+//   [row block of 32][16 contraction indices][real, imaginary][piece][lane][i].
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 #define DENSE_T_MAX 13
 #define DENSE_THREADS 512
 #define DENSE_COLS 256  // column-table entries per op: 2^(T - k) <= 2^(13 - 5)
 #define DENSE_WAVES (DENSE_THREADS / 64)
 
+// The three bf16 pieces of a matrix entry, rounded to nearest even.
+static __host__ __device__ inline void split_entry(double x, uint16_t *piece) {
+    for (int i = 0; i < 3; i++) {
+        const float f = (float)x;
+        uint32_t u;
+        __builtin_memcpy(&u, &f, 4);
+        u += 0x7fffu + ((u >> 16) & 1u);
+        piece[i] = (uint16_t)(u >> 16);
+        u &= 0xffff0000u;
+        float h;
+        __builtin_memcpy(&h, &u, 4);
+        x -= (double)h;
+    }
+}
+
+// Position of entry (r, c) of a 2^k x 2^k matrix, part 0 / 1 (real / imaginary), in
+// 16-bit words; the pieces follow 512 words apart.
+static __host__ __device__ inline size_t entry_pos(int k, uint32_t r, uint32_t c, uint32_t part) {
+    const uint32_t lane = (r & 31u) | (((c >> 3) & 1u) << 5);
+    return ((((size_t)(r >> 5) << (k - 4)) + (c >> 4)) * 6 + part * 3) * 512 + lane * 8 + (c & 7u);
+}
+
+// Two FP32 amplitude parts as pairs of bf16 pieces: hi + mid + lo is x exactly.
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    auto round2 = [](float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2){a, b}, bf2)); };
+    hi = round2(x0, x1);
+    x0 -= __uint_as_float(hi << 16);
+    x1 -= __uint_as_float(hi & 0xffff0000u);
+    mid = round2(x0, x1);
+    x0 -= __uint_as_float(mid << 16);
+    x1 -= __uint_as_float(mid & 0xffff0000u);
+    lo = round2(x0, x1);
+}
+
 // LDS slot of tile element e: the low 5 bits are xored with bits 5..9 and
 // 10..14, spreading power-of-two strides over the 32 banks (a bijection:
 // only the low bits change, by a function of the others).
 __device__ __forceinline__ uint32_t dswz(uint32_t e) { return e ^ ((e >> 5) & 31u) ^ ((e >> 10) & 31u); }
 
-// One dense op on the tile in LDS.  Work item = CB chunks of 32 columns x RB
-// row blocks of 32 rows (RB x CB = 2 result tiles); one item per wave at
-// T = 13.  k = 5 takes RB = 2, CB = 1: an item holds all 2^(k+1) rows of its
-// columns.  Wider ops take RB = 1, CB = 2 where the tile has two chunks: each
-// A operand (the matrix, from L2) then feeds two MFMAs, which halves the
-// matrix traffic per MFMA (for k = 7 every workgroup reads 256 KiB of matrix
-// per op).  coloff[c] is column c's tile offset (c's bits placed on the tile
-// bits outside the op), a table the host forms per op.  The B rows of the
-// op's bits 1..k-1 step with the submask increment x' = ((x | ~S) + 1) & S
-// (op bits ascending); the LDS swizzle is linear, so a B address is the
-// lane's column part xor the swizzle of x, a scalar.
-template <int KL, int CB>
-__device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restrict__ im, uint32_t T,
-                                         const dq_dense_op &op, const float *__restrict__ mat,
-                                         const uint32_t *__restrict__ coloff, uint32_t tid) {
-    constexpr int K = 1 << KL, M = 2 * K, MB = M / 32;
-    constexpr int RB = CB == 2 ? 1 : (MB < 2 ? MB : 2);  // row blocks per work item
-    constexpr int NA = RB * CB;                           // result tiles per work item
-    constexpr int NQ = K / 4;                             // groups of four contraction pairs (both halves)
-    const uint32_t NC = 1u << (T - KL);
-    const uint32_t NCG = NC / (32 * CB);                  // column groups
-    const uint32_t items = NCG * (MB / RB);
-    const uint32_t w = tid >> 6, lane = tid & 63;
-    uint32_t used = 0;
-    for (int j = 0; j < KL; j++) used |= 1u << op.bits[j];
-    const uint32_t b0 = 1u << op.bits[0];
-    const uint32_t S = used & ~b0;  // tile bits of matrix-index bits 1..k-1
-    __syncthreads();  // the previous op's writes (or the tile load) are done
-    v16f acc[NA];
+// One dense op on the tile in LDS.  First every wave splits its share of the tile
+// into B operands (`frag`: 64 lanes x 16 bytes of one piece, [column block of 32]
+// [16 contraction indices][real, imaginary][piece]), once per op: a wave that split
+// the columns it multiplies would repeat the work of every other row block.
+// Then a wave multiplies one row block by one column block, 24 MFMAs for 6 + 6
+// operands loaded, A (from L2) and B (LDS) one step of 16 ahead; at T = 13 every
+// k gives exactly 8 such items.  coloff[c] is column c's tile offset (c's bits
+// placed on the tile bits outside the op), a table the host forms per op.  Deposit
+// and swizzle are linear over GF(2), so an LDS slot is the xor of the column's
+// and of sd[b] = dswz(1 << bits[b]) over the set bits b of the matrix index.
+template <int KL>
+__device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restrict__ im, uint4 *__restrict__ frag, uint32_t T,
+                                         const dq_dense_op &op, const uint4 *__restrict__ mat,
+                                         const uint32_t *__restrict__ coloff, uint32_t lane, uint32_t w) {
+    constexpr uint32_t K = 1u << KL, KS = K / 16, RB = K / 32;
+    const uint32_t NCB = 1u << (T - KL - 5);
+    const uint32_t nf = NCB * KS * 2;  // operands of the tile, at most 4 a wave
+    uint32_t sd[KL];
 #pragma unroll
-    for (int a = 0; a < NA; a++)
-        for (int v = 0; v < 16; v++) acc[a][v] = 0.0f;
-    const uint32_t item = w;
-    const bool busy = item < items;  // uniform over the wave
-    const uint32_t cg = item % NCG, rg = item / NCG;
-    if (busy) {
-        uint32_t lz[CB];
+    for (int b = 0; b < KL; b++) sd[b] = dswz(1u << op.bits[b]);
+    const uint32_t cb = w & (NCB - 1), rb = w >> (T - KL - 5);
+    const bool busy = rb < RB;  // uniform over the wave
+    uint4 a[2][6], x[2][6];
+    const uint4 *__restrict__ ma = mat + (size_t)(busy ? rb : 0) * KS * 6 * 64 + lane;
 #pragma unroll
-        for (int c = 0; c < CB; c++)
-            lz[c] = dswz(coloff[(cg * CB + c) * 32 + (lane & 31u)] | ((lane >> 5) ? b0 : 0u));
-        const float4 *__restrict__ ma = reinterpret_cast<const float4 *>(mat) + (size_t)(rg * RB) * NQ * 64 + lane;
-        // A operands load two groups ahead of their MFMAs into a four-slot
-        // ring, B operands (LDS) one group ahead into a two-slot ring: with the
-        // loop unrolled by 4 every slot is a fixed register set (no copies
-        // that would wait for the loads), and a scheduling barrier keeps each
-        // group's loads ahead of its MFMAs.
-        float4 ab[4][RB];
-        float bb[2][CB][4];
-        uint32_t x = 0;
-        // B rows of group q for every chunk: four steps of x over the real
-        // half (q < NQ/2), then again from 0 over the imaginary half
-        auto read_b = [&](int q, float (*b)[4]) {
-            if (q == NQ / 2) x = 0;
-            const float *__restrict__ src = q < NQ / 2 ? re : im;
+    for (int i = 0; i < 6; i++) a[0][i] = ma[i * 64];
+    __syncthreads();  // the tile is complete, the last op's operands have been read
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t sx = dswz(x);
+    for (uint32_t j = 0; j < 4; j++) {
+        const uint32_t f = j * DENSE_WAVES + w;
+        if (f >= nf) break;
+        const uint32_t ks = (f >> 1) & (KS - 1), c = (f >> 1) / KS;
+        uint32_t z = dswz(coloff[c * 32 + (lane & 31u)]) ^ ((lane >> 5) ? sd[3] : 0u);
 #pragma unroll
-                for (int c = 0; c < CB; c++) b[c][i] = src[sx ^ lz[c]];
-                x = ((x | ~S) + 1u) & S;
-            }
-        };
+        for (int b = 4; b < KL; b++) z ^= ((ks >> (b - 4)) & 1u) ? sd[b] : 0u;
+        const float *__restrict__ src = (f & 1u) ? im : re;
+        float v[8];
 #pragma unroll
-        for (int r = 0; r < RB; r++) {
-            ab[0][r] = ma[(size_t)r * NQ * 64];
-            ab[1][r] = ma[((size_t)r * NQ + 1) * 64];  // NQ >= 8
+        for (int i = 0; i < 8; i++) v[i] = src[z ^ ((i & 1) ? sd[0] : 0u) ^ ((i & 2) ? sd[1] : 0u) ^ ((i & 4) ? sd[2] : 0u)];
+        uint4 h, m, l;
+        split_pair(v[0], v[1], h.x, m.x, l.x);
+        split_pair(v[2], v[3], h.y, m.y, l.y);
+        split_pair(v[4], v[5], h.z, m.z, l.z);
+        split_pair(v[6], v[7], h.w, m.w, l.w);
+        uint4 *__restrict__ d = frag + f * 192 + lane;
+        d[0] = h;
+        d[64] = m;
+        d[128] = l;
+    }
+    __syncthreads();
+    if (!busy) return;
+    v16f yr, yi, cr, ci;  // leading products, the others
+#pragma unroll
+    for (int v = 0; v < 16; v++) yr[v] = yi[v] = cr[v] = ci[v] = 0.0f;
+    const uint4 *__restrict__ mb = frag + cb * KS * 2 * 192 + lane;
+#pragma unroll
+    for (int i = 0; i < 6; i++) x[0][i] = mb[i * 64];
+    auto mma = [](const uint4 &p, const uint4 &q, const v16f &acc) {
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, p), __builtin_bit_cast(v8bf, q), acc, 0, 0, 0);
+    };
+#pragma unroll
+    for (uint32_t s = 0; s < KS; s++) {
+        if (s + 1 < KS) {
+#pragma unroll
+            for (int i = 0; i < 6; i++) a[(s + 1) & 1][i] = ma[((s + 1) * 6 + i) * 64];
+#pragma unroll
+            for (int i = 0; i < 6; i++) x[(s + 1) & 1][i] = mb[((s + 1) * 6 + i) * 64];
         }
-        read_b(0, bb[0]);
-#pragma unroll 4
-        for (int q = 0; q < NQ; q++) {
-            if (q + 2 < NQ) {
+        __builtin_amdgcn_sched_barrier(0);  // the next step's loads stay ahead of the products
+        const uint4 *ur = a[s & 1], *ui = ur + 3, *xr = x[s & 1], *xi = xr + 3;
+        uint4 un[3];
 #pragma unroll
-                for (int r = 0; r < RB; r++) ab[(q + 2) & 3][r] = ma[((size_t)r * NQ + q + 2) * 64];
-            }
-            if (q + 1 < NQ) read_b(q + 1, bb[(q + 1) & 1]);
-            __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < 3; i++)
+            un[i] = make_uint4(ui[i].x ^ 0x80008000u, ui[i].y ^ 0x80008000u, ui[i].z ^ 0x80008000u, ui[i].w ^ 0x80008000u);
+        yr = mma(ur[0], xr[0], yr);
+        yi = mma(ui[0], xr[0], yi);
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+        for (int t = 0; t < 5; t++) {  // pieces (p, q) of matrix and amplitude with p + q = 2, then 1
+            const int p = t < 3 ? t : t - 3, q = (t < 3 ? 2 : 1) - p;
+            cr = mma(ur[p], xr[q], cr);
+            ci = mma(ui[p], xr[q], ci);
+        }
+        yr = mma(un[0], xi[0], yr);
+        yi = mma(ur[0], xi[0], yi);
 #pragma unroll
-                for (int r = 0; r < RB; r++)
-#pragma unroll
-                    for (int c = 0; c < CB; c++)
-                        acc[r * CB + c] =
-                            __builtin_amdgcn_mfma_f32_32x32x2f32(ab[q & 3][r][i], bb[q & 1][c][i], acc[r * CB + c], 0, 0, 0);
+        for (int t = 0; t < 5; t++) {
+            const int p = t < 3 ? t : t - 3, q = (t < 3 ? 2 : 1) - p;
+            cr = mma(un[p], xi[q], cr);
+            ci = mma(ur[p], xi[q], ci);
         }
     }
-    // Write in place once every wave has read what it overwrites.  With
-    // RB = MB (k = 5) a work item holds all rows of its columns, so a wave
-    // reads exactly the tile elements it writes and program order suffices;
-    // otherwise a column's rows are split over several waves.
-    if constexpr (MB > RB) __syncthreads();
-    if (busy) {
-        // Result register v of this lane is row 32 rb + 8 (v / 4) + 4 (lane / 32)
-        // + v % 4 (rb = rg RB + r); rows below K are real parts.  Its tile element
-        // is the row's bits deposited on the op's bits, or the column's bits;
-        // deposit and swizzle are linear over GF(2), so the LDS slot is the xor of
-        // sd[b] = dswz(1 << bits[b]) over the row's set bits b, xor a lane part.
-        uint32_t sd[KL];
+    // Register v of this lane is row 32 rb + 8 (v / 4) + 4 (lane / 32) + v % 4.
+    // Nothing reads the tile until the next barrier.
+    uint32_t z = dswz(coloff[cb * 32 + (lane & 31u)]) ^ ((lane >> 5) ? sd[2] : 0u);
 #pragma unroll
-        for (int b = 0; b < KL; b++) sd[b] = dswz(1u << op.bits[b]);
+    for (int b = 5; b < KL; b++) z ^= ((rb >> (b - 5)) & 1u) ? sd[b] : 0u;
 #pragma unroll
-        for (int c = 0; c < CB; c++) {
-            const uint32_t lp = dswz(coloff[(cg * CB + c) * 32 + (lane & 31u)]) ^ ((lane >> 5) ? sd[2] : 0u);
-#pragma unroll
-            for (int r = 0; r < RB; r++) {
-                const uint32_t r0 = (rg * RB + r) * 32;  // the row block's first row (bits 5 and up)
-                uint32_t ur = 0;
-#pragma unroll
-                for (int b = 5; b < KL; b++) ur ^= ((r0 >> b) & 1u) ? sd[b] : 0u;
-                float *__restrict__ dst = (r0 >> KL) ? im : re;
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const uint32_t u = ur ^ ((v & 1) ? sd[0] : 0u) ^ ((v & 2) ? sd[1] : 0u) ^ ((v & 4) ? sd[3] : 0u) ^
-                                       ((v & 8) ? sd[4] : 0u);
-                    dst[u ^ lp] = acc[r * CB + c][v];
-                }
-            }
-        }
+    for (int v = 0; v < 16; v++) {
+        const uint32_t u = z ^ ((v & 1) ? sd[0] : 0u) ^ ((v & 2) ? sd[1] : 0u) ^ ((v & 4) ? sd[3] : 0u) ^ ((v & 8) ? sd[4] : 0u);
+        re[u] = yr[v] + cr[v];
+        im[u] = yi[v] + ci[v];
     }
 }
 
-// One dense block over every tile of an FP32 state: grid = tiles, 512 threads;
-// at most 128 VGPRs so that two workgroups (64 KiB of LDS each) share a CU.
+// One dense block over every tile of an FP32 state: grid = tiles, 512 threads; the
+// tile (64 KiB at T = 13) and its operands (96 KiB) fill a CU's LDS, so a SIMD has two
+// waves and up to 256 VGPRs each.
 template <int KL>
-__global__ void __launch_bounds__(DENSE_THREADS, 4)
-dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restrict__ ops, const float *__restrict__ mats,
+__global__ void __launch_bounds__(DENSE_THREADS, 2)
+dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restrict__ ops, const uint4 *__restrict__ mats,
              const uint32_t *__restrict__ ctab, typename V2<float>::type *__restrict__ st) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const uint32_t T = blk->tile_bits;
     const uint32_t NT = 1u << T;
     float *re = reinterpret_cast<float *>(lds_raw);
     float *im = re + NT;
+    uint4 *frag = reinterpret_cast<uint4 *>(im + NT);
     const uint32_t tid = threadIdx.x;
     const uint64_t base = tile_base(blk->nontile_mask, blockIdx.x);
     // tile_q read as four words (scalar loads; byte loads would put these
@@ -1235,16 +1265,10 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
             im[z] = v[i].y;
         }
     }
-    const size_t msz = (size_t)(2u << KL) * (2u << KL);
-    // ops wider than 5 bits pair two column chunks per work item when the
-    // tile has them (T >= k + 6; T is uniform over the launch)
-    const bool pair = KL >= 6 && T >= (uint32_t)KL + 6;
+    constexpr size_t msz = (size_t)12 << (2 * KL);  // bytes of a matrix
     for (uint32_t o = 0; o < blk->op_count; o++) {
         const dq_dense_op op = ops[blk->op_begin + o];
-        const float *m = mats + op.mat * msz;
-        const uint32_t *ct = ctab + (size_t)(blk->op_begin + o) * DENSE_COLS;
-        if (pair) dense_op<KL, 2>(re, im, T, op, m, ct, tid);
-        else dense_op<KL, 1>(re, im, T, op, m, ct, tid);
+        dense_op<KL>(re, im, frag, T, op, mats + op.mat * (msz / 16), ctab + (size_t)(blk->op_begin + o) * DENSE_COLS, lane, wv);
     }
     __syncthreads();
     {
@@ -1274,8 +1298,7 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
 // 28.7-31.8 ms of a flush and were uploaded (11 MB); the flush now takes 14.7 ms.
 template <int KL>
 __global__ void __launch_bounds__(256)
-dense_form(const dq_small_gate *__restrict__ gates, const uint32_t *__restrict__ begin, float *__restrict__ mats) {
-    constexpr int K = 1 << KL, M = 2 * K;
+dense_form(const dq_small_gate *__restrict__ gates, const uint32_t *__restrict__ begin, uint16_t *__restrict__ mats) {
     constexpr int J = KL == 7 ? 2 : 1;      // amplitudes per lane
     constexpr int CW = KL == 5 ? 2 : 1;     // columns per wave
     constexpr uint32_t LN = 64 / CW;        // lanes per column
@@ -1329,19 +1352,19 @@ dense_form(const dq_small_gate *__restrict__ gates, const uint32_t *__restrict__
             }
         }
     }
-    float *__restrict__ D = mats + (size_t)blockIdx.y * ((size_t)M * M);
-    auto put = [&](uint32_t row, uint32_t col, float v) {  // real matrix element (row, col)
-        const uint32_t rb = row >> 5, l = (row & 31u) | ((col & 1u) << 5), p = col >> 1;
-        D[(((size_t)rb * (M / 8) + p / 4) * 64 + l) * 4 + p % 4] = v;
+    uint16_t *__restrict__ D = mats + (size_t)blockIdx.y * ((size_t)6 << (2 * KL));
+    auto put = [&](uint32_t r, uint32_t part, double v) {
+        uint16_t piece[3];
+        split_entry(v, piece);
+        uint16_t *__restrict__ d = D + entry_pos(KL, r, c, part);
+        d[0] = piece[0];
+        d[512] = piece[1];
+        d[1024] = piece[2];
     };
 #pragma unroll
     for (int j = 0; j < J; j++) {
-        const uint32_t r = i0 + LN * j;
-        const float a = (float)re[j], b = (float)im[j];
-        put(r, c, a);
-        put(r, K + c, -b);
-        put(K + r, c, b);
-        put(K + r, K + c, a);
+        put(i0 + LN * j, 0, re[j]);
+        put(i0 + LN * j, 1, im[j]);
     }
 }
 
@@ -1829,9 +1852,9 @@ extern "C" int dq_device_init(int device) {
         }
         HIPC(hipFuncSetAttribute((const void *)small_kernel<double>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
         HIPC(hipFuncSetAttribute((const void *)small_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
-        HIPC(hipFuncSetAttribute((const void *)dense_kernel<5>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
-        HIPC(hipFuncSetAttribute((const void *)dense_kernel<6>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
-        HIPC(hipFuncSetAttribute((const void *)dense_kernel<7>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+        HIPC(hipFuncSetAttribute((const void *)dense_kernel<5>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+        HIPC(hipFuncSetAttribute((const void *)dense_kernel<6>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+        HIPC(hipFuncSetAttribute((const void *)dense_kernel<7>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
         g_device = device;
     }
     return DQ_OK;
@@ -3195,14 +3218,14 @@ extern "C" int dq_compare_states(const void *a, int prec_a, const void *b, int p
 
 // ---- dense sweeps -------------------------------------------------------------
 namespace {
-size_t dense_mat_floats(int k) { return (size_t)(2u << k) * (2u << k); }
-size_t dense_lds_bytes(uint32_t T) { return 2 * ((size_t)4 << T); }
+size_t dense_mat_bytes(int k) { return (size_t)12 << (2 * k); }  // three pieces of two parts
+size_t dense_lds_bytes(uint32_t T) { return (size_t)20 << T; }   // the tile, its operands
 }  // namespace
 
 extern "C" size_t dq_dense_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats) {
     if (k < 5 || k > 7) return 0;
     return align_up(n_blocks * sizeof(dq_dense_block), 256) + align_up(n_ops * sizeof(dq_dense_op), 256) +
-           align_up((size_t)n_mats * dense_mat_floats(k) * sizeof(float), 256) +
+           align_up((size_t)n_mats * dense_mat_bytes(k), 256) +
            align_up((size_t)n_ops * DENSE_COLS * sizeof(uint32_t), 256);
 }
 
@@ -3260,7 +3283,7 @@ static int dense_columns(int k, const dq_dense_block *blocks, uint32_t n_blocks,
 }
 
 static int dense_launch(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_block *d_blocks,
-                        const dq_dense_op *d_ops, const float *d_mats, const uint32_t *d_ct, void *state, hipStream_t s) {
+                        const dq_dense_op *d_ops, const uint4 *d_mats, const uint32_t *d_ct, void *state, hipStream_t s) {
     auto *st = (typename V2<float>::type *)state;
     for (uint32_t i = 0; i < n_blocks; i++) {
         const dq_dense_block &b = blocks[i];
@@ -3284,28 +3307,23 @@ extern "C" int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_bl
     if (ws_bytes < need) return fail(DQ_ERR_ARG, "dq_apply_dense: workspace %zu < %zu bytes", ws_bytes, need);
     int rc = validate_dense(k, blocks, n_blocks, ops, n_ops, n_mats);
     if (rc) return rc;
-    // upload: blocks | ops | real matrices in MFMA operand order | column tables
+    // upload: blocks | ops | matrices in MFMA operand order | column tables
     const size_t ob = align_up(n_blocks * sizeof(dq_dense_block), 256);
     const size_t mo = ob + align_up(n_ops * sizeof(dq_dense_op), 256);
-    const int K = 1 << k, M = 2 * K;
-    const size_t co = mo + align_up((size_t)n_mats * dense_mat_floats(k) * sizeof(float), 256);
+    const uint32_t K = 1u << k;
+    const size_t co = mo + align_up((size_t)n_mats * dense_mat_bytes(k), 256);
     std::vector<unsigned char> buf(co + (size_t)n_ops * DENSE_COLS * sizeof(uint32_t), 0);
     memcpy(buf.data(), blocks, n_blocks * sizeof(dq_dense_block));
     if (n_ops) memcpy(buf.data() + ob, ops, n_ops * sizeof(dq_dense_op));
-    float *dst = reinterpret_cast<float *>(buf.data() + mo);
     for (uint32_t mi = 0; mi < n_mats; mi++) {
-        const double *U = mats + (size_t)mi * K * K * 2;
-        float *D = dst + (size_t)mi * dense_mat_floats(k);
-        for (int rb = 0; rb < M / 32; rb++)
-            for (int p = 0; p < M / 2; p++)
-                for (int l = 0; l < 64; l++) {
-                    const int r = rb * 32 + (l & 31), c = 2 * p + (l >> 5);
-                    const int ur = r & (K - 1), uc = c & (K - 1);
-                    const double Ure = U[2 * ((size_t)ur * K + uc)], Uim = U[2 * ((size_t)ur * K + uc) + 1];
-                    double a;
-                    if (r < K) a = c < K ? Ure : -Uim;
-                    else a = c < K ? Uim : Ure;
-                    D[(((size_t)rb * (M / 8) + p / 4) * 64 + l) * 4 + p % 4] = (float)a;
+        const double *U = mats + ((size_t)mi << (2 * k)) * 2;
+        uint16_t *D = reinterpret_cast<uint16_t *>(buf.data() + mo + mi * dense_mat_bytes(k));
+        for (uint32_t r = 0; r < K; r++)
+            for (uint32_t c = 0; c < K; c++)
+                for (uint32_t part = 0; part < 2; part++) {
+                    uint16_t piece[3];
+                    split_entry(U[2 * ((size_t)r * K + c) + part], piece);
+                    for (int i = 0; i < 3; i++) D[entry_pos(k, r, c, part) + 512 * i] = piece[i];
                 }
     }
     rc = dense_columns(k, blocks, n_blocks, ops, n_ops, reinterpret_cast<uint32_t *>(buf.data() + co));
@@ -3313,7 +3331,7 @@ extern "C" int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_bl
     rc = stage_upload(d_ws, buf, stream);
     if (rc) return rc;
     unsigned char *d = (unsigned char *)d_ws;
-    return dense_launch(k, blocks, n_blocks, (const dq_dense_block *)d, (const dq_dense_op *)(d + ob), (const float *)(d + mo),
+    return dense_launch(k, blocks, n_blocks, (const dq_dense_block *)d, (const dq_dense_op *)(d + ob), (const uint4 *)(d + mo),
                         (const uint32_t *)(d + co), state, (hipStream_t)stream);
 }
 
@@ -3331,7 +3349,7 @@ DenseGatesWs dense_gates_ws(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n
     w.begin = w.gates + align_up((size_t)n_gates * sizeof(dq_small_gate), 256);
     w.upload = w.begin + ((size_t)n_mats + 1) * sizeof(uint32_t);
     w.mats = align_up(w.upload, 256);
-    w.total = w.mats + (size_t)n_mats * dense_mat_floats(k) * sizeof(float);
+    w.total = w.mats + (size_t)n_mats * dense_mat_bytes(k);
     return w;
 }
 }  // namespace
@@ -3373,17 +3391,17 @@ extern "C" int dq_apply_dense_gates(int k, const dq_dense_block *blocks, uint32_
     hipStream_t s = (hipStream_t)stream;
     const auto *d_gates = (const dq_small_gate *)(d + w.gates);
     const auto *d_begin = (const uint32_t *)(d + w.begin);
-    float *d_mats = (float *)(d + w.mats);
+    unsigned char *d_mats = d + w.mats;
     for (uint32_t m0 = 0; m0 < n_mats; m0 += 65535u) {
         const uint32_t nm = std::min(n_mats - m0, 65535u);
         const uint32_t *gb = d_begin + m0;
-        float *dm = d_mats + (size_t)m0 * dense_mat_floats(k);
+        uint16_t *dm = (uint16_t *)(d_mats + (size_t)m0 * dense_mat_bytes(k));
         if (k == 5) hipLaunchKernelGGL(dense_form<5>, dim3(4, nm), dim3(256), 0, s, d_gates, gb, dm);
         else if (k == 6) hipLaunchKernelGGL(dense_form<6>, dim3(16, nm), dim3(256), 0, s, d_gates, gb, dm);
         else hipLaunchKernelGGL(dense_form<7>, dim3(32, nm), dim3(256), 0, s, d_gates, gb, dm);
         HIPC(hipGetLastError());
     }
-    return dense_launch(k, blocks, n_blocks, (const dq_dense_block *)d, (const dq_dense_op *)(d + w.ops), d_mats,
+    return dense_launch(k, blocks, n_blocks, (const dq_dense_block *)d, (const dq_dense_op *)(d + w.ops), (const uint4 *)d_mats,
                         (const uint32_t *)(d + w.cols), state, s);
 }
 
