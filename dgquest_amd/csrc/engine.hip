@@ -1048,7 +1048,10 @@ compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB
 // roundings instead of 2 K), the other five share the second ones.  What is left out is at most
 // 3 * 2^-25 of a product's magnitude, less than the rounding of its two FP32 factors.
 // Measured over 15 to 25 qubits, depth 20: error against 64 bits 1.9e-7 .. 3.4e-7 (FP32 MFMA
-// 7.4e-7 .. 1.3e-6); 25 qubits, k = 7, 42 ops in 26 blocks: 13.9 -> 8.5 ms of kernels.
+// 7.4e-7 .. 1.3e-6).  25 qubits, depth 20, kernels of a flush with FP32 MFMA -> now: k = 7
+// (42 ops in 26 blocks) 13.9 -> 8.5 ms, k = 6 and 5 6.5 and 4.8 ms.  An op of k = 7 runs
+// at 1.1-1.3 PFLOP/s of bf16, what a large library product reaches (1.36): clocks
+// fall as the run goes on, so vector instructions beside the products cost time too.
 //
 // v_mfma_f32_32x32x16_bf16: lane l supplies A[l % 32][8 (l / 32) + i] and
 // B[8 (l / 32) + i][l % 32], i = 0..7 in 16 bytes; result register v of lane l is
@@ -1058,7 +1061,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 #define DENSE_T_MAX 13
-#define DENSE_THREADS 512
+#define DENSE_THREADS 256
 #define DENSE_COLS 256  // column-table entries per op: 2^(T - k) <= 2^(13 - 5)
 #define DENSE_WAVES (DENSE_THREADS / 64)
 
@@ -1103,113 +1106,134 @@ __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t &hi, uin
 // only the low bits change, by a function of the others).
 __device__ __forceinline__ uint32_t dswz(uint32_t e) { return e ^ ((e >> 5) & 31u) ^ ((e >> 10) & 31u); }
 
-// One dense op on the tile in LDS.  First every wave splits its share of the tile
-// into B operands (`frag`: 64 lanes x 16 bytes of one piece, [column block of 32]
-// [16 contraction indices][real, imaginary][piece]), once per op: a wave that split
-// the columns it multiplies would repeat the work of every other row block.
-// Then a wave multiplies one row block by one column block, 24 MFMAs for 6 + 6
-// operands loaded, A (from L2) and B (LDS) one step of 16 ahead; at T = 13 every
-// k gives exactly 8 such items.  coloff[c] is column c's tile offset (c's bits
-// placed on the tile bits outside the op), a table the host forms per op.  Deposit
-// and swizzle are linear over GF(2), so an LDS slot is the xor of the column's
-// and of sd[b] = dswz(1 << bits[b]) over the set bits b of the matrix index.
+// One dense op on the tile in LDS.  A work item is RP row blocks of 32 rows by one
+// block of 32 columns; at T = 13 every wave has one (k = 5: two).  Per step of 16
+// contraction indices a wave reads 16 amplitude parts a lane from the tile, splits them
+// and issues 24 MFMAs for each row block.  Waves that share columns (k = 7: two) split them
+// each: the vector instructions run while the matrix unit is busy, and operands
+// split once into LDS (96 KiB beside the tile) left room for one workgroup per CU, whose
+// loads, stores, splits and products then took turns (k = 5 7.0 ms, k = 6 7.5, k = 7 the
+// same).  Matrix operands (L2) come two
+// units of 24 MFMAs ahead, amplitudes one step.  coloff[c] is column c's tile offset
+// (c's bits placed on the tile bits outside the op), a table the host forms per op.
+// Deposit and swizzle are linear over GF(2), so an LDS slot is the xor of the column's and
+// of sd[b] = dswz(1 << bits[b]) over the set bits b of the matrix index.
 template <int KL>
-__device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restrict__ im, uint4 *__restrict__ frag, uint32_t T,
-                                         const dq_dense_op &op, const uint4 *__restrict__ mat,
-                                         const uint32_t *__restrict__ coloff, uint32_t lane, uint32_t w) {
-    constexpr uint32_t K = 1u << KL, KS = K / 16, RB = K / 32;
-    const uint32_t NCB = 1u << (T - KL - 5);
-    const uint32_t nf = NCB * KS * 2;  // operands of the tile, at most 4 a wave
+__device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restrict__ im, uint32_t T, const dq_dense_op &op,
+                                         const uint4 *__restrict__ mat, const uint32_t *__restrict__ coloff, uint32_t lane,
+                                         uint32_t w) {
+    constexpr uint32_t K = 1u << KL, KS = K / 16, RB = K / 32, RP = RB >= 2 ? 2 : 1;
+    const uint32_t lc = T - KL - 5, NCB = 1u << lc, items = NCB * (RB / RP);
     uint32_t sd[KL];
 #pragma unroll
     for (int b = 0; b < KL; b++) sd[b] = dswz(1u << op.bits[b]);
-    const uint32_t cb = w & (NCB - 1), rb = w >> (T - KL - 5);
-    const bool busy = rb < RB;  // uniform over the wave
-    uint4 a[2][6], x[2][6];
-    const uint4 *__restrict__ ma = mat + (size_t)(busy ? rb : 0) * KS * 6 * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < 6; i++) a[0][i] = ma[i * 64];
-    __syncthreads();  // the tile is complete, the last op's operands have been read
-#pragma unroll
-    for (uint32_t j = 0; j < 4; j++) {
-        const uint32_t f = j * DENSE_WAVES + w;
-        if (f >= nf) break;
-        const uint32_t ks = (f >> 1) & (KS - 1), c = (f >> 1) / KS;
-        uint32_t z = dswz(coloff[c * 32 + (lane & 31u)]) ^ ((lane >> 5) ? sd[3] : 0u);
-#pragma unroll
-        for (int b = 4; b < KL; b++) z ^= ((ks >> (b - 4)) & 1u) ? sd[b] : 0u;
-        const float *__restrict__ src = (f & 1u) ? im : re;
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = src[z ^ ((i & 1) ? sd[0] : 0u) ^ ((i & 2) ? sd[1] : 0u) ^ ((i & 4) ? sd[2] : 0u)];
-        uint4 h, m, l;
-        split_pair(v[0], v[1], h.x, m.x, l.x);
-        split_pair(v[2], v[3], h.y, m.y, l.y);
-        split_pair(v[4], v[5], h.z, m.z, l.z);
-        split_pair(v[6], v[7], h.w, m.w, l.w);
-        uint4 *__restrict__ d = frag + f * 192 + lane;
-        d[0] = h;
-        d[64] = m;
-        d[128] = l;
-    }
-    __syncthreads();
-    if (!busy) return;
-    v16f yr, yi, cr, ci;  // leading products, the others
-#pragma unroll
-    for (int v = 0; v < 16; v++) yr[v] = yi[v] = cr[v] = ci[v] = 0.0f;
-    const uint4 *__restrict__ mb = frag + cb * KS * 2 * 192 + lane;
-#pragma unroll
-    for (int i = 0; i < 6; i++) x[0][i] = mb[i * 64];
     auto mma = [](const uint4 &p, const uint4 &q, const v16f &acc) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, p), __builtin_bit_cast(v8bf, q), acc, 0, 0, 0);
     };
+    bool first = true;
+    for (uint32_t item = w; RB > RP ? first : item < items; item += DENSE_WAVES) {
+        const bool busy = item < items;  // uniform over the wave
+        const uint32_t cb = item & (NCB - 1), rb = busy ? (item >> lc) * RP : 0;
+        const uint4 *__restrict__ ma = mat + (size_t)rb * KS * 6 * 64 + lane;
+        uint4 a[2][6];
+        auto load_a = [&](uint4 *to, uint32_t s, uint32_t r) {
 #pragma unroll
-    for (uint32_t s = 0; s < KS; s++) {
-        if (s + 1 < KS) {
+            for (int i = 0; i < 6; i++) to[i] = ma[((r * KS + s) * 6 + i) * 64];
+        };
+        load_a(a[0], 0, 0);
+        load_a(a[1], RP == 2 ? 0 : 1, RP == 2 ? 1 : 0);
+        const uint32_t zc = dswz(coloff[cb * 32 + (lane & 31u)]);
+        if (first) __syncthreads();  // the tile is complete
+        first = false;
+        v16f acc[RP][4];  // real, imaginary: the leading products, the others
+        if (busy) {
 #pragma unroll
-            for (int i = 0; i < 6; i++) a[(s + 1) & 1][i] = ma[((s + 1) * 6 + i) * 64];
+            for (uint32_t r = 0; r < RP; r++)
 #pragma unroll
-            for (int i = 0; i < 6; i++) x[(s + 1) & 1][i] = mb[((s + 1) * 6 + i) * 64];
+                for (int c = 0; c < 4; c++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) acc[r][c][v] = 0.0f;
+            const uint32_t zl = zc ^ ((lane >> 5) ? sd[3] : 0u);
+            float xr[8], xi[8];
+            auto read_x = [&](uint32_t s) {
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    uint32_t u = ((i & 1) ? sd[0] : 0u) ^ ((i & 2) ? sd[1] : 0u) ^ ((i & 4) ? sd[2] : 0u);
+#pragma unroll
+                    for (int b = 4; b < KL; b++) u ^= ((s >> (b - 4)) & 1u) ? sd[b] : 0u;
+                    xr[i] = re[zl ^ u];
+                    xi[i] = im[zl ^ u];
+                }
+            };
+            read_x(0);
+            // with two row blocks a unit's slot is its row block, also in a real loop
+            constexpr int UF = RP == 2 ? 1 : KS;
+#pragma unroll UF
+            for (uint32_t s = 0; s < KS; s++) {
+                uint4 br[3], bi[3];
+                split_pair(xr[0], xr[1], br[0].x, br[1].x, br[2].x);
+                split_pair(xr[2], xr[3], br[0].y, br[1].y, br[2].y);
+                split_pair(xr[4], xr[5], br[0].z, br[1].z, br[2].z);
+                split_pair(xr[6], xr[7], br[0].w, br[1].w, br[2].w);
+                split_pair(xi[0], xi[1], bi[0].x, bi[1].x, bi[2].x);
+                split_pair(xi[2], xi[3], bi[0].y, bi[1].y, bi[2].y);
+                split_pair(xi[4], xi[5], bi[0].z, bi[1].z, bi[2].z);
+                split_pair(xi[6], xi[7], bi[0].w, bi[1].w, bi[2].w);
+                if (s + 1 < KS) read_x(s + 1);
+#pragma unroll
+                for (uint32_t r = 0; r < RP; r++) {
+                    __builtin_amdgcn_sched_barrier(0);  // loads stay ahead of the products that cover them
+                    uint4 *slot = a[RP == 2 ? r : (s & 1)];
+                    const uint4 *ur = slot, *ui = ur + 3;
+                    auto neg = [](const uint4 &q) {
+                        return make_uint4(q.x ^ 0x80008000u, q.y ^ 0x80008000u, q.z ^ 0x80008000u, q.w ^ 0x80008000u);
+                    };
+                    v16f &yr = acc[r][0], &yi = acc[r][1], &cr = acc[r][2], &ci = acc[r][3];
+                    yr = mma(ur[0], br[0], yr);
+                    yi = mma(ui[0], br[0], yi);
+#pragma unroll
+                    for (int t = 0; t < 5; t++) {  // pieces (p, q) of matrix and amplitude with p + q = 2, then 1
+                        const int p = t < 3 ? t : t - 3, q = (t < 3 ? 2 : 1) - p;
+                        cr = mma(ur[p], br[q], cr);
+                        ci = mma(ui[p], br[q], ci);
+                    }
+                    const uint4 un[3] = {neg(ui[0]), neg(ui[1]), neg(ui[2])};
+                    yr = mma(un[0], bi[0], yr);
+                    yi = mma(ur[0], bi[0], yi);
+#pragma unroll
+                    for (int t = 0; t < 5; t++) {
+                        const int p = t < 3 ? t : t - 3, q = (t < 3 ? 2 : 1) - p;
+                        cr = mma(un[p], bi[q], cr);
+                        ci = mma(ur[p], bi[q], ci);
+                    }
+                    if (s + 2 / RP < KS) load_a(slot, s + 2 / RP, r);
+                }
+            }
         }
-        __builtin_amdgcn_sched_barrier(0);  // the next step's loads stay ahead of the products
-        const uint4 *ur = a[s & 1], *ui = ur + 3, *xr = x[s & 1], *xi = xr + 3;
-        uint4 un[3];
+        // In place: an item with every row of its columns reads exactly the tile
+        // elements it writes; otherwise every wave has to have read them.
+        if constexpr (RB > RP) __syncthreads();
+        if (!busy) break;
+        // Register v of this lane is row 32 (rb + r) + 8 (v / 4) + 4 (lane / 32) + v % 4.
 #pragma unroll
-        for (int i = 0; i < 3; i++)
-            un[i] = make_uint4(ui[i].x ^ 0x80008000u, ui[i].y ^ 0x80008000u, ui[i].z ^ 0x80008000u, ui[i].w ^ 0x80008000u);
-        yr = mma(ur[0], xr[0], yr);
-        yi = mma(ui[0], xr[0], yi);
+        for (uint32_t r = 0; r < RP; r++) {
+            uint32_t z = zc ^ ((lane >> 5) ? sd[2] : 0u);
 #pragma unroll
-        for (int t = 0; t < 5; t++) {  // pieces (p, q) of matrix and amplitude with p + q = 2, then 1
-            const int p = t < 3 ? t : t - 3, q = (t < 3 ? 2 : 1) - p;
-            cr = mma(ur[p], xr[q], cr);
-            ci = mma(ui[p], xr[q], ci);
-        }
-        yr = mma(un[0], xi[0], yr);
-        yi = mma(ur[0], xi[0], yi);
+            for (int b = 5; b < KL; b++) z ^= (((rb + r) >> (b - 5)) & 1u) ? sd[b] : 0u;
 #pragma unroll
-        for (int t = 0; t < 5; t++) {
-            const int p = t < 3 ? t : t - 3, q = (t < 3 ? 2 : 1) - p;
-            cr = mma(un[p], xi[q], cr);
-            ci = mma(ur[p], xi[q], ci);
+            for (int v = 0; v < 16; v++) {
+                const uint32_t u = z ^ ((v & 1) ? sd[0] : 0u) ^ ((v & 2) ? sd[1] : 0u) ^ ((v & 4) ? sd[3] : 0u) ^ ((v & 8) ? sd[4] : 0u);
+                re[u] = acc[r][0][v] + acc[r][2][v];
+                im[u] = acc[r][1][v] + acc[r][3][v];
+            }
         }
     }
-    // Register v of this lane is row 32 rb + 8 (v / 4) + 4 (lane / 32) + v % 4.
-    // Nothing reads the tile until the next barrier.
-    uint32_t z = dswz(coloff[cb * 32 + (lane & 31u)]) ^ ((lane >> 5) ? sd[2] : 0u);
-#pragma unroll
-    for (int b = 5; b < KL; b++) z ^= ((rb >> (b - 5)) & 1u) ? sd[b] : 0u;
-#pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const uint32_t u = z ^ ((v & 1) ? sd[0] : 0u) ^ ((v & 2) ? sd[1] : 0u) ^ ((v & 4) ? sd[3] : 0u) ^ ((v & 8) ? sd[4] : 0u);
-        re[u] = yr[v] + cr[v];
-        im[u] = yi[v] + ci[v];
-    }
+    if (first) __syncthreads();  // a wave without an item
 }
 
-// One dense block over every tile of an FP32 state: grid = tiles, 512 threads; the
-// tile (64 KiB at T = 13) and its operands (96 KiB) fill a CU's LDS, so a SIMD has two
-// waves and up to 256 VGPRs each.
+// One dense block over every tile of an FP32 state: grid = tiles, 256 threads.  Two
+// workgroups (64 KiB of LDS each at T = 13) share a CU, a wave of either on each SIMD
+// with up to 256 VGPRs: one's loads and stores run beside the other's products.
 template <int KL>
 __global__ void __launch_bounds__(DENSE_THREADS, 2)
 dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restrict__ ops, const uint4 *__restrict__ mats,
@@ -1219,7 +1243,6 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
     const uint32_t NT = 1u << T;
     float *re = reinterpret_cast<float *>(lds_raw);
     float *im = re + NT;
-    uint4 *frag = reinterpret_cast<uint4 *>(im + NT);
     const uint32_t tid = threadIdx.x;
     const uint64_t base = tile_base(blk->nontile_mask, blockIdx.x);
     // tile_q read as four words (scalar loads; byte loads would put these
@@ -1231,35 +1254,37 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
     uint64_t hq[DENSE_T_MAX];
 #pragma unroll
     for (int b = 0; b < DENSE_T_MAX; b++) hq[b] = 1ull << ((tq[b >> 2] >> (8 * (b & 3))) & 0xffu);
-    // Element e = tid + 512 i of the tile holds the amplitude whose qubits are
+    // Element e = tid + 256 i of the tile holds the amplitude whose qubits are
     // e's bits placed on tile_q (bits 0..5 are qubits 0..5).  The placement and
-    // the LDS swizzle are linear, so the thread's part (bits 0..8) is formed
-    // once and the part of i (bits 9 and up) is a scalar.
-    // Bits 6..8 of e are the wave index, a scalar: the thread's part of an
+    // the LDS swizzle are linear, so the thread's part (bits 0..7) is formed
+    // once and the part of i (bits 8 and up) is a scalar.
+    // Bits 6 and 7 of e are the wave index, a scalar: the thread's part of an
     // address is its lane alone (qubits 0..5), a 32-bit offset on a scalar base.
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t lane = tid & 63u;
-    uint64_t tg = base;
-#pragma unroll
-    for (int b = 6; b < 9; b++)
-        if ((wv >> (b - 6)) & 1u) tg |= hq[b];
+    const uint64_t tg = base | ((wv & 1u) ? hq[6] : 0ull) | ((wv & 2u) ? hq[7] : 0ull);
     const uint32_t tz = dswz(tid);
-    // i < NI = 2^(T - 9) (2..16) runs over the tile bits 9 and up, whose qubits
-    // are scalars.  Every thread issues 16 loads before using the first;
+    // i < NI = 2^(T - 8) (4..32) runs over the tile bits 8 and up, whose qubits
+    // are scalars.  Every thread issues 32 loads before using the first;
     // below T = 13 index i stands for element i mod NI, so the extra loads,
     // LDS writes and stores repeat an element with the same value (no branch).
+    constexpr int LI = 1 << (DENSE_T_MAX - 8);
     const uint32_t NI = NT / DENSE_THREADS;
-    const uint64_t h9 = T > 9 ? hq[9] : 0, h10 = T > 10 ? hq[10] : 0, h11 = T > 11 ? hq[11] : 0,
-                   h12 = T > 12 ? hq[12] : 0;
+    uint64_t hi[DENSE_T_MAX - 8];
+#pragma unroll
+    for (int b = 8; b < DENSE_T_MAX; b++) hi[b - 8] = T > (uint32_t)b ? hq[b] : 0ull;
     auto gaddr = [&](uint32_t i) {
-        return tg | ((i & 1u) ? h9 : 0ull) | ((i & 2u) ? h10 : 0ull) | ((i & 4u) ? h11 : 0ull) | ((i & 8u) ? h12 : 0ull);
+        uint64_t g = tg;
+#pragma unroll
+        for (int b = 0; b < DENSE_T_MAX - 8; b++) g |= ((i >> b) & 1u) ? hi[b] : 0ull;
+        return g;
     };
     {
-        typename V2<float>::type v[16];
+        typename V2<float>::type v[LI];
 #pragma unroll
-        for (int i = 0; i < 16; i++) v[i] = __builtin_nontemporal_load(lane_ptr(st + gaddr((uint32_t)i & (NI - 1)), lane));
+        for (int i = 0; i < LI; i++) v[i] = __builtin_nontemporal_load(lane_ptr(st + gaddr((uint32_t)i & (NI - 1)), lane));
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < LI; i++) {
             const uint32_t z = tz ^ dswz(((uint32_t)i & (NI - 1)) * DENSE_THREADS);
             re[z] = v[i].x;
             im[z] = v[i].y;
@@ -1268,23 +1293,23 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
     constexpr size_t msz = (size_t)12 << (2 * KL);  // bytes of a matrix
     for (uint32_t o = 0; o < blk->op_count; o++) {
         const dq_dense_op op = ops[blk->op_begin + o];
-        dense_op<KL>(re, im, frag, T, op, mats + op.mat * (msz / 16), ctab + (size_t)(blk->op_begin + o) * DENSE_COLS, lane, wv);
+        dense_op<KL>(re, im, T, op, mats + op.mat * (msz / 16), ctab + (size_t)(blk->op_begin + o) * DENSE_COLS, lane, wv);
     }
     __syncthreads();
     {
-        typename V2<float>::type v[16];
+        // opaque copies: the addresses are formed again here instead of being kept
+        // live through every op
+        uint32_t lane2 = lane, tz2 = tz;
+        asm volatile("" : "+v"(lane2), "+v"(tz2));
+        typename V2<float>::type v[LI];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const uint32_t z = tz ^ dswz(((uint32_t)i & (NI - 1)) * DENSE_THREADS);
+        for (int i = 0; i < LI; i++) {
+            const uint32_t z = tz2 ^ dswz(((uint32_t)i & (NI - 1)) * DENSE_THREADS);
             v[i].x = re[z];
             v[i].y = im[z];
         }
-        // an opaque copy of the lane: the store addresses are formed again here
-        // instead of the load addresses being kept live through every op
-        uint32_t lane2 = lane;
-        asm volatile("" : "+v"(lane2));
 #pragma unroll
-        for (int i = 0; i < 16; i++) __builtin_nontemporal_store(v[i], lane_ptr(st + gaddr((uint32_t)i & (NI - 1)), lane2));
+        for (int i = 0; i < LI; i++) __builtin_nontemporal_store(v[i], lane_ptr(st + gaddr((uint32_t)i & (NI - 1)), lane2));
     }
 }
 
@@ -1852,9 +1877,9 @@ extern "C" int dq_device_init(int device) {
         }
         HIPC(hipFuncSetAttribute((const void *)small_kernel<double>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
         HIPC(hipFuncSetAttribute((const void *)small_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
-        HIPC(hipFuncSetAttribute((const void *)dense_kernel<5>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
-        HIPC(hipFuncSetAttribute((const void *)dense_kernel<6>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
-        HIPC(hipFuncSetAttribute((const void *)dense_kernel<7>, hipFuncAttributeMaxDynamicSharedMemorySize, 163840));
+        HIPC(hipFuncSetAttribute((const void *)dense_kernel<5>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+        HIPC(hipFuncSetAttribute((const void *)dense_kernel<6>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+        HIPC(hipFuncSetAttribute((const void *)dense_kernel<7>, hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
         g_device = device;
     }
     return DQ_OK;
@@ -3219,7 +3244,7 @@ extern "C" int dq_compare_states(const void *a, int prec_a, const void *b, int p
 // ---- dense sweeps -------------------------------------------------------------
 namespace {
 size_t dense_mat_bytes(int k) { return (size_t)12 << (2 * k); }  // three pieces of two parts
-size_t dense_lds_bytes(uint32_t T) { return (size_t)20 << T; }   // the tile, its operands
+size_t dense_lds_bytes(uint32_t T) { return (size_t)8 << T; }
 }  // namespace
 
 extern "C" size_t dq_dense_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats) {
