@@ -194,6 +194,7 @@ struct SweepOne {
     dq_block blk;
     uint32_t baux[DQ_BAUX];
     dq_job job;
+    double *part;  // where the tiles' probability sums go, or null
 };
 
 // Non-tile qubits of tile number t (t < 2^31) from the block's runs.
@@ -362,6 +363,59 @@ __device__ __forceinline__ void warm_lines(const unsigned char *p, uint32_t byte
         (void)__hip_atomic_load(reinterpret_cast<const uint32_t *>(p + i), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
+// Probability sums of a tile as it is stored, from the registers: for every tile bit
+// (lane bits, register bits, wave bits) the sum of |a|^2 over the amplitudes with the
+// bit 0, then the total, to part[slot * workgroups + workgroup]; prob_stage2 makes P(0)
+// of every qubit of them.  A read-out after a flush took a read of the whole state; the
+// sums cost 5 FP64 instructions an amplitude and, with the lane and wave sums left
+// to one wave each by way of LDS, ~1 KB of LDS traffic a wave.  A 26-qubit FP64 Trotter step
+// with P(0) 1377 -> 1201 us, 17 qubits FP32 with their sums added up by the host 229 -> 224 us.
+// t: a thread's total, z[r]: its sum with register bit r 0.  Only sums of
+// non-negative terms: an exact 0 stays one.
+template <int R, int W>
+__device__ __forceinline__ void tile_sums(double t, const double *z, double *__restrict__ part, uint32_t lane, uint32_t wv) {
+    constexpr int NW = 1 << W, T = 6 + R + W;
+    auto *red = lds_at<double>(0);  // [1 + R][wave][lane]
+    __syncthreads();                // other waves may still read the last exchange
+    red[wv * 64 + lane] = t;
+#pragma unroll
+    for (int r = 0; r < R; r++) red[((1 + r) * NW + wv) * 64 + lane] = z[r];
+    __syncthreads();
+    auto column = [&](int v, uint32_t skip) {  // over the waves without bit `skip`
+        double a = 0.0;
+#pragma unroll
+        for (uint32_t w = 0; w < NW; w++) {
+            const double x = red[(v * NW + w) * 64 + lane];
+            a += (w & skip) ? 0.0 : x;
+        }
+        return a;
+    };
+    auto lanes = [&](double a, int from) {
+#pragma unroll
+        for (int k = 0; k < 6; k++)
+            if (k >= from) a += __shfl_xor(a, 1 << k, 64);
+        return a;
+    };
+    auto put = [&](int slot, double a) {
+        if (lane == 0) part[(uint64_t)slot * gridDim.x + blockIdx.x] = a;
+    };
+    for (uint32_t job = wv; job < 1 + R + W; job += NW) {
+        if (job == 0) {
+            double a = column(0, 0);
+#pragma unroll
+            for (int q = 0; q < 6; q++) {
+                put(q, lanes(a, q + 1));  // lane 0 has bit q 0
+                a += __shfl_xor(a, 1 << q, 64);
+            }
+            put(T, a);
+        } else if (job <= R) {
+            put(5 + job, lanes(column(job, 0), 0));
+        } else {
+            put(5 + job, lanes(column(0, 1u << (job - 1 - R)), 0));
+        }
+    }
+}
+
 // A launch of one job reads it, its block and block_aux from the kernel's
 // arguments (`one`): the tile's addresses are then one memory latency away
 // instead of three (argument, job, block).  A batch reads them per job.
@@ -404,6 +458,23 @@ sweep_kernel(const SweepOne one, const dq_job *__restrict__ jobs, const dq_block
     process_tile<T, R, W, XM>(a, phases + blk->phase_begin, nph, pa, prog, base | hi, tid, wv, false);
     if (store_needs_barrier<W>(blk)) __syncthreads();
     DQ_STORE_TILE(a, base);
+    if (gridDim.y == 1 && ka->part) {
+        double t = 0.0, z[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) z[r] = 0.0;
+#pragma unroll
+        for (int j = 0; j < (1 << R); j++) {
+            const double x = (double)a.re[j], y = (double)a.im[j], p = x * x + y * y;
+            t += p;
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (!((j >> r) & 1)) z[r] += p;
+            if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // not every product at once: they would not fit
+        }
+        // the lane formed anew: kept through the interpreter it would cost a register
+        const uint32_t l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        tile_sums<R, W>(t, z, ka->part, l, wv);
+    }
 }
 
 // Small registers (n <= 13): whole state in LDS, one workgroup per job.  Ops
@@ -615,9 +686,10 @@ struct ProbOut {
 // Stage 2: one workgroup per output q (0..n).  A number bit below cb sums its
 // slot; one at or above cb sums the totals of the workgroups whose index bit
 // (bit - cb) is 0; q == n and a qubit fixed to 0 sum every total.
-__global__ void __launch_bounds__(256) prob_stage2(const double *__restrict__ part, uint32_t groups, int n, int cb,
-                                                   const ProbOut po, double *__restrict__ out) {
-    __shared__ double red[4];
+template <int NT>
+__global__ void __launch_bounds__(NT) prob_stage2(const double *__restrict__ part, uint32_t groups, int n, int cb,
+                                                  const ProbOut po, double *__restrict__ out) {
+    __shared__ double red[NT / 64];
     const int q = blockIdx.x;
     const uint32_t tid = threadIdx.x;
     const int bit = q == n ? PROB_FIXED0 : po.bit[q];
@@ -626,14 +698,20 @@ __global__ void __launch_bounds__(256) prob_stage2(const double *__restrict__ pa
     const double *__restrict__ src = part + (uint64_t)slot * groups;
     double acc = 0.0;
 #pragma unroll 8
-    for (uint32_t g = tid; g < groups; g += 256) {
+    for (uint32_t g = tid; g < groups; g += NT) {
         const double v = src[g];
         acc += (g & skip) ? 0.0 : v;
     }
     acc = wave_sum(acc);
     if ((tid & 63) == 0) red[tid >> 6] = acc;
     __syncthreads();
-    if (tid == 0) out[q] = bit == PROB_FIXED1 ? 0.0 : po.scale * ((red[0] + red[1]) + (red[2] + red[3]));
+    if (tid == 0) {
+#pragma unroll
+        for (int k = NT / 128; k; k /= 2)
+#pragma unroll
+            for (int i = 0; i < k; i++) red[i] = red[2 * i] + red[2 * i + 1];
+        out[q] = bit == PROB_FIXED1 ? 0.0 : po.scale * red[0];
+    }
 }
 
 // Both stages in one launch of one workgroup of 16 waves, for up to 2^PROB_ONE_BITS
@@ -2783,9 +2861,9 @@ static int validate_block(const dq_block &b, const dq_phase *phases, uint32_t n_
     return DQ_OK;
 }
 
-extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_blocks, const dq_phase *phases,
-                               uint32_t n_phases, const dq_op *ops, uint32_t n_ops, const dq_job *jobs,
-                               const uint32_t *job_begin, uint32_t n_launch, void *d_ws, size_t ws_bytes, void *stream) {
+static int apply_blocks(int prec, const dq_block *blocks, uint32_t n_blocks, const dq_phase *phases, uint32_t n_phases,
+                        const dq_op *ops, uint32_t n_ops, const dq_job *jobs, const uint32_t *job_begin, uint32_t n_launch,
+                        double *part, void *d_ws, size_t ws_bytes, void *stream) {
     if (prec != DQ_F32 && prec != DQ_F64) return fail(DQ_ERR_ARG, "dq_apply_blocks: bad precision %d", prec);
     if (n_launch == 0) return DQ_OK;
     if (!blocks || !phases || !jobs || !job_begin || !d_ws) return fail(DQ_ERR_ARG, "dq_apply_blocks: null argument");
@@ -2934,7 +3012,9 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
             bool multi = false;
             for (uint32_t j = j0; j < j0 + nj; j++) multi |= blocks[jobs[j].block].phase_count > 1;
             const int xm = exchange_mode(prec, (int)b0.reg_bits, (int)b0.wave_bits, (int)b0.tile_bits);
-            const size_t lds = multi ? ((size_t)1 << b0.tile_bits) * exchange_elem_bytes(prec, xm) : 0;
+            size_t lds = multi ? ((size_t)1 << b0.tile_bits) * exchange_elem_bytes(prec, xm) : 0;
+            const bool sums = part && l == n_launch - 1;
+            if (sums) lds = std::max(lds, ((size_t)(1 + b0.reg_bits) * 64 * sizeof(double)) << b0.wave_bits);
             if (lds > 131072) return fail(DQ_ERR_UNSUPPORTED, "tile of %d bits needs %zu bytes of LDS", b0.tile_bits, lds);
             const uint64_t tiles = 1ull << (n - b0.tile_bits);
             if (tiles > 0x7fffffffull || nj > 65535 || ((tiles << (6 + b0.wave_bits)) >> 32))
@@ -2945,12 +3025,93 @@ extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_bloc
             one.blk = b0;
             memcpy(one.baux, baux.data() + (size_t)jobs[j0].block * DQ_BAUX, sizeof one.baux);
             one.job = jobs[j0];
+            one.part = sums ? part : nullptr;
             hipLaunchKernelGGL(fn, dim3((unsigned)tiles, nj), dim3(64u << b0.wave_bits), lds, (hipStream_t)stream, one,
                                d_jobs + j0, d_blocks, d_phases, d_prog, d_paux, d_baux);
         }
         HIPC(hipGetLastError());
     }
     return DQ_OK;
+}
+
+extern "C" int dq_apply_blocks(int prec, const dq_block *blocks, uint32_t n_blocks, const dq_phase *phases,
+                               uint32_t n_phases, const dq_op *ops, uint32_t n_ops, const dq_job *jobs,
+                               const uint32_t *job_begin, uint32_t n_launch, void *d_ws, size_t ws_bytes, void *stream) {
+    return apply_blocks(prec, blocks, n_blocks, phases, n_phases, ops, n_ops, jobs, job_begin, n_launch, nullptr, d_ws, ws_bytes, stream);
+}
+
+// ---- P(0) of every qubit from the sums of the last sweep -------------------------
+// Up to kPartHost tiles write their sums to a result slot and the host adds them up: a
+// launch less (4-5 us).  From kPartMax tiles on (their sums take 16 MiB) the state
+// is read again.
+constexpr uint32_t kPartHost = 32, kPartMax = 1u << 17;
+
+extern "C" size_t dq_block_sums_bytes(const dq_block *b) {
+    if (!b || b->reg_bits == 0 || b->n_qubits > PROB_MAX_QUBITS || b->tile_bits > b->n_qubits) return 0;
+    const uint32_t log = b->n_qubits - b->tile_bits;
+    if (log >= 32 || (1u << log) > kPartMax) return 0;
+    return ((size_t)(b->tile_bits + 1) << log) * sizeof(double);
+}
+
+extern "C" int dq_block_sums_on_host(const dq_block *b) {
+    return dq_block_sums_bytes(b) && (1u << (b->n_qubits - b->tile_bits)) <= kPartHost;
+}
+
+extern "C" int dq_apply_blocks_sums(int prec, const dq_block *blocks, uint32_t n_blocks, const dq_phase *phases,
+                                    uint32_t n_phases, const dq_op *ops, uint32_t n_ops, const dq_job *jobs,
+                                    const uint32_t *job_begin, uint32_t n_launch, double *sums, size_t sums_bytes, void *d_ws,
+                                    size_t ws_bytes, void *stream) {
+    if (!blocks || !jobs || !job_begin || !sums || n_launch == 0) return fail(DQ_ERR_ARG, "dq_apply_blocks_sums: null argument");
+    const dq_job &last = jobs[job_begin[n_launch - 1]];
+    if (job_begin[n_launch] - job_begin[n_launch - 1] != 1 || last.block >= n_blocks)
+        return fail(DQ_ERR_ARG, "dq_apply_blocks_sums: the last launch must have one job");
+    const size_t need = dq_block_sums_bytes(blocks + last.block);
+    if (!need || sums_bytes < need) return fail(DQ_ERR_ARG, "dq_apply_blocks_sums: sums of %zu bytes", sums_bytes);
+    return apply_blocks(prec, blocks, n_blocks, phases, n_phases, ops, n_ops, jobs, job_begin, n_launch, sums, d_ws, ws_bytes, stream);
+}
+
+extern "C" int dq_prob_of_sums(const dq_block *b, const double *sums, double *out, double *d_out, void *stream) {
+    const size_t bytes = dq_block_sums_bytes(b);
+    if (!bytes || !sums || !out) return fail(DQ_ERR_ARG, "dq_prob_of_sums: bad arguments");
+    const int n = (int)b->n_qubits, T = (int)b->tile_bits;
+    const uint32_t groups = 1u << (n - T);
+    ProbOut po;
+    memset(&po, 0, sizeof po);
+    po.scale = 1.0;
+    int outside = T;
+    for (int q = 0; q < n; q++) {
+        const uint64_t m = 1ull << q;
+        int bit = q < 6 ? q : -1;
+        for (uint32_t r = 0; r < b->reg_bits; r++)
+            if (b->st_reg[r] == m) bit = 6 + (int)r;
+        for (uint32_t w = 0; w < b->wave_bits; w++)
+            if (b->st_wave[w] == m) bit = 6 + (int)(b->reg_bits + w);
+        if (b->nontile_mask & m) bit = outside++;
+        if (bit < 0) return fail(DQ_ERR_ARG, "dq_prob_of_sums: qubit %d is in no place", q);
+        po.bit[q] = (uint8_t)bit;
+    }
+    if (dq_block_sums_on_host(b)) {
+        std::vector<double> v(bytes / sizeof(double));
+        const int rc = dq_result_wait(sums, v.data(), bytes, stream);
+        if (rc) return rc;
+        for (int q = 0; q <= n; q++) {
+            const int bit = q == n ? T : po.bit[q];
+            const double *src = v.data() + (size_t)std::min(bit, T) * groups;
+            const uint32_t skip = q < n && bit >= T ? 1u << (bit - T) : 0u;
+            double a = 0.0;
+            for (uint32_t g = 0; g < groups; g++)
+                if (!(g & skip)) a += src[g];
+            out[q] = a;
+        }
+        return DQ_OK;
+    }
+    if (!d_out) return fail(DQ_ERR_ARG, "dq_prob_of_sums: null output");
+    ResultSlot res((n + 1) * sizeof(double), d_out);
+    hipStream_t s = (hipStream_t)stream;
+    if (groups > 8192) hipLaunchKernelGGL(prob_stage2<1024>, dim3(n + 1), dim3(1024), 0, s, sums, groups, n, T, po, (double *)res.dst);
+    else hipLaunchKernelGGL(prob_stage2<256>, dim3(n + 1), dim3(256), 0, s, sums, groups, n, T, po, (double *)res.dst);
+    HIPC(hipGetLastError());
+    return res.collect(out, (n + 1) * sizeof(double), stream);
 }
 
 // Split of 2^nf amplitudes over prob_stage1's workgroups: cb bits each, 2^JB
@@ -3035,7 +3196,7 @@ static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, 
 #undef DQ_PROB1J
 #undef DQ_PROB1
     HIPC(hipGetLastError());
-    hipLaunchKernelGGL(prob_stage2, dim3(n + 1), dim3(256), 0, stream, part, p.groups, n, p.cb, po, d_out);
+    hipLaunchKernelGGL(prob_stage2<256>, dim3(n + 1), dim3(256), 0, stream, part, p.groups, n, p.cb, po, d_out);
     HIPC(hipGetLastError());
     return DQ_OK;
 }

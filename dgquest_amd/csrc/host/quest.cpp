@@ -220,7 +220,17 @@ void ensure_ws(QuregState *s, size_t bytes) {
     s->ws_cap = cap;
 }
 
-static void run_plan(QuregState *s, const Plan &P) {
+// The sums of a state's probabilities that its last sweep writes: where, and the
+// block whose tiles they are of.
+struct StateSums {
+    double *at = nullptr;   // a result slot or device memory
+    double *d_out = nullptr;
+    bool slot = false;
+    dq_block block;
+};
+
+// Runs a plan; with `sums`, its last sweep writes them if it can (sums->at is set then).
+static void run_plan(QuregState *s, const Plan &P, StateSums *sums = nullptr) {
     if (P.blocks.empty()) return;
     const uint32_t nb = (uint32_t)P.blocks.size();
     std::vector<dq_job> jobs(nb);
@@ -233,10 +243,30 @@ static void run_plan(QuregState *s, const Plan &P) {
         begin[i] = i;
     }
     begin[nb] = nb;
-    ensure_ws(s, dq_apply_ws_bytes(nb, (uint32_t)P.phases.size(), (uint32_t)P.ops.size(), nb));
-    ENG(dq_apply_blocks(s->prec, P.blocks.data(), nb, P.phases.data(), (uint32_t)P.phases.size(),
-                        P.ops.empty() ? nullptr : P.ops.data(), (uint32_t)P.ops.size(), jobs.data(), begin.data(), nb,
-                        s->d_ws, s->ws_cap, s->stream));
+    size_t ws = dq_apply_ws_bytes(nb, (uint32_t)P.phases.size(), (uint32_t)P.ops.size(), nb);
+    const size_t bytes = sums ? dq_block_sums_bytes(&P.blocks.back()) : 0;
+    if (bytes) {
+        sums->block = P.blocks.back();
+        if (dq_block_sums_on_host(&sums->block)) {
+            sums->at = (double *)dq_result_acquire(bytes);
+            sums->slot = sums->at != nullptr;
+        } else {
+            const size_t off = (ws + 255) / 256 * 256, out = off + (bytes + 255) / 256 * 256;
+            ws = out + (s->n + 1) * sizeof(double);
+            ensure_ws(s, ws);
+            sums->at = (double *)((unsigned char *)s->d_ws + off);
+            sums->d_out = (double *)((unsigned char *)s->d_ws + out);
+        }
+    }
+    ensure_ws(s, ws);
+    const dq_op *ops = P.ops.empty() ? nullptr : P.ops.data();
+    if (bytes && sums->at)
+        ENG(dq_apply_blocks_sums(s->prec, P.blocks.data(), nb, P.phases.data(), (uint32_t)P.phases.size(), ops,
+                                 (uint32_t)P.ops.size(), jobs.data(), begin.data(), nb, sums->at, bytes, s->d_ws, s->ws_cap,
+                                 s->stream));
+    else
+        ENG(dq_apply_blocks(s->prec, P.blocks.data(), nb, P.phases.data(), (uint32_t)P.phases.size(), ops,
+                            (uint32_t)P.ops.size(), jobs.data(), begin.data(), nb, s->d_ws, s->ws_cap, s->stream));
 }
 
 // Rotating lanes in whole-register plans (DGQ_ROTATE=0 turns them off, for
@@ -298,7 +328,7 @@ static bool rotation_for(const QuregState *s) {
     return rotation_allowed(s);
 }
 
-void flush(QuregState *s, bool home) {
+void flush(QuregState *s, bool home, bool probs) {
     if (s->recorder) engine_fatal("a recording register cannot execute or read its state", DQ_ERR_UNSUPPORTED);
     if (s->pending.empty() && s->init_kind == DQ_INIT_LOAD) return;
     s->det_base = false;
@@ -315,6 +345,7 @@ void flush(QuregState *s, bool home) {
     }
     const auto t0 = std::chrono::steady_clock::now();
     const unsigned long long state_bytes = (unsigned long long)(s->prec == DQ_F64 ? 16 : 8) << s->n;
+    StateSums sums;
     s->last_dense_flops = 0.0;
     if (s->pending.empty()) {
         ENG(dq_init_state(s->d_state, s->n, s->prec, s->init_kind, s->init_index, s->init_value, s->stream));
@@ -356,7 +387,7 @@ void flush(QuregState *s, bool home) {
             cache_plan(s, s->tune, rot, P, false, end_lanes);
         }
         if (home) rename_to_home(P, s->n, s->l2p);
-        run_plan(s, P);
+        run_plan(s, P, probs ? &sums : nullptr);
         if (!P.moved.empty()) {  // the plan moved qubits: logical q now sits at moved[l2p[q]]
             for (int q = 0; q < s->n; q++) s->l2p[q] = P.moved[s->l2p[q]];
             for (int q = 0; q < s->n; q++) s->p2l[s->l2p[q]] = q;
@@ -370,6 +401,15 @@ void flush(QuregState *s, bool home) {
     s->init_kind = DQ_INIT_LOAD;
     s->probs_dirty = true;
     s->last_flush_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    if (sums.at) {
+        s->p0.assign(s->n + 1, 0.0);
+        ENG(dq_prob_of_sums(&sums.block, sums.at, s->p0.data(), sums.d_out, s->stream));
+        if (sums.slot) dq_result_release(sums.at);
+        s->probs_dirty = false;
+        s->det_pending = 0;
+        s->det_slack = 0.0;
+        s->det_base = true;
+    }
 }
 
 // Are the recorded gates nothing but measurement collapses, of qubits not
@@ -410,7 +450,7 @@ void ensure_probs(QuregState *s) {
         s->det_slack = 0.0;
         return;
     }
-    flush(s);
+    flush(s, false, true);
     if (!s->probs_dirty) return;
     s->det_pending = 0;
     s->det_slack = 0.0;

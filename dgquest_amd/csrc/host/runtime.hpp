@@ -79,7 +79,7 @@ namespace dgq {
 void ensure_ws(QuregState *s, size_t bytes);
 // home: the caller wants the state in logical qubit order next; a plan that
 // generates its state then ends there as far as it can (rename_to_home).
-void flush(QuregState *s, bool home = false);
+void flush(QuregState *s, bool home = false, bool probs = false);
 void ensure_probs(QuregState *s);
 void materialize_mapping(QuregState *s);
 

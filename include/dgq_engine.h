@@ -199,6 +199,23 @@ int dq_apply_blocks(int prec,
                     const dq_job *jobs, const uint32_t *job_begin, uint32_t n_launch,
                     void *d_ws, size_t ws_bytes, void *stream);
 
+/* dq_apply_blocks whose last launch (of one job) also writes, as it stores the
+ * state, every tile's sums of |a|^2 to `sums` (dq_block_sums_bytes of that
+ * block; 0: not available for it): device memory, or a result slot where
+ * dq_block_sums_on_host says so.  dq_prob_of_sums makes of them what
+ * dq_prob_zero_all reads from the state: out[q] = P(q = 0) for the n qubits as
+ * they were stored, out[n] = the total.  d_out: n + 1 doubles of device memory
+ * (unused with a slot).  It waits for the result. */
+int dq_apply_blocks_sums(int prec,
+                         const dq_block *blocks, uint32_t n_blocks,
+                         const dq_phase *phases, uint32_t n_phases,
+                         const dq_op *ops, uint32_t n_ops,
+                         const dq_job *jobs, const uint32_t *job_begin, uint32_t n_launch,
+                         double *sums, size_t sums_bytes, void *d_ws, size_t ws_bytes, void *stream);
+size_t dq_block_sums_bytes(const dq_block *b);
+int dq_block_sums_on_host(const dq_block *b);
+int dq_prob_of_sums(const dq_block *b, const double *sums, double *out, double *d_out, void *stream);
+
 /* Bytes of device workspace dq_apply_blocks needs for these counts. */
 size_t dq_apply_ws_bytes(uint32_t n_blocks, uint32_t n_phases, uint32_t n_ops, uint32_t n_jobs);
 
