@@ -3081,6 +3081,19 @@ extern "C" int dq_apply_blocks_sums(int prec, const dq_block *blocks, uint32_t n
     return apply_blocks(prec, blocks, n_blocks, phases, n_phases, ops, n_ops, jobs, job_begin, n_launch, sums, d_ws, ws_bytes, stream);
 }
 
+// prob_stage2 on the host.
+static void prob_add(const double *part, uint32_t groups, int n, int cb, const ProbOut &po, double *out) {
+    for (int q = 0; q <= n; q++) {
+        const int bit = q == n ? PROB_FIXED0 : po.bit[q];
+        const double *src = part + (size_t)std::min(bit, cb) * groups;
+        const uint32_t skip = bit >= cb && bit < PROB_FIXED0 ? 1u << (bit - cb) : 0u;
+        double a = 0.0;
+        for (uint32_t g = 0; g < groups; g++)
+            if (!(g & skip)) a += src[g];
+        out[q] = bit == PROB_FIXED1 ? 0.0 : po.scale * a;
+    }
+}
+
 extern "C" int dq_prob_of_sums(const dq_block *b, const double *sums, double *out, double *d_out, void *stream) {
     const size_t bytes = dq_block_sums_bytes(b);
     if (!bytes || !sums || !out) return fail(DQ_ERR_ARG, "dq_prob_of_sums: bad arguments");
@@ -3105,15 +3118,7 @@ extern "C" int dq_prob_of_sums(const dq_block *b, const double *sums, double *ou
         std::vector<double> v(bytes / sizeof(double));
         const int rc = dq_result_wait(sums, v.data(), bytes, stream);
         if (rc) return rc;
-        for (int q = 0; q <= n; q++) {
-            const int bit = q == n ? T : po.bit[q];
-            const double *src = v.data() + (size_t)std::min(bit, T) * groups;
-            const uint32_t skip = q < n && bit >= T ? 1u << (bit - T) : 0u;
-            double a = 0.0;
-            for (uint32_t g = 0; g < groups; g++)
-                if (!(g & skip)) a += src[g];
-            out[q] = a;
-        }
+        prob_add(v.data(), groups, n, T, po, out);
         return DQ_OK;
     }
     if (!d_out) return fail(DQ_ERR_ARG, "dq_prob_of_sums: null output");
@@ -3131,6 +3136,7 @@ extern "C" int dq_prob_of_sums(const dq_block *b, const double *sums, double *ou
 // a thread has 16 loads in flight and workgroups are added up to 2^PROB_GROUPS,
 // from where the loop inside a workgroup grows.
 #define PROB_GROUPS 13
+constexpr int kProbHostBits = 18;
 struct ProbSplit {
     int cb, jb;
     uint32_t groups;
@@ -3153,16 +3159,8 @@ static size_t prob_part_bytes(int nf) {
 
 extern "C" size_t dq_prob_ws_bytes(int n) { return prob_part_bytes(n) + 64 * sizeof(double); }
 
-static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, uint64_t fixed_value, double scale,
-                       double *d_out, void *d_ws, size_t ws_bytes, hipStream_t stream) {
-    if (!state || !d_out || !d_ws || n < 1 || n > PROB_MAX_QUBITS || (prec != DQ_F32 && prec != DQ_F64))
-        return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad arguments");
-    if ((fixed_mask >> n) || (fixed_value & ~fixed_mask)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad fixed bits");
-    const int nf = n - __builtin_popcountll(fixed_mask);
-    if (ws_bytes < prob_part_bytes(nf)) return fail(DQ_ERR_ARG, "dq_prob_zero_all_async: workspace too small");
-    const ProbSplit p = prob_split(nf);
-    ProbBits pb;
-    ProbOut po;
+// The number bits of a state's free qubits and what stage 2 makes of every qubit.
+static int prob_bits(int n, uint64_t fixed_mask, uint64_t fixed_value, double scale, ProbBits &pb, ProbOut &po) {
     memset(&pb, 0, sizeof pb);
     memset(&po, 0, sizeof po);
     pb.fixed = fixed_value;
@@ -3177,17 +3175,10 @@ static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, 
             pb.img[f++] = b;
         }
     }
-    // One launch where a workgroup's 8 loads per thread cover the state: the second
-    // launch takes longer (3.5 us) than what more workgroups would save.
-    if (nf <= PROB_ONE_BITS) {
-        if (prec == DQ_F64)
-            hipLaunchKernelGGL(prob_one<double>, dim3(1), dim3(1024), 0, stream, (const V2<double>::type *)state, pb, nf, n, po, d_out);
-        else
-            hipLaunchKernelGGL(prob_one<float>, dim3(1), dim3(1024), 0, stream, (const V2<float>::type *)state, pb, nf, n, po, d_out);
-        HIPC(hipGetLastError());
-        return DQ_OK;
-    }
-    double *part = (double *)d_ws;
+    return f;
+}
+
+static int prob_sums(const void *state, int prec, const ProbBits &pb, int nf, const ProbSplit &p, double *part, hipStream_t stream) {
 #define DQ_PROB1(T_, JB_)                                                                          \
     hipLaunchKernelGGL((prob_stage1<T_, JB_>), dim3(p.groups), dim3(256), 0, stream, (const V2<T_>::type *)state, pb, nf, \
                        p.cb, part)
@@ -3207,6 +3198,32 @@ static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, 
 #undef DQ_PROB1J
 #undef DQ_PROB1
     HIPC(hipGetLastError());
+    return DQ_OK;
+}
+
+static int prob_launch(const void *state, int n, int prec, uint64_t fixed_mask, uint64_t fixed_value, double scale,
+                       double *d_out, void *d_ws, size_t ws_bytes, hipStream_t stream) {
+    if (!state || !d_out || !d_ws || n < 1 || n > PROB_MAX_QUBITS || (prec != DQ_F32 && prec != DQ_F64))
+        return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad arguments");
+    if ((fixed_mask >> n) || (fixed_value & ~fixed_mask)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad fixed bits");
+    ProbBits pb;
+    ProbOut po;
+    const int nf = prob_bits(n, fixed_mask, fixed_value, scale, pb, po);
+    if (ws_bytes < prob_part_bytes(nf)) return fail(DQ_ERR_ARG, "dq_prob_zero_all_async: workspace too small");
+    const ProbSplit p = prob_split(nf);
+    // One launch where a workgroup's 8 loads per thread cover the state: the second
+    // launch takes longer (3.5 us) than what more workgroups would save.
+    if (nf <= PROB_ONE_BITS) {
+        if (prec == DQ_F64)
+            hipLaunchKernelGGL(prob_one<double>, dim3(1), dim3(1024), 0, stream, (const V2<double>::type *)state, pb, nf, n, po, d_out);
+        else
+            hipLaunchKernelGGL(prob_one<float>, dim3(1), dim3(1024), 0, stream, (const V2<float>::type *)state, pb, nf, n, po, d_out);
+        HIPC(hipGetLastError());
+        return DQ_OK;
+    }
+    double *part = (double *)d_ws;
+    const int rc = prob_sums(state, prec, pb, nf, p, part, stream);
+    if (rc) return rc;
     hipLaunchKernelGGL(prob_stage2<256>, dim3(n + 1), dim3(256), 0, stream, part, p.groups, n, p.cb, po, d_out);
     HIPC(hipGetLastError());
     return DQ_OK;
@@ -3223,6 +3240,30 @@ extern "C" int dq_prob_zero_all_fixed(const void *state, int n, int prec, uint64
     if (ws_bytes < dq_prob_ws_bytes(n)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: workspace too small");
     const size_t part_bytes = prob_part_bytes(n);
     double *d_out = (double *)((unsigned char *)d_ws + part_bytes);
+    if (!state || !d_ws || (prec != DQ_F32 && prec != DQ_F64)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad arguments");
+    if ((fixed_mask >> n) || (fixed_value & ~fixed_mask)) return fail(DQ_ERR_ARG, "dq_prob_zero_all: bad fixed bits");
+    ProbBits pb;
+    ProbOut po;
+    const int nf = prob_bits(n, fixed_mask, fixed_value, scale, pb, po);
+    if (fixed_mask && nf <= kProbHostBits) {
+        // (Whole states are summed as dq_prob_zero_all_noalloc does, to the same bits.)  Up to 64 workgroups write their sums to a result slot and the host adds them up: no
+        // second launch (4.5 us), and up to 2^13 amplitudes no single workgroup (4.8
+        // against 7.6 us).  23 qubits measured one after another 603 -> 541 us.
+        ProbSplit p;
+        p.cb = std::min(nf, std::max(8, nf - 6));
+        p.jb = std::max(0, p.cb - 8);
+        p.groups = 1u << (nf - p.cb);
+        const size_t bytes = (size_t)p.groups * (p.cb + 1) * sizeof(double);
+        ResultSlot res(bytes, nullptr);
+        if (res.host) {
+            int rc = prob_sums(state, prec, pb, nf, p, (double *)res.host, (hipStream_t)stream);
+            std::vector<double> v(bytes / sizeof(double));
+            if (!rc) rc = res.collect(v.data(), bytes, stream);
+            if (rc) return rc;
+            prob_add(v.data(), p.groups, n, p.cb, po, out);
+            return DQ_OK;
+        }
+    }
     ResultSlot res((n + 1) * sizeof(double), d_out);
     const int rc = prob_launch(state, n, prec, fixed_mask, fixed_value, scale, (double *)res.dst, d_ws, part_bytes, (hipStream_t)stream);
     if (rc) return rc;
