@@ -81,7 +81,7 @@ def parse():
     ap.add_argument("--resident-bv", type=int, default=34,
                     help="qubits of the Bernstein-Vazirani run held resident in HBM (0 = skip)")
     ap.add_argument("--precision-qubits", type=int, default=32,
-                    help="grid-circuit size of the FP32 MFMA precision-form run (0 = skip)")
+                    help="grid-circuit size of the dense precision-form run (0 = skip)")
     ap.add_argument("--precision-k", type=str, default="5,6,7")
     return ap.parse_args()
 
@@ -491,10 +491,10 @@ def precision_form(q64, args):
     """Config 4: a 4 x (n/4) grid circuit of depth 20 (sqrt X/Y/W per qubit per
     cycle, CZ on four edge patterns in rotation), seed 4.  FP64 butterflies on
     the GPU give the reference state; then an FP32 state runs the same circuit
-    as dense 2^k x 2^k blocks on FP32 MFMA for each k.  Reported per k: time of
+    as dense 2^k x 2^k blocks on MFMA for each k.  Reported per k: time of
     the dense sweeps (HIP events on the register's stream), dense ops,
-    GEMM flops (8 * 2^k * 2^n per op), MFMA utilisation against the 157.3
-    TFLOP/s FP32 dense peak, HBM GB/s, fidelity |<psi64|psi32>|^2 (normalised)
+    FP32 GEMM flops (8 * 2^k * 2^n per op), MFMA utilisation of the six bf16
+    products that make an FP32 one against the 2.5 PFLOP/s bf16 dense peak, HBM GB/s, fidelity |<psi64|psi32>|^2 (normalised)
     and max |delta amplitude|."""
     import ctypes as C
 
@@ -540,14 +540,14 @@ def precision_form(q64, args):
         rows[f"k{k}"] = {"ms": round(ms, 2), "sweeps": ds["sweeps"], "dense_ops": ds["ops"],
                          "gemm_TFLOP": round(ds["flops"] / 1e12, 2),
                          "TFLOPs": round(ds["flops"] / (ms * 1e-3) / 1e12, 2),
-                         "mfma_utilisation": round(ds["flops"] / (ms * 1e-3) / 157.3e12, 4),
+                         "mfma_utilisation": round(6 * ds["flops"] / (ms * 1e-3) / 2.5e15, 4),
                          "hbm_GBps": round(hbm, 1), "fidelity": fid, "raw_overlap_sq": abs(cmp["inner"]) ** 2,
                          "max_abs_err": cmp["max_abs_diff"], "host_plan_ms": round(ds["flush_ms"], 1)}
         q32.destroyQureg(st, env32)
     q64.destroyQureg(ref, env)
     return {"workload": f"{n}-qubit 4x{cols} grid circuit, depth 20, sqrt X/Y/W + CZ patterns, seed 4",
             "fp64_reference_ms": round(ms64, 2), "fp64_sweeps": sweeps64, "fp32_dense": rows,
-            "mfma_peak_TFLOPs": 157.3}
+            "mfma_peak_TFLOPs": 2500.0}
 
 
 def main():

@@ -3,8 +3,8 @@
 // A flush becomes dense blocks: tiles of T = min(13, n) qubits (qubits 0..5
 // always in, for coalesced loads) selected on the full qubit support of every
 // gate, each split into dense ops whose support is at most k qubits.  An op's
-// 2^k x 2^k complex matrix is the product of its gates, formed on the host in
-// double precision; the device applies it to the FP32 state on MFMA
+// 2^k x 2^k complex matrix is the product of its gates, formed on the device in
+// double precision, which applies it to the FP32 state on MFMA
 // (dq_apply_dense).  Block selection is the reference's DAG selection
 // (src/cpp/DAG.cpp:219-259) counting controls and diagonals as well, since a
 // dense op has no free diagonal qubits.

@@ -273,7 +273,8 @@ int dq_prob_zero_all_noalloc(const void *state, int n_qubits, int prec, double *
  * order, and stores the tile back.  A dense op multiplies, for every
  * assignment of the other tile bits, the 2^k-vector of amplitudes indexed by
  * its k tile bits (matrix-index bit j = tile bit bits[j]) by a 2^k x 2^k
- * complex matrix, computed as one real GEMM per tile on FP32 MFMA with FP32
+ * complex matrix, computed as a GEMM per tile on bf16 MFMA, every FP32 factor as
+ * the sum of three bf16 pieces, with FP32
  * accumulation.  k is 5, 6 or 7, the same for all ops of a call, and
  * k + 5 <= T <= 13. */
 typedef struct dq_dense_block {
@@ -292,7 +293,7 @@ typedef struct dq_dense_op {
 
 /* Apply `n_blocks` dense blocks in order to an FP32 state of n qubits.
  * mats: n_mats complex matrices, 2^k x 2^k each, row-major {re, im} doubles
- * (host memory; rounded to float and laid out for MFMA by this call). */
+ * (host memory; split into bf16 pieces and laid out for MFMA by this call). */
 int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops, uint32_t n_ops,
                    const double *mats, uint32_t n_mats, void *state, void *d_ws, size_t ws_bytes, void *stream);
 size_t dq_dense_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats);

@@ -142,7 +142,7 @@ int dgq_tune_reload(const char *path);
 
 /* Precision form: from now on, flushes of this FP32 register run as dense
  * sweeps of width k (5, 6 or 7): the recorded gates are grouped into dense
- * 2^k x 2^k complex matrices, applied on FP32 MFMA with FP32 accumulation
+ * 2^k x 2^k complex matrices, applied as split FP32 products on MFMA with FP32 accumulation
  * inside 13-qubit tiles (dq_apply_dense).  k = 0 returns to fused
  * butterflies.  Gates recorded before the call run first, in the current
  * form.  -1 for a FP64, paged or too small register (k + 5 <= min(n, 13)). */
