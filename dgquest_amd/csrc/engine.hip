@@ -1777,6 +1777,12 @@ struct StageSlot {
     bool by_event = false; // that upload is guarded by ev, not by its number
     hipEvent_t ev = nullptr;
 };
+// Host memory of the staging and result protocols, which work while kernels run: the
+// host polls words that a kernel stores before it ends, and rewrites a buffer that an
+// earlier kernel has read without a wait for that kernel's stream.  Both need coherent
+// memory; without the flag the runtime and its environment decide.
+hipError_t shared_host_alloc(void **p, size_t bytes) { return hipHostMalloc(p, bytes, hipHostMallocPortable | hipHostMallocCoherent); }
+
 constexpr unsigned kStageMax = 64;
 constexpr size_t kStageHeader = 256;
 constexpr size_t kStageKernelBytes = 64 * 1024;
@@ -1857,7 +1863,7 @@ static int stage_pick(size_t bytes, StageSlot *&out) {
         s.cap = 0;
         size_t cap = kStageKernelBytes;
         while (cap < bytes) cap *= 2;
-        HIPC(hipHostMalloc(&s.host, kStageHeader + cap, hipHostMallocPortable));
+        HIPC(shared_host_alloc(&s.host, kStageHeader + cap));
         s.cap = cap;
         s.ticket = 0;
         s.by_event = false;
@@ -1943,7 +1949,7 @@ extern "C" void *dq_result_acquire(size_t bytes) {
         std::lock_guard<std::mutex> lk(g_result_mu);
         for (int i = 0; i < kResultMax && !slot; i++) {
             if (g_result_taken[i]) continue;
-            if (!g_result[i] && hipHostMalloc(&g_result[i], kResultBytes, hipHostMallocPortable) != hipSuccess) {
+            if (!g_result[i] && shared_host_alloc(&g_result[i], kResultBytes) != hipSuccess) {
                 (void)hipGetLastError();
                 g_result[i] = nullptr;
                 return nullptr;

@@ -1,0 +1,58 @@
+"""The engine's pools of pinned host memory (descriptor uploads, read-out results)
+against a stand-in for the HIP runtime (fake_hip.c); no GPU.
+
+Each test runs in a process of its own: the stand-in has to be loaded before
+the engine.
+"""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SETUP = """
+import ctypes as C, sys, threading, time
+hip = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+L = C.CDLL(sys.argv[2])
+L.dq_last_error.restype = C.c_char_p
+L.dq_result_acquire.restype = C.c_void_p
+L.dq_result_acquire.argtypes = [C.c_size_t]
+L.dq_readout_ws_bytes.restype = C.c_size_t
+hip.fake_flags.restype = C.c_uint32
+n = 8
+state = C.create_string_buffer(16 << n)
+states = (C.c_void_p * 1)(C.addressof(state))
+wsb = L.dq_readout_ws_bytes(n, 1, 0)
+
+def upload():  # a read-out uploads its state pointers; 0 or an error code
+    ws = C.create_string_buffer(wsb + 256)
+    keep.append(ws)
+    at = (C.addressof(ws) + 255) // 256 * 256
+    return L.dq_readout_many(2, n, states, 1, None, 0, None, None, C.c_void_p(at), C.c_size_t(wsb), None)
+
+keep = []
+"""
+
+
+def run(tmp_path, body):
+    fake = tmp_path / "libfake_hip.so"
+    subprocess.check_call(["cc", "-O1", "-shared", "-fPIC", "-pthread", "-o", str(fake), os.path.join(ROOT, "tests", "fake_hip.c")])
+    lib = os.path.join(ROOT, "dgquest_amd", "lib", "libdgq_engine.so")
+    p = subprocess.run([sys.executable, "-c", SETUP + body, str(fake), lib], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0, p.stdout + p.stderr
+
+
+def test_memory_shared_with_running_kernels_is_coherent(tmp_path):
+    # hipHostMallocCoherent (0x40000000): a host that polls sees a word before its kernel ends, and a kernel
+    # sees what the host wrote into a buffer that an earlier kernel has read
+    run(tmp_path, """
+assert L.dq_result_acquire(64)
+assert hip.fake_allocs() == 1
+assert upload() == 0, L.dq_last_error()
+assert hip.fake_allocs() == 2
+for i in range(2):
+    assert hip.fake_flags(i) & 0x40000000, hex(hip.fake_flags(i))
+    assert not hip.fake_flags(i) & 0x80000000
+""")
