@@ -477,6 +477,8 @@ static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value
     return true;
 }
 
+// p0 of the state with everything recorded.  The state itself may stay as it was
+// before recorded collapses: who reads it too flushes first.
 void ensure_probs(QuregState *s) {
     // Measuring qubit after qubit: the collapses stay recorded and P(0) comes
     // from the amplitudes they keep, half as many for every qubit measured,
@@ -632,6 +634,7 @@ Qureg createQureg(int numQubits, QuESTEnv env) {
 // order, all at full precision.  It lets an unmodified QuEST program (which
 // prints a few values to 6 decimals, or nothing) be checked afterwards.
 static void report_register(QuregState *s, const char *path) {
+    flush(s);  // the amplitudes are read below: ensure_probs may leave collapses recorded
     ensure_probs(s);
     const int n = s->n;
     const uint64_t na = std::min<uint64_t>(16, 1ull << n);
