@@ -458,9 +458,14 @@ void flush(QuregState *s, bool home, bool probs) {
     }
 }
 
+// The largest scale of what recorded collapses keep: beyond it the kept
+// amplitudes' squares come near the smallest FP64 numbers.
+static const long double kCollapseScale = 1e150L;
+
 // Are the recorded gates nothing but measurement collapses, of qubits not
 // collapsed to the other value before?  Then fixed / value are the index bits
-// they keep and scale what they multiply the kept probabilities by.
+// they keep and scale what they multiply the kept probabilities by.  (False
+// past the limit above too: the collapses run then.)
 static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value, double &scale) {
     fixed = value = 0;
     long double product = 1.0L;  // one rounding, not one per measured qubit
@@ -474,7 +479,7 @@ static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value
         product *= (long double)g.op[1] * g.op[1];
     }
     scale = (double)product;
-    return true;
+    return product <= kCollapseScale;
 }
 
 // p0 of the state with everything recorded.  The state itself may stay as it was
