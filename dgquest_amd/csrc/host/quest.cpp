@@ -458,18 +458,21 @@ void flush(QuregState *s, bool home, bool probs) {
     }
 }
 
-// The largest scale of what recorded collapses keep: beyond it the kept
-// amplitudes' squares come near the smallest FP64 numbers.
+// Collapses that stay recorded at most (a read of P(0) walks them), and the
+// largest scale of what they keep: beyond it the kept amplitudes' squares come
+// near the smallest FP64 numbers.
+static const size_t kCollapsesHeld = 64;
 static const long double kCollapseScale = 1e150L;
 
 // Are the recorded gates nothing but measurement collapses, of qubits not
 // collapsed to the other value before?  Then fixed / value are the index bits
 // they keep and scale what they multiply the kept probabilities by.  (False
-// past the limit above too: the collapses run then.)
+// past the limits above too: the collapses run then.)
 static bool only_collapses(const QuregState *s, uint64_t &fixed, uint64_t &value, double &scale) {
     fixed = value = 0;
     long double product = 1.0L;  // one rounding, not one per measured qubit
     if (s->recorder || s->paged || s->init_kind != DQ_INIT_LOAD || s->pending.empty()) return false;
+    if (s->pending.size() >= kCollapsesHeld) return false;
     for (const Gate &g : s->pending) {
         if (g.type != OP_COLLAPSE || g.cmask || popc64(g.tmask) != 1) return false;
         const uint64_t v = g.op[0] != 0.0 ? g.tmask : 0;

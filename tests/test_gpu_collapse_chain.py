@@ -28,3 +28,17 @@ def test_unlikely_outcomes(quest, env):
         assert abs(a.real ** 2 + a.imag ** 2 - 1.0) <= n * 1e-8
     finally:
         quest.destroyQureg(q, env)
+
+
+def test_a_collapse_repeated_many_times_stays_short(quest, env):
+    q = quest.createQureg(10, env)
+    try:
+        quest.initZeroState(q)
+        quest.hadamard(q, 3)
+        for _ in range(300):
+            quest.collapseToOutcome(q, 3, 1)
+        quest.dgq_flush(q)
+        assert quest.plan_stats(q)["gates_in"] <= 64
+        assert abs(quest.getAmp(q, 8).real - 1.0) <= 1e-12
+    finally:
+        quest.destroyQureg(q, env)
