@@ -2130,14 +2130,18 @@ extern "C" int dq_stream_wait_event(void *stream, void *ev) {
 static inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // Upper bound of the device program built from n_ops descriptors in n_phases
-// phases: at most 320 bytes per descriptor.  A complex matrix in FP64 behind
-// a workgroup-condition op takes 128.  A register table of 2^R entries spans
-// 1 + 2^R / 4 descriptors; fused with shears and emitted once per assignment
-// of at most two folded workgroup bits, it takes at most 4 x (32 + 16 +
-// 16 * 2^R + 16 * R) bytes (2560 at R = 5, against 9 x 320).  Plus an END op
+// phases: at most kOpBytes per descriptor.  A complex matrix in FP64 behind
+// a workgroup-condition op takes 128, a FAN op 16 and 32 per term.  A register
+// table of 2^R entries takes 16 + 16 * 2^R bytes, emitted once per assignment
+// of at most two folded workgroup bits, each copy behind a 32-byte condition:
+// 2240 at R = 5.  The planner's tables span 1 + 2^R / 4 descriptors (9 x 320);
+// one made of plain phases folds only the bits whose copies fit what its own
+// descriptors bring (ProgBuilder::build).  Shears fused with it take 16 * R
+// in each copy, what the first of them brings (4 x 80).  Plus an END op
 // per phase, and padding so the interpreter's fixed-size header loads stay in
 // the buffer.
-static size_t prog_bound(uint32_t n_phases, uint32_t n_ops) { return (size_t)n_ops * 320 + (size_t)n_phases * 16 + 256; }
+static constexpr size_t kOpBytes = 320;
+static size_t prog_bound(uint32_t n_phases, uint32_t n_ops) { return n_ops * kOpBytes + (size_t)n_phases * 16 + 256; }
 
 extern "C" size_t dq_apply_ws_bytes(uint32_t n_blocks, uint32_t n_phases, uint32_t n_ops, uint32_t n_jobs) {
     return align_up(n_blocks * sizeof(dq_block), 256) + align_up(n_phases * sizeof(dq_phase), 256) +
@@ -2648,6 +2652,7 @@ struct ProgBuilder {
         bool pending = false;  // tab_ holds a table not yet emitted
         std::vector<WgDiag> wgd;  // workgroup-conditioned factors of the pending table
         uint64_t wg_bits = 0;     // their workgroup bits
+        size_t from = 0;          // descriptors that the table of the current run is made of
         auto is_diag = [](const dq_op &o) {
             return o.kind == DQ_OP_NEG || o.kind == DQ_OP_PHASE || o.kind == DQ_OP_DIAGR;
         };
@@ -2688,9 +2693,12 @@ struct ProgBuilder {
             wg_bits = 0;
         };
         // a NEG / PHASE with one workgroup-bit condition, folded into the pending table
+        // where the copies that a new bit makes fit the bytes of prog_bound
         auto fold_wg = [&](const dq_op &o, double fr, double fi) {
             if (o.c_thr || __builtin_popcountll(o.c_wg) != 1) return false;
-            if (!(wg_bits & o.c_wg) && __builtin_popcountll(wg_bits) >= kWgFoldBits) return false;
+            const int nb = __builtin_popcountll(wg_bits | o.c_wg);
+            if (nb > kWgFoldBits || ((32 + 16 + 2 * NR * ts) << nb) > kOpBytes * (from + 1)) return false;
+            from++;
             wgd.push_back({o.c_wg, o.v_wg, o.c_reg, o.v_reg, fr, fi});
             wg_bits |= o.c_wg;
             pending = true;
@@ -2708,9 +2716,11 @@ struct ProgBuilder {
             const unsigned char *m = reinterpret_cast<const unsigned char *>(o.m);
             if (is_diag(o) && !in_run) {
                 fold_run = false;
+                from = 0;
                 double plain = 0.0;  // vector instructions of the run's unconditioned ops, each on its own
                 for (uint32_t k2 = k; k2 < count && is_diag(ops[k2]); k2 += ops[k2].kind == DQ_OP_DIAGR ? 1 + ops[k2].tbit : 1) {
                     const dq_op &d = ops[k2];
+                    if (!d.c_thr && !d.c_wg) from += d.kind == DQ_OP_DIAGR ? 1 + d.tbit : 1;
                     if (d.kind == DQ_OP_DIAGR) fold_run |= !d.c_wg;
                     else if (!d.c_thr && !d.c_wg) plain += (d.kind == DQ_OP_NEG ? 2.0 : 4.0) * (NR >> __builtin_popcount(d.c_reg));
                 }
