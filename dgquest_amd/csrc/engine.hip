@@ -23,6 +23,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -1787,6 +1788,7 @@ constexpr unsigned kStageMax = 64;
 constexpr size_t kStageHeader = 256;
 constexpr size_t kStageKernelBytes = 64 * 1024;
 constexpr unsigned kStageThreads = 1024;
+constexpr std::chrono::seconds kStageWait(60);
 std::mutex g_stage_mu;
 StageSlot g_stage[kStageMax];
 unsigned g_stage_used = 0;
@@ -1831,28 +1833,43 @@ static int stage_free(const StageSlot &c) {
     return -1;
 }
 
-// A slot whose last upload has been read, with room for `bytes` (g_stage_mu is held).
-static int stage_pick(size_t bytes, StageSlot *&out) {
+// A slot whose last upload has been read, with room for `bytes`; lk holds g_stage_mu.
+// With every slot in flight, waits for the first that comes free, without the lock:
+// uploads of other threads go on.  After kStageWait it waits for the device instead,
+// which ends with an error if an upload can no longer be read.
+static int stage_pick(std::unique_lock<std::mutex> &lk, size_t bytes, StageSlot *&out) {
     StageSlot *slot = nullptr;
-    for (unsigned k = 0; k < g_stage_used && !slot; k++) {
-        StageSlot &c = g_stage[(g_stage_next + k) % g_stage_used];
-        const int f = stage_free(c);
-        if (f < 0) return DQ_ERR_HIP;
-        if (f) slot = &c;
-    }
-    if (!slot && g_stage_used < kStageMax) {
-        slot = &g_stage[g_stage_used];
-        HIPC(hipEventCreateWithFlags(&slot->ev, hipEventDisableTiming));
-        g_stage_used++;
-    }
-    if (!slot) {
-        slot = &g_stage[g_stage_next % g_stage_used];
-        if (slot->by_event) {
-            HIPC(hipEventSynchronize(slot->ev));
-        } else {
-            HIPC(hipDeviceSynchronize());  // the copy's stream may be gone: wait for all of them
-            if (stage_free(*slot) != 1) return fail(DQ_ERR_HIP, "stage_upload: an earlier upload never completed");
+    std::chrono::steady_clock::time_point until{};
+    bool waited = false;
+    for (;;) {
+        for (unsigned k = 0; k < g_stage_used && !slot; k++) {
+            StageSlot &c = g_stage[(g_stage_next + k) % g_stage_used];
+            const int f = stage_free(c);
+            if (f < 0) return DQ_ERR_HIP;
+            if (f) slot = &c;
         }
+        if (slot) break;
+        if (g_stage_used < kStageMax) {
+            slot = &g_stage[g_stage_used];
+            HIPC(hipEventCreateWithFlags(&slot->ev, hipEventDisableTiming));
+            g_stage_used++;
+            break;
+        }
+        const auto now = std::chrono::steady_clock::now();
+        if (until == std::chrono::steady_clock::time_point{}) until = now + kStageWait;
+        if (now < until) {
+            lk.unlock();
+            std::this_thread::sleep_for(std::chrono::microseconds(20));
+            lk.lock();
+            continue;
+        }
+        if (waited) return fail(DQ_ERR_HIP, "stage_upload: an earlier upload never completed");
+        waited = true;
+        until = {};
+        lk.unlock();
+        const hipError_t e = hipDeviceSynchronize();
+        lk.lock();
+        if (e != hipSuccess) return fail(DQ_ERR_HIP, "hipDeviceSynchronize failed: %s", hipGetErrorString(e));
     }
     g_stage_next = (unsigned)(slot - g_stage) + 1;
     StageSlot &s = *slot;
@@ -1875,8 +1892,8 @@ static int stage_pick(size_t bytes, StageSlot *&out) {
 // Puts up to kStageKernelBytes in a slot for a kernel that reads it itself and then
 // stores the ticket to the slot's first word; stage_undo if that kernel is not launched.
 static int stage_fill(const std::vector<unsigned char> &src, StageSlot *&slot) {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
-    const int rc = stage_pick(src.size(), slot);
+    std::unique_lock<std::mutex> lk(g_stage_mu);
+    const int rc = stage_pick(lk, src.size(), slot);
     if (rc) return rc;
     memcpy((unsigned char *)slot->host + kStageHeader, src.data(), src.size());
     slot->ticket++;
@@ -1890,9 +1907,9 @@ static void stage_undo(StageSlot *slot) {
 }
 
 static int stage_upload(void *d_dst, const std::vector<unsigned char> &src, void *stream) {
-    std::lock_guard<std::mutex> lk(g_stage_mu);
+    std::unique_lock<std::mutex> lk(g_stage_mu);
     StageSlot *slot = nullptr;
-    const int rc = stage_pick(src.size(), slot);
+    const int rc = stage_pick(lk, src.size(), slot);
     if (rc) return rc;
     StageSlot &s = *slot;
     unsigned char *data = (unsigned char *)s.host + kStageHeader;

@@ -56,3 +56,30 @@ for i in range(2):
     assert hip.fake_flags(i) & 0x40000000, hex(hip.fake_flags(i))
     assert not hip.fake_flags(i) & 0x80000000
 """)
+
+
+def test_uploads_past_a_long_queue_wait_for_one_slot_only(tmp_path):
+    # 64 uploads of a busy stream hold every slot; two more threads upload.  One upload read is one of them
+    # served: neither waits for the device to be idle, nor for the other.
+    run(tmp_path, """
+done = []
+for _ in range(64):
+    assert upload() == 0
+assert hip.fake_queued() == 64
+threads = [threading.Thread(target=lambda: done.append(upload()), daemon=True) for _ in range(2)]
+for t in threads:
+    t.start()
+time.sleep(0.2)
+seen = [len(done)]
+for k in range(2):
+    hip.fake_run(1)
+    end = time.time() + 5
+    while len(done) <= k and time.time() < end:
+        time.sleep(0.001)
+    seen.append(len(done))
+queued, syncs = hip.fake_queued(), hip.fake_syncs()
+while any(t.is_alive() for t in threads):  # let them end either way
+    hip.fake_run(1000)
+assert seen == [0, 1, 2], seen
+assert queued == 64 and syncs == 0 and done == [0, 0], (queued, syncs, done)
+""")
