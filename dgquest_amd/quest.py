@@ -190,13 +190,13 @@ class QuEST:
         L.dgq_recorder_plan_dense.argtypes = [Qureg, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                               C.c_void_p, C.c_void_p]
 
-        # circuits are recorded natively (csrc/host/pyrecord.cpp): gate name -> (argument shape, C function)
+        # circuits are recorded natively (csrc/host/pyrecord.cpp) where that library is built (it needs Python's
+        # headers), gate by gate otherwise: gate name -> (argument shape, C function)
         rec = os.path.join(libdir, "libdgq_pyrecord.so")
-        if not os.path.exists(rec):
-            raise RuntimeError(f"{rec} is not built; run dgquest_amd.build.build()")
-        self._record = C.PyDLL(rec).dgq_py_record
-        self._record.restype = C.py_object
-        self._record.argtypes = [C.py_object, C.py_object, C.c_int, C.POINTER(Qureg), C.py_object]
+        self._record = C.PyDLL(rec).dgq_py_record if os.path.exists(rec) else None
+        if self._record:
+            self._record.restype = C.py_object
+            self._record.argtypes = [C.py_object, C.py_object, C.c_int, C.POINTER(Qureg), C.py_object]
         self._record_table = {g: (_RECORD_SHAPES.index(ks), C.cast(getattr(L, g), C.c_void_p).value)
                               for g, ks in GATE_SIGNATURES.items() if ks in _RECORD_SHAPES}
 
@@ -247,6 +247,10 @@ class QuEST:
         def one(g):
             self.apply(q, g[0], g[1], g[2] if len(g) > 2 else ())
 
+        if not self._record:
+            for g in circuit:
+                one(g)
+            return
         table = self._record_table if type(self).apply is QuEST.apply and "apply" not in self.__dict__ else {}
         self._record(table, one, self.prec, C.byref(q), circuit)
 
