@@ -6,8 +6,9 @@
 // registers up to about 21 qubits was more than the GPU's part of the pass
 // (12 qubits, 84 gates: 66 of 140 us; 21 qubits, 372 gates: 386 of 745 us).
 //
-// Called through ctypes.PyDLL: the interpreter lock is held and a Python
-// exception left set on return is raised by the caller.
+// Called through ctypes.PyDLL: the interpreter lock is held, but for a moment
+// every kGatesPerTurn gates, and a Python exception left set on return is raised
+// by the caller.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -35,6 +36,10 @@ void call(void *f, int shape, const Qureg &r, const int *q, const double *p) {
         case QQRR: ((void (*)(Qureg, int, int, T, T))f)(r, q[0], q[1], (T)p[0], (T)p[1]); break;
     }
 }
+
+// Gates (under 0.1 us each) between two chances for other threads and signal handlers,
+// which an interpreted loop gives at every gate.
+constexpr unsigned kGatesPerTurn = 256;
 
 bool plain_list(PyObject *o) { return PyTuple_CheckExact(o) || PyList_CheckExact(o); }
 
@@ -75,6 +80,7 @@ extern "C" PyObject *dgq_py_record(PyObject *table, PyObject *fallback, int prec
     PyObject *iter = PyObject_GetIter(circuit);
     if (!iter) return nullptr;
     const Qureg r = *reg;
+    unsigned turn = 0;
     while (PyObject *g = PyIter_Next(iter)) {
         void *f = nullptr;
         int shape = 0, q[2];
@@ -92,6 +98,11 @@ extern "C" PyObject *dgq_py_record(PyObject *table, PyObject *fallback, int prec
         }
         Py_DECREF(g);
         if (!ok) break;
+        if (++turn % kGatesPerTurn == 0) {
+            if (PyErr_CheckSignals()) break;
+            Py_BEGIN_ALLOW_THREADS
+            Py_END_ALLOW_THREADS
+        }
     }
     Py_DECREF(iter);
     if (PyErr_Occurred()) return nullptr;
