@@ -1819,6 +1819,15 @@ stage_copy(const uint4 *__restrict__ src, uint4 *__restrict__ dst, uint32_t n16,
     if (threadIdx.x == 0) __hip_atomic_store(read, ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
+// A launch with an error code of its own: hipGetLastError also reports what an earlier
+// call left, and a staging buffer is in use if the kernel that reads it was launched.
+template <typename T> struct Same { using type = T; };
+template <typename... A>
+static hipError_t launch(void (*f)(A...), dim3 grid, dim3 block, size_t lds, void *stream, typename Same<A>::type... a) {
+    void *args[] = {(void *)&a...};
+    return hipLaunchKernel((const void *)f, grid, block, args, lds, (hipStream_t)stream);
+}
+
 // 1: the slot's last upload has been read, 0: not yet, -1: error (set)
 static int stage_free(const StageSlot &c) {
     if (!c.host) return 1;
@@ -1917,9 +1926,8 @@ static int stage_upload(void *d_dst, const std::vector<unsigned char> &src, void
     if (src.size() <= kStageKernelBytes && src.size() % 16 == 0 && (uintptr_t)d_dst % 16 == 0) {
         s.ticket++;
         s.by_event = false;
-        hipLaunchKernelGGL(stage_copy, dim3(1), dim3(kStageThreads), 0, (hipStream_t)stream, (const uint4 *)data, (uint4 *)d_dst,
-                           (uint32_t)(src.size() / 16), (uint32_t *)s.host, s.ticket);
-        const hipError_t e = hipGetLastError();
+        const hipError_t e = launch(stage_copy, dim3(1), dim3(kStageThreads), 0, stream, (const uint4 *)data, (uint4 *)d_dst,
+                                    (uint32_t)(src.size() / 16), (uint32_t *)s.host, s.ticket);
         if (e != hipSuccess) {
             s.ticket--;  // nothing was enqueued: the slot is free
             return fail(DQ_ERR_HIP, "stage_copy: %s", hipGetErrorString(e));
@@ -3164,12 +3172,12 @@ static int apply_blocks(int prec, const dq_block *blocks, uint32_t n_blocks, con
             one.read = slot ? (uint32_t *)slot->host : nullptr;
             one.n16 = (uint32_t)(buf.size() / 16);
             one.ticket = slot ? slot->ticket : 0;
-            hipLaunchKernelGGL(fn, dim3((unsigned)tiles, nj), dim3(64u << b0.wave_bits), lds, (hipStream_t)stream, one,
-                               d_jobs + j0, d_blocks, d_phases, d_prog, d_paux, d_baux);
+            HIPC(launch(fn, dim3((unsigned)tiles, nj), dim3(64u << b0.wave_bits), lds, stream, one, d_jobs + j0, d_blocks, d_phases,
+                        d_prog, d_paux, d_baux));
+            undo.slot = nullptr;  // the kernel reads it
         }
         HIPC(hipGetLastError());
     }
-    undo.slot = nullptr;
     return DQ_OK;
 }
 

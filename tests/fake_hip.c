@@ -16,7 +16,7 @@ typedef struct { const void *src; void *dst; uint32_t n16, *read, ticket; } copy
 
 static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
 static copy queue[1024];
-static int head, tail, syncs;
+static int head, tail, syncs, stream_syncs, pending;
 static uint32_t flags[1024];
 static int allocs;
 static __thread dim3 cfg_grid, cfg_block;
@@ -32,6 +32,10 @@ int fake_queued(void) {
 int fake_syncs(void) { return syncs; }
 int fake_allocs(void) { return allocs; }
 uint32_t fake_flags(int i) { return flags[i]; }
+int fake_stream_syncs(void) { return stream_syncs; }
+/* An error that an earlier call of the program left, reported by every hipGetLastError. */
+void fake_pending(int e) { pending = e; }
+const void *fake_source(int i) { return queue[i].src; }
 
 /* Runs up to n queued copies, oldest first. */
 void fake_run(int n) {
@@ -89,8 +93,12 @@ int hipEventCreateWithFlags(void **ev, uint32_t f) {
 int hipEventQuery(void *ev) { (void)ev; return 0; }
 int hipEventRecord(void *ev, void *stream) { (void)ev, (void)stream; return 0; }
 int hipEventSynchronize(void *ev) { (void)ev; return 0; }
-int hipStreamSynchronize(void *stream) { (void)stream; return 0; }
-int hipGetLastError(void) { return 0; }
+int hipStreamSynchronize(void *stream) {
+    (void)stream;
+    stream_syncs++;
+    return 0;
+}
+int hipGetLastError(void) { return pending; }
 int hipMemcpyAsync(void *dst, const void *src, size_t bytes, int kind, void *stream) {
     (void)kind, (void)stream;
     memcpy(dst, src, bytes);

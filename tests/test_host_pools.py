@@ -40,7 +40,7 @@ def run(tmp_path, body):
     fake = tmp_path / "libfake_hip.so"
     subprocess.check_call(["cc", "-O1", "-shared", "-fPIC", "-pthread", "-o", str(fake), os.path.join(ROOT, "tests", "fake_hip.c")])
     lib = os.path.join(ROOT, "dgquest_amd", "lib", "libdgq_engine.so")
-    p = subprocess.run([sys.executable, "-c", SETUP + body, str(fake), lib], capture_output=True, text=True, timeout=120)
+    p = subprocess.run([sys.executable, "-c", SETUP + body, str(fake), lib], capture_output=True, text=True, timeout=120, cwd=ROOT)
     assert p.returncode == 0, p.stdout + p.stderr
 
 
@@ -82,4 +82,52 @@ while any(t.is_alive() for t in threads):  # let them end either way
     hip.fake_run(1000)
 assert seen == [0, 1, 2], seen
 assert queued == 64 and syncs == 0 and done == [0, 0], (queued, syncs, done)
+""")
+
+
+def test_a_buffer_whose_kernel_was_launched_is_in_use_whatever_error_is_pending(tmp_path):
+    # an error that another call left says nothing about this launch: the copy will read its buffer
+    run(tmp_path, """
+hip.fake_source.restype = C.c_void_p
+hip.fake_pending(600)
+upload()
+upload()
+hip.fake_pending(0)
+assert upload() == 0
+assert hip.fake_queued() == 3
+assert len({hip.fake_source(i) for i in range(3)}) == 3
+""")
+
+
+def test_a_one_tile_sweep_that_was_launched_keeps_its_buffer(tmp_path):
+    run(tmp_path, """
+import numpy as np
+from dgquest_amd import circuits, quest as Q
+api = Q.load(2)
+r = api.dgq_create_recorder(10)
+api.apply_circuit(r, circuits.layered_u3_cz(10, 2, 1))
+blocks, phases, ops, _ = api.recorder_plan(r, k=4, R=3, W=1)
+assert len(blocks) == 1
+job = np.zeros(1, dtype=np.dtype([("state", "<u8"), ("block", "<u4"), ("pad", "<u4"), ("base_hi", "<u8")]))
+big = C.create_string_buffer(16 << 10)
+job["state"] = C.addressof(big)
+begin = (C.c_uint32 * 2)(0, 1)
+L.dq_apply_ws_bytes.restype = C.c_size_t
+wsb = L.dq_apply_ws_bytes(1, len(phases), len(ops), 1)
+ws = C.create_string_buffer(wsb + 256)
+at = (C.addressof(ws) + 255) // 256 * 256
+
+def sweep():
+    vp = C.c_void_p
+    return L.dq_apply_blocks(2, vp(blocks.ctypes.data), 1, vp(phases.ctypes.data), len(phases), vp(ops.ctypes.data), len(ops),
+                             vp(job.ctypes.data), begin, 1, vp(at), C.c_size_t(wsb), None)
+
+before = hip.fake_allocs()
+assert sweep() == 0, L.dq_last_error()
+assert hip.fake_allocs() == before + 1 and hip.fake_queued() == 0  # its workgroup reads the buffer, never run here
+hip.fake_pending(600)
+assert sweep() != 0
+hip.fake_pending(0)
+assert sweep() == 0
+assert hip.fake_allocs() == before + 3
 """)
