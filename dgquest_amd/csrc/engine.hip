@@ -2022,16 +2022,21 @@ namespace {
 struct ResultSlot {
     void *host;
     void *dst;
-    ResultSlot(size_t bytes, void *fallback) : host(dq_result_acquire(bytes)), dst(host ? host : fallback) {}
-    ~ResultSlot() { dq_result_release(host); }
+    hipStream_t stream;
+    bool waited = false;
+    ResultSlot(size_t bytes, void *fallback, void *s) : host(dq_result_acquire(bytes)), dst(host ? host : fallback), stream((hipStream_t)s) {}
+    ~ResultSlot() {
+        if (host && !waited) (void)hipStreamSynchronize(stream);  // an error came before: kernels may still store to it
+        dq_result_release(host);
+    }
     ResultSlot(const ResultSlot &) = delete;
     ResultSlot &operator=(const ResultSlot &) = delete;
-    // Waits for the results of the kernels enqueued on `stream` and hands them over.
-    int collect(void *out, size_t bytes, void *stream) {
-        hipStream_t s = (hipStream_t)stream;
+    // Waits for the results of the kernels enqueued on the stream and hands them over.
+    int collect(void *out, size_t bytes) {
+        waited = true;
         if (host) return dq_result_wait(host, out, bytes, stream);
-        HIPC(hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToHost, s));
-        HIPC(hipStreamSynchronize(s));
+        HIPC(hipMemcpyAsync(out, dst, bytes, hipMemcpyDeviceToHost, stream));
+        HIPC(hipStreamSynchronize(stream));
         return DQ_OK;
     }
 };
@@ -3258,12 +3263,12 @@ extern "C" int dq_prob_of_sums(const dq_block *b, const double *sums, double *ou
         return DQ_OK;
     }
     if (!d_out) return fail(DQ_ERR_ARG, "dq_prob_of_sums: null output");
-    ResultSlot res((n + 1) * sizeof(double), d_out);
+    ResultSlot res((n + 1) * sizeof(double), d_out, stream);
     hipStream_t s = (hipStream_t)stream;
     if (groups > 8192) hipLaunchKernelGGL(prob_stage2<1024>, dim3(n + 1), dim3(1024), 0, s, sums, groups, n, T, po, (double *)res.dst);
     else hipLaunchKernelGGL(prob_stage2<256>, dim3(n + 1), dim3(256), 0, s, sums, groups, n, T, po, (double *)res.dst);
     HIPC(hipGetLastError());
-    return res.collect(out, (n + 1) * sizeof(double), stream);
+    return res.collect(out, (n + 1) * sizeof(double));
 }
 
 // Split of 2^nf amplitudes over prob_stage1's workgroups: cb bits each, 2^JB
@@ -3390,20 +3395,20 @@ extern "C" int dq_prob_zero_all_fixed(const void *state, int n, int prec, uint64
         p.jb = std::max(0, p.cb - 8);
         p.groups = 1u << (nf - p.cb);
         const size_t bytes = (size_t)p.groups * (p.cb + 1) * sizeof(double);
-        ResultSlot res(bytes, nullptr);
+        ResultSlot res(bytes, nullptr, stream);
         if (res.host) {
             int rc = prob_sums(state, prec, pb, nf, p, (double *)res.host, (hipStream_t)stream);
             std::vector<double> v(bytes / sizeof(double));
-            if (!rc) rc = res.collect(v.data(), bytes, stream);
+            if (!rc) rc = res.collect(v.data(), bytes);
             if (rc) return rc;
             prob_add(v.data(), p.groups, n, p.cb, po, out);
             return DQ_OK;
         }
     }
-    ResultSlot res((n + 1) * sizeof(double), d_out);
+    ResultSlot res((n + 1) * sizeof(double), d_out, stream);
     const int rc = prob_launch(state, n, prec, fixed_mask, fixed_value, scale, (double *)res.dst, d_ws, part_bytes, (hipStream_t)stream);
     if (rc) return rc;
-    return res.collect(out, (n + 1) * sizeof(double), stream);
+    return res.collect(out, (n + 1) * sizeof(double));
 }
 
 extern "C" int dq_prob_zero_all(const void *state, int n, int prec, double *out, void *d_ws, size_t ws_bytes, void *stream) {
@@ -3910,7 +3915,7 @@ extern "C" int dq_read_amps(const void *state, int n, int prec, const int *l2p, 
     const size_t bytes = count * 2 * sizeof(double);
     const size_t need = align_up(64 * sizeof(int), 256) + bytes;
     if (!d_ws || ws_bytes < need) return fail(DQ_ERR_ARG, "dq_read_amps: workspace %zu < %zu bytes", ws_bytes, need);
-    ResultSlot res(bytes, (unsigned char *)d_ws + align_up(64 * sizeof(int), 256));
+    ResultSlot res(bytes, (unsigned char *)d_ws + align_up(64 * sizeof(int), 256), stream);
     const unsigned blocks = (unsigned)((count + 255) / 256);
     if (prec == DQ_F64)
         hipLaunchKernelGGL(read_kernel<double>, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
@@ -3919,7 +3924,7 @@ extern "C" int dq_read_amps(const void *state, int n, int prec, const int *l2p, 
         hipLaunchKernelGGL(read_kernel<float>, dim3(blocks), dim3(256), 0, (hipStream_t)stream,
                            (const V2<float>::type *)state, n, map, start, count, (double *)res.dst);
     HIPC(hipGetLastError());
-    return res.collect(out, bytes, stream);
+    return res.collect(out, bytes);
 }
 
 extern "C" int dq_write_amps(void *state, int n, int prec, uint64_t start, uint64_t count, const double *re,

@@ -131,3 +131,20 @@ hip.fake_pending(0)
 assert sweep() == 0
 assert hip.fake_allocs() == before + 3
 """)
+
+
+def test_a_failed_read_out_gives_its_result_slot_back_when_its_kernels_are_done(tmp_path):
+    # the kernels of a call that ends with an error may still store to the slot
+    run(tmp_path, """
+m = 14  # two launches of 256 threads each
+big = C.create_string_buffer(16 << m)
+L.dq_prob_ws_bytes.restype = C.c_size_t
+wsb = L.dq_prob_ws_bytes(m)
+ws = C.create_string_buffer(wsb)
+out = (C.c_double * (m + 1))()
+hip.fake_pending(600)
+assert L.dq_prob_zero_all(big, m, 2, out, ws, C.c_size_t(wsb), None) != 0
+assert hip.fake_stream_syncs() == 1
+assert L.dq_read_amps(big, m, 2, None, C.c_uint64(0), C.c_uint64(4), out, ws, C.c_size_t(wsb), None) != 0
+assert hip.fake_stream_syncs() == 2
+""")
