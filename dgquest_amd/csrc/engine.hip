@@ -1172,7 +1172,7 @@ compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB
 // (NC = 2^(T-k) columns): Yr = Ur Xr - Ui Xi, Yi = Ui Xr + Ur Xi.
 //
 // Each FP32 factor is the sum of three bf16 numbers (8 significant bits each, 24 in
-// all: the split of an FP32 amplitude is exact), and a real product is the six
+// all), and a real product is the six
 // piece products of order up to 2^-16, on v_mfma_f32_32x32x16_bf16 with FP32
 // sums: 16 times the rate of v_mfma_f32_32x32x2f32, so 2.7 times for a product.
 // The leading products have accumulators of their own (their sums take 2 K / 16
@@ -1184,6 +1184,17 @@ compare_stage1(const typename V2<TA>::type *__restrict__ a, const typename V2<TB
 // at 1.1-1.3 PFLOP/s of bf16, what a large library product reaches (1.36): clocks
 // fall as the run goes on, so vector instructions beside the products cost time too.
 //
+// bf16 ends at 2^-133 where FP32 goes to 2^-149, so the lower pieces of a factor below
+// 2^-110 would lose bits.  Matrices are scaled by 2^DENSE_SCALE_LOG, and so are the
+// amplitudes of a tile as it is loaded: the split of an FP32 amplitude is exact, also of
+// a denormal one.  Every op then leaves the tile scaled by as much again; that is
+// taken off as the tile is stored, or by an op that would go beyond
+// DENSE_SCALE_MAX (taken off at every op it cost 4%, so 2%: 25 qubits, depth 10, k = 5, 6
+// and 7 3.71 -> 3.84, 4.92 -> 5.08 and 6.09 -> 6.21 ms).  A tile with an
+// amplitude of 2^32 or more, which could overflow, is scaled down instead and its scale
+// restored by every op.  The scales are powers of two: results are the same
+// otherwise.  An infinite amplitude makes its column NaN.
+//
 // v_mfma_f32_32x32x16_bf16: lane l supplies A[l % 32][8 (l / 32) + i] and
 // B[8 (l / 32) + i][l % 32], i = 0..7 in 16 bytes; result register v of lane l is
 // C[8 (v / 4) + 4 (l / 32) + v % 4][l % 32].  A matrix is stored as those 16 bytes:
@@ -1192,12 +1203,15 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 #define DENSE_T_MAX 13
+#define DENSE_SCALE_LOG 16
+#define DENSE_SCALE_MAX 48
 #define DENSE_THREADS 256
 #define DENSE_COLS 256  // column-table entries per op: 2^(T - k) <= 2^(13 - 5)
 #define DENSE_WAVES (DENSE_THREADS / 64)
 
-// The three bf16 pieces of a matrix entry, rounded to nearest even.
+// The three bf16 pieces of a scaled matrix entry, rounded to nearest even.
 static __host__ __device__ inline void split_entry(double x, uint16_t *piece) {
+    x *= (double)(1 << DENSE_SCALE_LOG);
     for (int i = 0; i < 3; i++) {
         const float f = (float)x;
         uint32_t u;
@@ -1252,7 +1266,7 @@ __device__ __forceinline__ uint32_t dswz(uint32_t e) { return e ^ ((e >> 5) & 31
 template <int KL>
 __device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restrict__ im, uint32_t T, const dq_dense_op &op,
                                          const uint4 *__restrict__ mat, const uint32_t *__restrict__ coloff, uint32_t lane,
-                                         uint32_t w) {
+                                         uint32_t w, float fix) {
     constexpr uint32_t K = 1u << KL, KS = K / 16, RB = K / 32, RP = RB >= 2 ? 2 : 1;
     const uint32_t lc = T - KL - 5, NCB = 1u << lc, items = NCB * (RB / RP);
     uint32_t sd[KL];
@@ -1341,6 +1355,17 @@ __device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restri
                 }
             }
         }
+        if (busy) {
+#pragma unroll
+            for (uint32_t r = 0; r < RP; r++)
+#pragma unroll
+                for (int c = 0; c < 2; c++) acc[r][c] += acc[r][c + 2];
+            if (fix != 1.0f)  // uniform
+#pragma unroll
+                for (uint32_t r = 0; r < RP; r++)
+#pragma unroll
+                    for (int c = 0; c < 2; c++) acc[r][c] *= fix;
+        }
         // In place: an item with every row of its columns reads exactly the tile
         // elements it writes; otherwise every wave has to have read them.
         if constexpr (RB > RP) __syncthreads();
@@ -1354,8 +1379,8 @@ __device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restri
 #pragma unroll
             for (int v = 0; v < 16; v++) {
                 const uint32_t u = z ^ ((v & 1) ? sd[0] : 0u) ^ ((v & 2) ? sd[1] : 0u) ^ ((v & 4) ? sd[3] : 0u) ^ ((v & 8) ? sd[4] : 0u);
-                re[u] = acc[r][0][v] + acc[r][2][v];
-                im[u] = acc[r][1][v] + acc[r][3][v];
+                re[u] = acc[r][0][v];
+                im[u] = acc[r][1][v];
             }
         }
     }
@@ -1370,6 +1395,7 @@ __global__ void __launch_bounds__(DENSE_THREADS, 2)
 dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restrict__ ops, const uint4 *__restrict__ mats,
              const uint32_t *__restrict__ ctab, typename V2<float>::type *__restrict__ st) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
+    __shared__ uint32_t wave_large[DENSE_WAVES];  // has the wave loaded an amplitude of 2^32 or more?
     const uint32_t T = blk->tile_bits;
     const uint32_t NT = 1u << T;
     float *re = reinterpret_cast<float *>(lds_raw);
@@ -1410,21 +1436,39 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
         for (int b = 0; b < DENSE_T_MAX - 8; b++) g |= ((i >> b) & 1u) ? hi[b] : 0ull;
         return g;
     };
+    auto power = [](int e) { return __uint_as_float((uint32_t)(127 + e) << 23); };
+    bool large;
     {
         typename V2<float>::type v[LI];
 #pragma unroll
         for (int i = 0; i < LI; i++) v[i] = __builtin_nontemporal_load(lane_ptr(st + gaddr((uint32_t)i & (NI - 1)), lane));
+        float top = 0.0f;
+#pragma unroll
+        for (int i = 0; i < LI; i++) top = fmaxf(top, fmaxf(fabsf(v[i].x), fabsf(v[i].y)));
+        const uint64_t any = __ballot(top >= 0x1p32f);
+        if (lane == 0) wave_large[wv] = any != 0;
+        __syncthreads();
+        uint32_t l = 0;
+#pragma unroll
+        for (int w = 0; w < DENSE_WAVES; w++) l |= wave_large[w];
+        large = __builtin_amdgcn_readfirstlane(l) != 0;
+        const float s = large ? power(-DENSE_SCALE_LOG) : power(DENSE_SCALE_LOG);
 #pragma unroll
         for (int i = 0; i < LI; i++) {
             const uint32_t z = tz ^ dswz(((uint32_t)i & (NI - 1)) * DENSE_THREADS);
-            re[z] = v[i].x;
-            im[z] = v[i].y;
+            re[z] = v[i].x * s;
+            im[z] = v[i].y * s;
         }
     }
     constexpr size_t msz = (size_t)12 << (2 * KL);  // bytes of a matrix
+    const int first = large ? -DENSE_SCALE_LOG : DENSE_SCALE_LOG, most = large ? first : DENSE_SCALE_MAX;
+    int scale = first;  // the tile's, as a power of two
     for (uint32_t o = 0; o < blk->op_count; o++) {
         const dq_dense_op op = ops[blk->op_begin + o];
-        dense_op<KL>(re, im, T, op, mats + op.mat * (msz / 16), ctab + (size_t)(blk->op_begin + o) * DENSE_COLS, lane, wv);
+        scale += DENSE_SCALE_LOG;
+        const int off = scale > most ? scale - first : 0;
+        scale -= off;
+        dense_op<KL>(re, im, T, op, mats + op.mat * (msz / 16), ctab + (size_t)(blk->op_begin + o) * DENSE_COLS, lane, wv, power(-off));
     }
     __syncthreads();
     {
@@ -1433,11 +1477,12 @@ dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restri
         uint32_t lane2 = lane, tz2 = tz;
         asm volatile("" : "+v"(lane2), "+v"(tz2));
         typename V2<float>::type v[LI];
+        const float s = power(-scale);
 #pragma unroll
         for (int i = 0; i < LI; i++) {
             const uint32_t z = tz2 ^ dswz(((uint32_t)i & (NI - 1)) * DENSE_THREADS);
-            v[i].x = re[z];
-            v[i].y = im[z];
+            v[i].x = re[z] * s;
+            v[i].y = im[z] * s;
         }
 #pragma unroll
         for (int i = 0; i < LI; i++) __builtin_nontemporal_store(v[i], lane_ptr(st + gaddr((uint32_t)i & (NI - 1)), lane2));

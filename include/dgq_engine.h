@@ -293,7 +293,8 @@ typedef struct dq_dense_op {
 
 /* Apply `n_blocks` dense blocks in order to an FP32 state of n qubits.
  * mats: n_mats complex matrices, 2^k x 2^k each, row-major {re, im} doubles
- * (host memory; split into bf16 pieces and laid out for MFMA by this call). */
+ * (host memory; split into bf16 pieces, 24 bits in all from 2^-126 to 2^112,
+ * and laid out for MFMA by this call). */
 int dq_apply_dense(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops, uint32_t n_ops,
                    const double *mats, uint32_t n_mats, void *state, void *d_ws, size_t ws_bytes, void *stream);
 size_t dq_dense_ws_bytes(int k, uint32_t n_blocks, uint32_t n_ops, uint32_t n_mats);
@@ -312,8 +313,8 @@ typedef struct dq_small_gate {
 
 /* dq_apply_dense with the matrices formed on the device: matrix i is the
  * product of gates[gate_begin[i]] .. gates[gate_begin[i + 1] - 1], applied in
- * that order (gate_begin has n_mats + 1 entries), computed in FP64 and rounded
- * to float once. */
+ * that order (gate_begin has n_mats + 1 entries), computed in FP64 and split
+ * into bf16 pieces once. */
 int dq_apply_dense_gates(int k, const dq_dense_block *blocks, uint32_t n_blocks, const dq_dense_op *ops, uint32_t n_ops,
                          const dq_small_gate *gates, const uint32_t *gate_begin, uint32_t n_mats, void *state, void *d_ws,
                          size_t ws_bytes, void *stream);
