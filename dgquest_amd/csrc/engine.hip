@@ -1569,8 +1569,7 @@ dense_form(const dq_small_gate *__restrict__ gates, const uint32_t *__restrict__
     }
 }
 
-// one workgroup: out = {re <a|b>, im <a|b>, <a|a>, <b|b>, max |a_i - b_i|}
-// One workgroup per slot.
+// out = {re <a|b>, im <a|b>, <a|a>, <b|b>, max |a_i - b_i|}: one workgroup per slot.
 __global__ void __launch_bounds__(256) compare_stage2(const double *__restrict__ part, uint32_t ngroups, double *__restrict__ out) {
     __shared__ double red[4];
     const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
@@ -1811,9 +1810,11 @@ static uint32_t exchange_elem_bytes(int prec, int xm) {
 // Up to kStageKernelBytes a kernel of one workgroup makes the copy and, once it
 // has read the buffer, stores the upload's number into it.  An event recorded
 // after the copy instead costs the stream 4.5 us before its next kernel starts
-// (two launches and a wait: 12.9 us, with an event between them 17.4 us).  One
-// workgroup has 64 KiB in flight at once, the latency of the host link; longer
-// uploads go through the copy engine and an event.
+// (two launches and a wait: 12.9 us, with an event between them 17.4 us).  The
+// compiler keeps stage_copy's array in LDS and waits for each of its up to four
+// loads a thread, so 64 KiB take up to four latencies of the host link one after
+// another (bring_descriptors has its loads in flight together); longer uploads go
+// through the copy engine and an event.
 // ----------------------------------------------------------------------------
 namespace {
 struct StageSlot {
@@ -1996,7 +1997,10 @@ static int stage_upload(void *d_dst, const std::vector<unsigned char> &src, void
 // The caller need not wait for the stream either: a slot is handed out with
 // every word set to kUnwritten, and each word is ready once it holds anything
 // else.  A word is stored once, by a thread that has read its inputs, so when
-// all of them have arrived nothing the kernels read or write is in use any more.  Launch
+// all of them have arrived nothing the kernels read is in use any more.  What else a
+// kernel writes may still be on its way: a sweep that writes tile sums has issued the
+// stores of its state by then, not completed them.  Work on the same stream is ordered
+// after it; another stream needs an event or a wait for this one.  Launch
 // and wait for a kernel that stores one word 10.9 -> 5.4 us, 8192 words 11.8 -> 8.5 us.
 // A wait longer than kResultPoll goes on as a wait for the stream, which also ends it
 // where a result is that very word (no operation makes it: a signalling NaN) or

@@ -42,8 +42,8 @@ size of each op code is fixed (op_size below).
                 FM_* code (never an op of its own), v_thr = bytes of the op.
                 Term: u32 lane condition (mask | value << 16, 0: every lane),
                 u32 workgroup condition (0: none; bit number | 1 << 8 | value
-                << 9) | 1 << 10 on the last term, [8 bytes of padding in FP64,]
-                re, im
+                << 9) | 1 << 10 on the last term, 8 bytes of padding, re, im
+                (doubles in either precision)
 Scalar registers s36..s71 are reserved by the asm (clobbered; the compiler
 keeps the SGPRs above s71 for itself, and at 8 waves per SIMD it may not use
 any above s71):

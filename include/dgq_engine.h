@@ -169,7 +169,9 @@ int dq_memcpy_async(void *dst, const void *src, size_t bytes, int kind, void *st
  * device memory).  Slots are shared by all threads and streams.
  * dq_result_wait waits until kernels enqueued on `stream` have stored all
  * `bytes` (a multiple of 8) and copies them to `out`; release the slot after
- * it. */
+ * it.  The stream may still be busy then: what else those kernels write (the
+ * state, of a sweep that writes its sums to a slot) is complete for later work
+ * on `stream`, and for other streams after an event or dq_stream_sync. */
 void *dq_result_acquire(size_t bytes);
 int dq_result_wait(const void *slot, void *out, size_t bytes, void *stream);
 void dq_result_release(void *slot);
@@ -205,7 +207,8 @@ int dq_apply_blocks(int prec,
  * dq_block_sums_on_host says so.  dq_prob_of_sums makes of them what
  * dq_prob_zero_all reads from the state: out[q] = P(q = 0) for the n qubits as
  * they were stored, out[n] = the total.  d_out: n + 1 doubles of device memory
- * (unused with a slot).  It waits for the result. */
+ * (unused with a slot).  It waits for the result, not for the stream (see
+ * dq_result_wait). */
 int dq_apply_blocks_sums(int prec,
                          const dq_block *blocks, uint32_t n_blocks,
                          const dq_phase *phases, uint32_t n_phases,
@@ -344,7 +347,6 @@ int dq_compare_states(const void *a, int prec_a, const void *b, int prec_b, int 
                       void *d_ws, size_t ws_bytes, void *stream);
 size_t dq_compare_ws_bytes(int n_qubits);
 
-/* 0 if all work recorded before `ev` has completed, 1 if not yet (no wait). */
 /* The qubits of a state permuted in place: the amplitude at index x moves to
  * the index whose bit dest[p] is bit p of x.  One pass over the state if dest
  * is an involution or moves few bits, two otherwise; no workspace, no sync.
@@ -353,6 +355,7 @@ size_t dq_compare_ws_bytes(int n_qubits);
  * (src/cpp/QuEST_gpu_kernel.cu:589-636) for a whole register. */
 int dq_permute_qubits(void *state, int n_qubits, int prec, const int *dest, void *stream);
 int dq_permute_launches(int n_qubits, int prec, const int *dest);
+/* 0 if all work recorded before `ev` has completed, 1 if not yet (no wait). */
 int dq_event_query(void *ev);
 /* Wait for the work recorded before `ev`. */
 int dq_event_sync(void *ev);

@@ -58,7 +58,9 @@ int dgq_sync(Qureg qureg);
 int dgq_read_state(Qureg qureg, unsigned long long start, unsigned long long count, double *out);
 
 /* The HIP stream (hipStream_t) this register's kernels run on, for event
- * timing around its sweeps. */
+ * timing around its sweeps.  Calls that return a result (probabilities,
+ * amplitudes, samples, overlaps) wait for it, not for the stream: before another
+ * stream uses the state, dgq_sync or an event on this one. */
 void *dgq_stream(Qureg qureg);
 
 /* Algorithmic HBM bytes of the last flush: every sweep reads and writes the
