@@ -1944,11 +1944,21 @@ static int stage_pick(std::unique_lock<std::mutex> &lk, size_t bytes, StageSlot 
     return DQ_OK;
 }
 
+// An upload cannot be part of a graph: its replays would read the staging buffer
+// again after it went to other uploads.
+static int stage_capture(void *stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    HIPC(hipStreamIsCapturing((hipStream_t)stream, &status));
+    return status == hipStreamCaptureStatusNone ? DQ_OK : fail(DQ_ERR_UNSUPPORTED, "descriptors cannot be uploaded while their stream is captured");
+}
+
 // Puts up to kStageKernelBytes in a slot for a kernel that reads it itself and then
 // stores the ticket to the slot's first word; stage_undo if that kernel is not launched.
-static int stage_fill(const std::vector<unsigned char> &src, StageSlot *&slot) {
+static int stage_fill(const std::vector<unsigned char> &src, StageSlot *&slot, void *stream) {
+    int rc = stage_capture(stream);
+    if (rc) return rc;
     std::unique_lock<std::mutex> lk(g_stage_mu);
-    const int rc = stage_pick(lk, src.size(), slot);
+    rc = stage_pick(lk, src.size(), slot);
     if (rc) return rc;
     memcpy((unsigned char *)slot->host + kStageHeader, src.data(), src.size());
     slot->ticket++;
@@ -1962,9 +1972,11 @@ static void stage_undo(StageSlot *slot) {
 }
 
 static int stage_upload(void *d_dst, const std::vector<unsigned char> &src, void *stream) {
+    int rc = stage_capture(stream);
+    if (rc) return rc;
     std::unique_lock<std::mutex> lk(g_stage_mu);
     StageSlot *slot = nullptr;
-    const int rc = stage_pick(lk, src.size(), slot);
+    rc = stage_pick(lk, src.size(), slot);
     if (rc) return rc;
     StageSlot &s = *slot;
     unsigned char *data = (unsigned char *)s.host + kStageHeader;
@@ -3178,7 +3190,7 @@ static int apply_blocks(int prec, const dq_block *blocks, uint32_t n_blocks, con
               lookup(prec, b.reg_bits, b.wave_bits, exchange_mode(prec, (int)b.reg_bits, (int)b.wave_bits, (int)b.tile_bits), true);
     }
     StageSlot *slot = nullptr;
-    int rc = own ? stage_fill(buf, slot) : stage_upload(d_ws, buf, stream);
+    int rc = own ? stage_fill(buf, slot, stream) : stage_upload(d_ws, buf, stream);
     if (rc) return rc;
     struct Undo {
         StageSlot *slot;

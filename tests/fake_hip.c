@@ -16,7 +16,7 @@ typedef struct { const void *src; void *dst; uint32_t n16, *read, ticket; } copy
 
 static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
 static copy queue[1024];
-static int head, tail, syncs, stream_syncs, pending;
+static int head, tail, syncs, stream_syncs, pending, capturing;
 static uint32_t flags[1024];
 static int allocs;
 static __thread dim3 cfg_grid, cfg_block;
@@ -35,6 +35,8 @@ uint32_t fake_flags(int i) { return flags[i]; }
 int fake_stream_syncs(void) { return stream_syncs; }
 /* An error that an earlier call of the program left, reported by every hipGetLastError. */
 void fake_pending(int e) { pending = e; }
+/* Every stream is being captured (1) or none. */
+void fake_capture(int on) { capturing = on; }
 const void *fake_source(int i) { return queue[i].src; }
 
 /* Runs up to n queued copies, oldest first. */
@@ -96,6 +98,11 @@ int hipEventSynchronize(void *ev) { (void)ev; return 0; }
 int hipStreamSynchronize(void *stream) {
     (void)stream;
     stream_syncs++;
+    return 0;
+}
+int hipStreamIsCapturing(void *stream, int *status) {
+    (void)stream;
+    *status = capturing;
     return 0;
 }
 int hipGetLastError(void) { return pending; }

@@ -130,6 +130,21 @@ assert sweep() != 0
 hip.fake_pending(0)
 assert sweep() == 0
 assert hip.fake_allocs() == before + 3
+hip.fake_capture(1)
+assert sweep() != 0 and b"captur" in L.dq_last_error(), L.dq_last_error()
+""")
+
+
+def test_uploads_are_refused_while_their_stream_is_captured(tmp_path):
+    # a graph would read the staging buffer at every replay, long after it went to other uploads
+    run(tmp_path, """
+assert upload() == 0
+hip.fake_run(1)
+hip.fake_capture(1)
+assert upload() != 0 and b"captur" in L.dq_last_error(), L.dq_last_error()
+assert hip.fake_queued() == 0
+hip.fake_capture(0)
+assert upload() == 0
 """)
 
 
