@@ -221,7 +221,9 @@ __device__ __forceinline__ uint64_t tile_base_runs(CWords ba, uint32_t t) {
 
 // Occupancy target (waves per SIMD) of a sweep instantiation: the register
 // tile takes 2^R amplitudes x (2 * sizeof(T) / 4) VGPRs; allow 40 more for
-// addresses, coefficients and temporaries.
+// addresses, coefficients and temporaries.  Split-exchange R = 5 tiles need
+// more: 128 VGPRs and 4 spilled in FP32 (104 and none before the FAN op's FP64
+// factor and the sums for P(0)), 168 and 7 in FP64 (as before).
 template <typename T, int R, int XM>
 constexpr int sweep_waves_per_eu() {
     constexpr int amp = (1 << R) * (int)(2 * sizeof(T) / 4);
@@ -1390,6 +1392,7 @@ __device__ __forceinline__ void dense_op(float *__restrict__ re, float *__restri
 // One dense block over every tile of an FP32 state: grid = tiles, 256 threads.  Two
 // workgroups (64 KiB of LDS each at T = 13) share a CU, a wave of either on each SIMD
 // with up to 256 VGPRs: one's loads and stores run beside the other's products.
+// 40-54 SGPRs spill to VGPR lanes, at k = 6 two VGPRs to memory.
 template <int KL>
 __global__ void __launch_bounds__(DENSE_THREADS, 2)
 dense_kernel(const dq_dense_block *__restrict__ blk, const dq_dense_op *__restrict__ ops, const uint4 *__restrict__ mats,
